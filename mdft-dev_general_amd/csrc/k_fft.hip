@@ -1,14 +1,14 @@
-// k_fft.hip -- batched 3D complex FFTs of all projections, FP64.
+// k_fft.hip -- batched 3D complex FFTs of all projections, FP64 and FP32.
 //
 // Replaces the FFTW plans of src/module_energy_cproj_mrso.f90:256-267 and the
 // transforms at :306-329 (sign +1, unnormalised) and :690-719 (sign -1, then
 // scaled by 1/(nx ny nz)).  The projection field is stored as the reference's
-// deltarho_p(np,nx,ny,nz): projection index fastest.  Each pass transforms one
-// axis: a workgroup takes one grid line along the axis for PB consecutive
-// projections (a contiguous PB*16-byte run per grid point, so loads and stores
-// are coalesced for every axis), runs a mixed-radix Stockham FFT in LDS
-// (radix 8/4/2/3/5 stages, natural-order output, no bit reversal) and writes
-// the line back in place.
+// deltarho_p(np,nx,ny,nz): projection index fastest.  A pass transforms one axis
+// in place.  For each of them the field is [outer][n][C] with C contiguous columns:
+// C = np along x, nx np along y and nx ny np along z.  A workgroup takes PB columns
+// (128 bytes) of one outer index, runs a mixed-radix Stockham FFT and writes the
+// lines back.  Along y and z the columns of a workgroup may belong to two grid points,
+// so that every workgroup but the last has PB of them whatever np is.
 #include "mdft_internal.h"
 
 namespace {
@@ -27,7 +27,7 @@ template <typename V> __device__ inline V csub(V a, V b) { return mk<V>(a.x - b.
 template <typename V> __device__ inline V mul_si(V a, decltype(V::x) s) { return mk<V>(-s * a.y, s * a.x); }
 
 template <int R, typename V>
-struct Dft;
+struct Dft;  // composite radices below
 
 template <typename V>
 struct Dft<2, V> {
@@ -105,6 +105,87 @@ struct Dft<8, V> {
     }
 };
 
+// cos and sin of 2 pi k / n as compile-time constants: the angle is folded into [0, pi / 4]
+// by its index (exact), where the Taylor series to x^23 is correct to the last bits
+constexpr double kPi = 3.14159265358979323846;
+constexpr double taylor(double x, int first) {  // first 0: cos, 1: sin
+    double t = first ? x : 1.0, s = 0.0;
+    double terms[12] = {};
+    for (int i = 0; i < 12; i++) {
+        terms[i] = t;
+        t *= -x * x / (double)((2 * i + 1 + first) * (2 * i + 2 + first));
+    }
+    for (int i = 11; i >= 0; i--) s += terms[i];
+    return s;
+}
+constexpr double cos_turn(int k, int n);
+constexpr double sin_turn(int k, int n) {
+    k = ((k % n) + n) % n;
+    if (2 * k > n) return -sin_turn(n - k, n);
+    if (4 * k > n) return (4 * k == 2 * n) ? 0.0 : (n % 2 ? taylor(kPi * (n - 2 * k) / n, 1) : sin_turn(n / 2 - k, n));
+    if (8 * k > n) return taylor(kPi * (n - 4 * k) / (2.0 * n), 0);
+    return taylor(2.0 * kPi * k / n, 1);
+}
+constexpr double cos_turn(int k, int n) {
+    k = ((k % n) + n) % n;
+    if (2 * k > n) k = n - k;
+    if (4 * k > n) return -(n % 2 ? taylor(kPi * (n - 2 * k) / n, 0) : cos_turn(n / 2 - k, n));
+    if (8 * k > n) return taylor(kPi * (n - 4 * k) / (2.0 * n), 1);
+    return taylor(2.0 * kPi * k / n, 0);
+}
+static_assert(cos_turn(1, 8) - 0.70710678118654752440 < 2e-16 && cos_turn(1, 8) - 0.70710678118654752440 > -2e-16, "");
+static_assert(sin_turn(2, 5) - 0.58778525229247312917 < 2e-16 && sin_turn(2, 5) - 0.58778525229247312917 > -2e-16, "");
+static_assert(cos_turn(4, 9) + 0.93969262078590838405 < 2e-16 && cos_turn(4, 9) + 0.93969262078590838405 > -2e-16, "");
+
+// e^{s 2 pi i k / N} v for compile-time k
+template <int K, int N, typename V>
+__device__ inline V turn(V v, decltype(V::x) s) {
+    using T = decltype(V::x);
+    if constexpr (K % N == 0) return v;
+    else if constexpr ((4 * K) % N == 0) {
+        constexpr int q = (4 * K / N) % 4;
+        if constexpr (q == 1) return mul_si(v, s);
+        else if constexpr (q == 2) return mk<V>(-v.x, -v.y);
+        else return mul_si(v, -s);
+    } else {
+        constexpr T c = (T)cos_turn(K, N), w = (T)sin_turn(K, N);
+        return cmul(v, mk<V>(c, s * w));
+    }
+}
+
+// Composite radices: R = R1 R2 in registers, x[j2 + R2 j1] -> X[k1 + R1 k2]
+constexpr int first_factor(int r) { return r % 4 == 0 && r != 12 ? 4 : (r % 3 == 0 ? 3 : (r % 5 == 0 ? 5 : 2)); }
+template <int R, typename V>
+struct Dft {
+    static constexpr int R1 = first_factor(R), R2 = R / R1;
+    template <int J2, int K1>
+    static __device__ inline void twiddle(V *a, decltype(V::x) s) {
+        a[K1] = turn<J2 * K1, R>(a[K1], s);
+        if constexpr (K1 + 1 < R1) twiddle<J2, K1 + 1>(a, s);
+    }
+    template <int J2>
+    static __device__ inline void first(V *v, V (*y)[R1], decltype(V::x) s) {
+#pragma unroll
+        for (int j1 = 0; j1 < R1; j1++) y[J2][j1] = v[J2 + R2 * j1];
+        Dft<R1, V>::run(y[J2], s);
+        twiddle<J2, 0>(y[J2], s);
+        if constexpr (J2 + 1 < R2) first<J2 + 1>(v, y, s);
+    }
+    static __device__ inline void run(V *v, decltype(V::x) s) {
+        V y[R2][R1];
+        first<0>(v, y, s);
+#pragma unroll
+        for (int k1 = 0; k1 < R1; k1++) {
+            V z[R2];
+#pragma unroll
+            for (int j2 = 0; j2 < R2; j2++) z[j2] = y[j2][k1];
+            Dft<R2, V>::run(z, s);
+#pragma unroll
+            for (int k2 = 0; k2 < R2; k2++) v[k1 + R1 * k2] = z[k2];
+        }
+    }
+};
+
 // One Stockham stage of radix R over `rows` lines of length n held in LDS;
 // twiddles read from the FP64 table and rounded to the working precision.
 template <int R, typename V>
@@ -135,32 +216,49 @@ __device__ inline void stockham_stage(const V *src, V *dst, int n, int ld, int N
     }
 }
 
-struct LineGeom {
-    int n;          // transform length
-    long long es;   // element stride (grid points)
-    int na;         // size of the first other axis
-    long long sa;   // stride of the first other axis (points)
-    long long sb;   // stride of the second other axis (points)
-    int align;      // > 0: batches start where runs of `align` elements meet the cache-line grid
+// The lines of one pass: [outer][n][C], C contiguous columns; a workgroup takes the pb columns
+// from c0 = batch pb of one outer index.
+struct Cols {
+    size_t C;          // columns
+    unsigned pb;       // columns per workgroup
+    unsigned nbatch;   // workgroups per outer index
+    unsigned nwg;      // all workgroups
+    unsigned run;      // consecutive workgroups of one XCD
+    unsigned lines;    // > 1: a workgroup takes whole lines of `lines` outer indices (C small), pb = lines C rows
+    unsigned nouter;
 };
 
-template <int PB, typename V>
-__global__ __launch_bounds__(kThreads) void fft_axis(V *__restrict__ data, int np, LineGeom g, FftAxisPlan plan,
-                                                    double sgn_d, double scale_d) {
+// Workgroups go to the 8 XCDs round robin in dispatch order.  `run` consecutive ones are given to
+// one XCD (one L2), so that the 128-byte lines that two workgroups share are read from HBM once,
+// while all XCDs stay within 8 run workgroups of each other: ranges an eighth of the field apart
+// meet in the same memory channels.  Measured per evaluation (128^3, mmax 5, FP64; 6 passes): one
+// range per XCD 7.00 ms, runs of 96 6.95, 24 6.55-7.0, 8 7.02, round robin 7.69 ms; FP32 (shared
+// lines along x) 3.52, 3.45, 3.47, 3.52, 4.40 ms.
+constexpr unsigned kRun = 24;
+__device__ inline unsigned xcd_order(unsigned run) {
+    const unsigned g = blockIdx.x / (8 * run), w = blockIdx.x - g * 8 * run;
+    return (g * 8 + (w & 7)) * run + (w >> 3);
+}
+
+// Line lengths that are not known at compile time.
+template <typename V>
+__global__ __launch_bounds__(kThreads) void fft_axis(V *__restrict__ data, Cols g, FftAxisPlan plan, double sgn_d,
+                                                    double scale_d) {
     using T = decltype(V::x);
     extern __shared__ __align__(16) unsigned char fft_smem[];
     V *sbuf = reinterpret_cast<V *>(fft_smem);
     const T sgn = (T)sgn_d, scale = (T)scale_d;
-    const int n = g.n, ld = n + 1;
+    const int n = plan.n, ld = n + 1, PB = (int)g.pb;
+    const unsigned id = xcd_order(g.run);
+    if (id >= g.nwg) return;
     V *A = sbuf, *B = sbuf + PB * ld;
-    const int line = blockIdx.x;
-    const int a = line % g.na, b = line / g.na;
-    const long long base = (long long)a * g.sa + (long long)b * g.sb;
-    const int p0 = blockIdx.y * PB;
-    const int pb = (np - p0) < PB ? (np - p0) : PB;
-    for (int idx = threadIdx.x; idx < n * PB; idx += kThreads) {
-        const int p = idx % PB, e = idx / PB;
-        if (p < pb) A[p * ld + e] = data[(base + (long long)e * g.es) * np + p0 + p];
+    const unsigned o = id / g.nbatch;
+    const size_t c0 = (size_t)(id % g.nbatch) * g.pb;
+    V *base = data + (size_t)o * n * g.C + c0;
+    const int pb = (int)(g.C - c0 < g.pb ? g.C - c0 : g.pb);
+    for (int idx = threadIdx.x; idx < n * pb; idx += kThreads) {
+        const int p = idx % pb, e = idx / pb;
+        A[p * ld + e] = base[(size_t)e * g.C + p];
     }
     __syncthreads();
     V *src = A, *dst = B;
@@ -180,62 +278,78 @@ __global__ __launch_bounds__(kThreads) void fft_axis(V *__restrict__ data, int n
         src = dst;
         dst = t;
     }
-    for (int idx = threadIdx.x; idx < n * PB; idx += kThreads) {
-        const int p = idx % PB, e = idx / PB;
-        if (p < pb) {
-            V v = src[p * ld + e];
-            v.x *= scale;
-            v.y *= scale;
-            data[(base + (long long)e * g.es) * np + p0 + p] = v;
-        }
+    for (int idx = threadIdx.x; idx < n * pb; idx += kThreads) {
+        const int p = idx % pb, e = idx / pb;
+        V v = src[p * ld + e];
+        v.x *= scale;
+        v.y *= scale;
+        base[(size_t)e * g.C + p] = v;
     }
 }
 
-
-// ---- line lengths known at compile time: constant divisors and trip counts,
-// twiddles staged in LDS once per workgroup.
-constexpr int pick_radix(int rem) {
-    return (rem % 8 == 0 && rem > 8) ? 8 : (rem % 4 == 0 ? 4 : (rem % 2 == 0 ? 2 : (rem % 3 == 0 ? 3 : 5)));
+// ---- line lengths known at compile time: constant trip counts and twiddle indices, one LDS
+// buffer, the stages staged through registers.  A pass is bound by HBM: 4.8-5.3 TB/s of its one
+// read and one write at 96-180 points, where a plain copy reaches 4.8.  The lengths are those of
+// everyday boxes; the kernel above, with runtime radices, takes three to four times as long (six
+// FP32 passes at 100^3, mmax 4: 3.16 against 1.01 ms; at 180^3, mmax 5: 39.4 against 10.3 ms).
+constexpr bool is_radix(int r) {
+    return r == 2 || r == 3 || r == 4 || r == 5 || r == 6 || r == 8 || r == 9 || r == 10 || r == 12 || r == 15 || r == 16;
 }
+// The radix of the next stage for the remaining factor `rem`: two stages of nearly equal radix
+// where both are at most rmax, else the largest radix.
+constexpr int pick_radix(int rem, int rmax) {
+    int best = 0;
+    for (int r = 2; r <= rmax; r++)
+        if (is_radix(r) && rem % r == 0 && is_radix(rem / r) && rem / r <= rmax && r >= rem / r && !best) best = r;
+    if (best && rem > 5) return best;
+    if (rem <= rmax && is_radix(rem)) return rem;
+    for (int r = rmax; r >= 2; r--)
+        if (is_radix(r) && rem % r == 0) return r;
+    return 0;
+}
+// The largest radix: registers against passes over LDS.  FP64: a butterfly of 16 holds 64
+// registers (128^3: 16 and 8 took 7.85 ms where 8, 4 and 4 took 7.69).
+template <typename V> constexpr int rmax() { return sizeof(V) == 16 ? 10 : 16; }
 
-// In-place variant: one LDS line buffer per projection, the stages staged through
-// registers.  Task t of a stage is (row = t % PB, butterfly j = t / PB), so a wave's
-// consecutive lanes are consecutive projections of one grid point: the first stage
-// reads its inputs straight from HBM and the last writes its outputs straight back,
-// both in the 16 x 8 B (FP32) / 8 x 16 B (FP64) runs of a point record.
-template <int N, int Ns, int REM, int PB, bool FIRST, typename V>
-__device__ inline void run_stages(V *A, const V *twl, decltype(V::x) s, V *__restrict__ data, int np,
-                                  const LineGeom &g, long long base, int p0, int pb, decltype(V::x) scale) {
-    constexpr int R = pick_radix(REM), nb = N / R, ld = N + 1, tstep = N / (Ns * R);
+template <typename V> constexpr int columns() { return 128 / (int)sizeof(V); }
+
+// Task t of a stage is (row = t % pb, butterfly j = t / pb), so a wave's consecutive lanes are
+// consecutive columns: the first stage reads its inputs straight from HBM and the last writes
+// its outputs straight back, in runs of 128 bytes.  LDS holds [element][row].
+template <int N, int Ns, int REM, int T, bool FIRST, typename V>
+__device__ inline void run_stages(V *A, const V *twl, decltype(V::x) s, V *__restrict__ base, size_t es, unsigned pb,
+                                  unsigned magic, unsigned C, size_t ls, decltype(V::x) scale) {
+    constexpr int R = FIRST ? pick_radix(N, rmax<V>()) : (REM <= rmax<V>() && is_radix(REM) ? REM : pick_radix(REM, rmax<V>()));
+    constexpr int nb = N / R, tstep = N / (Ns * R), PB = columns<V>();
     constexpr bool LAST = (REM == R);
-    constexpr int NTASK = PB * nb, NT = (NTASK + kThreads - 1) / kThreads;
+    constexpr int NT = (PB * nb + T - 1) / T;
+    const unsigned ntask = pb * nb;
     V o[NT][R];
+    unsigned off[NT];  // rows past the batch's lines: LDS offset and memory offset of a valid one
 #pragma unroll
     for (int q = 0; q < NT; q++) {
-        const int task = threadIdx.x + q * kThreads;
-        if (NTASK % kThreads != 0 && task >= NTASK) continue;
-        const int row = task % PB, j = task / PB, k = j % Ns;
-        // FIRST: element e = j + r nb of the line at rowbase + r rstep; rows past the batch's
-        // projections are transformed too but never stored: they read the last valid row, so
-        // every load is issued unconditionally (a load under a branch made the wave wait for it
-        // before issuing the next)
-        const long long rowbase = (base + (long long)j * g.es) * np + p0 + (row < pb ? row : pb - 1);
-        const long long rstep = (long long)nb * g.es * np;
+        const unsigned task = threadIdx.x + q * T;
+        if (q > 0 && task >= ntask) continue;
+        const unsigned tk = task < ntask ? task : ntask - 1;
+        const unsigned j = (tk * magic) >> 20, row = tk - j * pb, k = j % Ns;
+        off[q] = (j / Ns * (Ns * R) + k) * pb + row;
         V v[R];
+        if constexpr (FIRST) {
+            // every load is issued unconditionally (a load under a branch made the wave wait for
+            // it before issuing the next)
+            const V *p = base + (ls ? (size_t)(row / C) * ls + row % C : (size_t)row) + (size_t)j * es;
 #pragma unroll
-        for (int r = 0; r < R; r++) {
-            const int e = j + r * nb;
-            V x;
-            if constexpr (FIRST) {
-                x = data[rowbase + r * rstep];
-            } else {
-                x = A[row * ld + e];
+            for (int r = 0; r < R; r++) v[r] = p[(size_t)r * nb * es];
+        } else {
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                V x = A[(j + r * nb) * pb + row];
+                if (r > 0) {
+                    const V w = twl[k * r * tstep];
+                    x = cmul(x, mk<V>(w.x, w.y * s));
+                }
+                v[r] = x;
             }
-            if (r > 0 && Ns > 1) {
-                const V w = twl[(k * r * tstep) % N];
-                x = cmul(x, mk<V>(w.x, w.y * s));
-            }
-            v[r] = x;
         }
         Dft<R, V>::run(v, s);
 #pragma unroll
@@ -244,75 +358,88 @@ __device__ inline void run_stages(V *A, const V *twl, decltype(V::x) s, V *__res
     if constexpr (!FIRST) __syncthreads();  // every read of this stage precedes its in-place writes
 #pragma unroll
     for (int q = 0; q < NT; q++) {
-        const int task = threadIdx.x + q * kThreads;
-        if (NTASK % kThreads != 0 && task >= NTASK) continue;
-        const int row = task % PB, j = task / PB, k = j % Ns;
-        const int ob = (j / Ns) * Ns * R + k;
+        const unsigned task = threadIdx.x + q * T;
+        if (task >= ntask) continue;
+        if constexpr (LAST) {
+            const unsigned j = (task * magic) >> 20, row = task - j * pb, k = j % Ns;
+            const unsigned e = j / Ns * (Ns * R) + k;
+            V *p = base + (ls ? (size_t)(row / C) * ls + row % C : (size_t)row) + (size_t)e * es;
 #pragma unroll
-        for (int r = 0; r < R; r++) {
-            if constexpr (LAST) {
-                if (row < pb) {
-                    V v = o[q][r];
-                    v.x *= scale;
-                    v.y *= scale;
-                    data[(base + (long long)(ob + r * Ns) * g.es) * np + p0 + row] = v;
-                }
-            } else {
-                A[row * ld + ob + r * Ns] = o[q][r];
+            for (int r = 0; r < R; r++) {
+                V v = o[q][r];
+                v.x *= scale;
+                v.y *= scale;
+                p[(size_t)r * Ns * es] = v;
             }
+        } else {
+#pragma unroll
+            for (int r = 0; r < R; r++) A[off[q] + r * Ns * pb] = o[q][r];
         }
     }
     if constexpr (!LAST) {
         __syncthreads();
-        run_stages<N, Ns * R, REM / R, PB, false, V>(A, twl, s, data, np, g, base, p0, pb, scale);
+        run_stages<N, Ns * R, REM / R, T, false, V>(A, twl, s, base, es, pb, magic, C, ls, scale);
     }
 }
 
-template <int N, int PB, typename V>
-__global__ __launch_bounds__(kThreads) void fft_axis_r(V *__restrict__ data, int np, LineGeom g, const double2 *tw,
-                                                      double sgn_d, double scale_d) {
+// threads of a workgroup: the butterflies of its largest stage, at most 256 (one butterfly of the
+// first stage each, which at 128 points of FP64 leaves half of them without a load: 128 threads
+// took 7.14 against 7.00 ms per evaluation)
+template <int N, int REM, typename V> constexpr int stage_tasks() {
+    constexpr int R = REM <= rmax<V>() && is_radix(REM) && REM != N ? REM : pick_radix(REM, rmax<V>());
+    constexpr int t = columns<V>() * (N / R);
+    if constexpr (REM == R) return t;
+    else {
+        constexpr int u = stage_tasks<N, REM / R, V>();
+        return t > u ? t : u;
+    }
+}
+template <int N, typename V> constexpr int fft_threads() {
+    constexpr int t = (stage_tasks<N, N, V>() + 63) / 64 * 64;
+    return t > 256 ? 256 : t;
+}
+
+template <int N, typename V>
+__global__ __launch_bounds__((fft_threads<N, V>())) void fft_cols(V *__restrict__ data, Cols g, unsigned magic,
+                                                                 const double2 *__restrict__ tw, double sgn_d,
+                                                                 double scale_d) {
     using T = decltype(V::x);
-    extern __shared__ __align__(16) unsigned char fft_smem[];
-    V *A = reinterpret_cast<V *>(fft_smem), *twl = A + PB * (N + 1);
-    const T sgn = (T)sgn_d, scale = (T)scale_d;
-    int line = blockIdx.x, by = blockIdx.y;
-    if (((g.es == 1 && np % PB != 0) || g.align > 0) && ((gridDim.x * gridDim.y) & 7) == 0) {
-        // cache lines shared between workgroups: along x the PB-runs of every other point
-        // straddle two lines, whose other halves belong to the neighbouring batches of the
-        // same line; with aligned batches (y, z) the partial lines at the ends of a point's
-        // record belong to the neighbouring lines.  Workgroups go to the 8 XCDs round robin
-        // in dispatch order, so each XCD (one L2) is given a contiguous range of lines with
-        // the batches of each line in consecutive slots: a shared line is read from HBM once
-        const unsigned id = blockIdx.x + gridDim.x * blockIdx.y, per = gridDim.x * gridDim.y / 8;
-        const unsigned G = (id & 7) * per + (id >> 3);
-        line = (int)(G / gridDim.y);
-        by = (int)(G % gridDim.y);
-    }
-    const int a = line % g.na, b = line / g.na;
-    const long long base = (long long)a * g.sa + (long long)b * g.sb;
-    int p0, pb;
-    const int s = g.align > 0 ? (int)((g.align - (base * np) % g.align) % g.align) : 0;
-    if (s == 0) {
-        p0 = by * PB;
-        pb = (np - p0) < PB ? (np - p0) : PB;
+    constexpr int TH = fft_threads<N, V>();
+    __shared__ V A[columns<V>() * N];
+    __shared__ V twl[N];
+    const unsigned id = xcd_order(g.run);
+    if (id >= g.nwg) return;
+    V *base;
+    unsigned pb = g.pb;
+    size_t ls = 0;
+    if (g.lines > 1) {
+        const unsigned o = id * g.lines, nl = g.nouter - o < g.lines ? g.nouter - o : g.lines;
+        base = data + (size_t)o * N * g.C;
+        pb = nl * (unsigned)g.C;
+        ls = (size_t)N * g.C;
     } else {
-        p0 = by == 0 ? 0 : s + (by - 1) * PB;
-        pb = by == 0 ? s : ((np - p0) < PB ? (np - p0) : PB);
+        const unsigned o = id / g.nbatch;
+        const size_t c0 = (size_t)(id - o * g.nbatch) * g.pb;
+        base = data + (size_t)o * N * g.C + c0;
+        if (g.C - c0 < pb) pb = (unsigned)(g.C - c0);
     }
-    if (pb <= 0) return;
-    for (int i = threadIdx.x; i < N; i += kThreads) twl[i] = mk<V>((T)tw[i].x, (T)tw[i].y);
-    __syncthreads();
-    run_stages<N, 1, N, PB, true, V>(A, twl, sgn, data, np, g, base, p0, pb, scale);
+    if (pb != g.pb) magic = (1u << 20) / pb + 1;
+    for (int i = threadIdx.x; i < N; i += TH) twl[i] = mk<V>((T)tw[i].x, (T)tw[i].y);
+    // (the barrier that ends the first stage covers the twiddles)
+    run_stages<N, 1, N, TH, true, V>(A, twl, (T)sgn_d, base, g.C, pb, magic, (unsigned)g.C, ls, (T)scale_d);
 }
 
-template <int PB, typename V>
-bool launch_axis_c(int n, dim3 grid, hipStream_t st, V *proj, int np, const LineGeom &g, const double2 *tw,
-                   double sign, double scale) {
-    const size_t lds = sizeof(V) * ((size_t)PB * (n + 1) + n);
+template <typename V>
+bool launch_cols(int n, const Cols &g, hipStream_t st, V *proj, const double2 *tw, double sign, double scale) {
+    const dim3 grid((g.nwg + 8 * g.run - 1) / (8 * g.run) * 8 * g.run);
+    const unsigned magic = (1u << 20) / g.pb + 1;  // exact quotients of task < 4096 by pb <= 16
     switch (n) {
 #define FFT_C(NN) \
-    case NN: hipLaunchKernelGGL((fft_axis_r<NN, PB, V>), grid, dim3(kThreads), lds, st, proj, np, g, tw, sign, scale); return true;
-        FFT_C(16) FFT_C(32) FFT_C(48) FFT_C(64) FFT_C(96) FFT_C(128) FFT_C(192) FFT_C(256)
+    case NN: hipLaunchKernelGGL((fft_cols<NN, V>), grid, dim3(fft_threads<NN, V>()), 0, st, proj, g, magic, tw, sign, scale); return true;
+        FFT_C(16) FFT_C(18) FFT_C(20) FFT_C(24) FFT_C(25) FFT_C(27) FFT_C(30) FFT_C(32) FFT_C(36) FFT_C(40) FFT_C(45)
+        FFT_C(48) FFT_C(50) FFT_C(54) FFT_C(60) FFT_C(64) FFT_C(72) FFT_C(75) FFT_C(80) FFT_C(81) FFT_C(90) FFT_C(96)
+        FFT_C(100) FFT_C(108) FFT_C(120) FFT_C(125) FFT_C(128) FFT_C(144) FFT_C(150) FFT_C(160) FFT_C(180) FFT_C(192)
+        FFT_C(200) FFT_C(240) FFT_C(256)
 #undef FFT_C
         default: return false;
     }
@@ -320,41 +447,40 @@ bool launch_axis_c(int n, dim3 grid, hipStream_t st, V *proj, int np, const Line
 
 template <typename V>
 hipError_t launch_fft3d(mdft_ctx *c, V *proj, int sign, int batch) {
-    const int nx = c->d.nx, ny = c->d.ny, nz = c->d.nz, np = batch > 0 ? batch : c->np;
-    const double scale_last = (sign < 0) ? 1.0 / (double)((long long)nx * ny * nz) : 1.0;
-    LineGeom geo[3] = {
-        {nx, 1, ny, (long long)nx, (long long)nx * ny, 0},
-        {ny, (long long)nx, nx, 1, (long long)nx * ny, 0},
-        {nz, (long long)nx * ny, nx, 1, (long long)nx, 0},
-    };
-    // PB projections per workgroup: 8 (FP64) or 16 (FP32) keeps 128-byte runs per grid point
-    constexpr int PBmax = sizeof(V) == 16 ? 8 : 16;
-    const int PB = (np % PBmax == 0 || np > PBmax) ? PBmax : 4;
-    // a point record of np elements that is not a whole number of cache lines puts the
-    // runs of odd points (say) across two lines; along an axis whose point stride times
-    // np is a whole number of lines, every point of a line shares the offset, and the
-    // batches can start on line boundaries (one more, shorter, batch per line)
-    for (int ax = 0; ax < 3; ax++)
-        if (PB == PBmax && (np % PBmax) != 0 && (geo[ax].es * np) % PBmax == 0) geo[ax].align = PBmax;
+    const int n[3] = {c->d.nx, c->d.ny, c->d.nz};
+    const size_t np = batch > 0 ? batch : c->np;
+    const double scale_last = (sign < 0) ? 1.0 / (double)((long long)n[0] * n[1] * n[2]) : 1.0;
+    size_t C = np;
     for (int ax = 0; ax < 3; ax++) {
-        const LineGeom &g = geo[ax];
-        const size_t lines = c->N / (size_t)g.n;
-        dim3 grid((unsigned)lines, (unsigned)((np + PB - 1) / PB + (g.align > 0 ? 1 : 0)));
         const double scale = (ax == 2) ? scale_last : 1.0;
-        const size_t lds = sizeof(V) * 2 * (size_t)PB * (g.n + 1);
-        if (PB == PBmax && launch_axis_c<PBmax, V>(g.n, grid, c->stream, proj, np, g, c->fft[ax].tw, (double)sign, scale)) {
-            hipError_t e = hipGetLastError();
-            if (e != hipSuccess) return e;
-            continue;
+        const unsigned PB = columns<V>();
+        Cols g;
+        g.C = C;
+        g.nouter = (unsigned)(c->N * np / (C * n[ax]));
+        g.lines = 1;
+        // equal batches: np = 70 in FP32 is 5 x 14, not 4 x 16 + 6
+        g.nbatch = (unsigned)((C + PB - 1) / PB);
+        g.pb = (unsigned)((C + g.nbatch - 1) / g.nbatch);
+        if (2 * C <= PB) {  // few columns: whole lines of several outer indices
+            g.lines = (unsigned)(PB / C);
+            g.pb = (unsigned)(g.lines * C);
+            g.nbatch = 1;
         }
-        if (PB == PBmax)
-            hipLaunchKernelGGL((fft_axis<PBmax, V>), grid, dim3(kThreads), lds, c->stream, proj, np, g, c->fft[ax],
-                               (double)sign, scale);
-        else
-            hipLaunchKernelGGL((fft_axis<4, V>), grid, dim3(kThreads), lds, c->stream, proj, np, g, c->fft[ax],
-                               (double)sign, scale);
-        hipError_t e = hipGetLastError();
+        g.nwg = g.lines > 1 ? (g.nouter + g.lines - 1) / g.lines : g.nouter * g.nbatch;
+        g.run = g.nwg < 8 * kRun ? (g.nwg + 7) / 8 : kRun;
+        if (!launch_cols<V>(n[ax], g, c->stream, proj, c->fft[ax].tw, (double)sign, scale)) {
+            if (g.lines > 1) {
+                g.lines = 1;
+                g.pb = g.C;
+                g.nwg = g.nouter;
+            }
+            const size_t lds = sizeof(V) * 2 * (size_t)g.pb * (n[ax] + 1);
+            hipLaunchKernelGGL((fft_axis<V>), dim3((g.nwg + 8 * g.run - 1) / (8 * g.run) * 8 * g.run), dim3(kThreads), lds, c->stream, proj, g,
+                               c->fft[ax], (double)sign, scale);
+        }
+        const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
+        C *= n[ax];
     }
     return hipSuccess;
 }

@@ -16,6 +16,7 @@
 #include <cfloat>
 
 #include "mdft_internal.h"
+#include "turns.h"
 
 namespace {
 
@@ -359,118 +360,144 @@ __device__ inline unsigned mul24(unsigned a, unsigned b) {
     return r;
 }
 
-// The constant tables of angl2proj_t in the layout of its LDS.  The image is built once per
-// context and precision (a2p_tab_build, the staging arithmetic run once) and each workgroup
-// copies it with 16-byte loads: the index arithmetic and FP64 -> T conversions of the
-// staging then run once instead of once per 4-point tile.
-template <int L, typename T> struct alignas(16) A2pTab {
-    using V = typename C2<T>::t;
+// ---- the angular transforms by rows.  A row holds the values of one (point, theta) over
+// (phi, psi), NPHI NPSI of them, and after the two DFTs its NF complex coefficients (mup, mu2):
+// mu2 = 0: mup = 0 .. L (the others are their conjugates, the values being real), mu2 = 1 .. H:
+// mup = -L .. L.  One thread transforms a row in registers, in place in LDS: both DFTs are of odd
+// length n, so the terms j and n - j are added and subtracted first and the outputs k and -k share
+// the sums, a third of the multiply-adds of the plain sums, and each value is read and written once
+// (one thread per output reads n values and n twiddles for each).
+template <int L> struct Rows : Dims<L> {
     using D = Dims<L>;
-    V twpsi[D::H1 * D::NPSI];  // (cos, sin)(2 pi mu2 ipsi / npsi) at [mu2][ipsi]
-    V twphi[D::W * D::NPHI];   // (cos, sin)(2 pi mup iphi / nphi) / (nphi npsi) at [mup + L][iphi]
-    T a2p[D::NP * D::NTH], fmv[D::NP];
-    int pmup[D::NP], pmu2[D::NP];
+    static constexpr int ROW = D::NPHI * D::NPSI, NF = L + 1 + D::H * D::W;
+    static constexpr int RS = (ROW > 2 * NF ? ROW : 2 * NF) | 1;  // odd: consecutive rows in different banks
+    static constexpr int item(int mup, int mu2) { return mu2 == 0 ? mup : L + 1 + (mu2 - 1) * D::W + mup + L; }
 };
 
-template <int L, typename T>
-__global__ __launch_bounds__(kThreads) void a2p_tab_build(A2pTab<L, T> *__restrict__ out, AngTables t) {
-    using D = Dims<L>;
-    using V = typename C2<T>::t;
-    constexpr int NP = D::NP, NTH = D::NTH, NPHI = D::NPHI, NPSI = D::NPSI, H1 = D::H1, W = D::W;
-    const int tid = threadIdx.x;
-    for (int i = tid; i < H1 * NPSI; i += kThreads) {
-        const int kk = ((i / NPSI) * (i % NPSI)) % NPSI;
-        out->twpsi[i] = mk<V>((T)t.cps[kk], (T)t.sps[kk]);
+// X(k) = sum_j x_j e^{+2 pi i j k / N}, k = -L .. L (at L + k), N = 2 L + 1
+template <int N, typename T>
+__device__ __forceinline__ void dft_odd(const T (&x)[N], const T (&y)[N], T (&ox)[N], T (&oy)[N]) {
+    constexpr int L = N / 2;
+    constexpr Turns<T, N> tw;
+    T sx[L + 1], sy[L + 1], dx[L + 1], dy[L + 1];
+    T x0 = x[0], y0 = y[0];
+#pragma unroll
+    for (int j = 1; j <= L; j++) {
+        sx[j] = x[j] + x[N - j];
+        sy[j] = y[j] + y[N - j];
+        dx[j] = x[j] - x[N - j];
+        dy[j] = y[j] - y[N - j];
+        x0 += sx[j];
+        y0 += sy[j];
     }
-    for (int i = tid; i < W * NPHI; i += kThreads) {
-        const int mup = i / NPHI - L, iphi = i % NPHI;
-        int kk = (mup * iphi) % NPHI;
-        kk += (kk < 0) ? NPHI : 0;
-        const double nrm = 1.0 / (double)(NPHI * NPSI);
-        out->twphi[i] = mk<V>((T)(t.cph[kk] * nrm), (T)(t.sph[kk] * nrm));
-    }
-    for (int i = tid; i < NP * NTH; i += kThreads) out->a2p[i] = (T)t.a2p[i];
-    for (int i = tid; i < NP; i += kThreads) {
-        out->fmv[i] = (T)t.fm[i];
-        out->pmup[i] = t.pmup[i];
-        out->pmu2[i] = t.pmu[i] / 2;
+    ox[L] = x0;
+    oy[L] = y0;
+#pragma unroll
+    for (int k = 1; k <= L; k++) {
+        T ax = x[0], ay = y[0], bx = 0, by = 0;  // the cos sum, and the sin sum times i
+#pragma unroll
+        for (int j = 1; j <= L; j++) {
+            const T c = tw.c[(j * k) % N], s = tw.s[(j * k) % N];
+            ax = fma(sx[j], c, ax);
+            ay = fma(sy[j], c, ay);
+            bx = fma(-dy[j], s, bx);
+            by = fma(dx[j], s, by);
+        }
+        ox[L + k] = ax + bx;
+        oy[L + k] = ay + by;
+        ox[L - k] = ax - bx;
+        oy[L - k] = ay - by;
     }
 }
 
-// The psi, phi and theta steps of angl2proj over one tile (o in LDS and visible to every
-// thread): G (psi DFT), F (phi DFT), then the theta contraction into the tile's projections.
-template <int L, int PT, typename T>
-__device__ inline void a2p_phases(const T *o, typename C2<T>::t *G, typename C2<T>::t *F, const A2pTab<L, T> &tb,
-                                  typename C2<T>::t *__restrict__ dst, int npts, int tid) {
-    using D = Dims<L>;
-    using V = typename C2<T>::t;
-    constexpr int NP = D::NP, NTH = D::NTH, NPHI = D::NPHI, NPSI = D::NPSI, H1 = D::H1, W = D::W;
-    const V *twpsi = tb.twpsi, *twphi = tb.twphi;
-    const T *a2p = tb.a2p, *fmv = tb.fmv;
-    const int *pmup = tb.pmup, *pmu2 = tb.pmu2;
-    for (int i = tid; i < npts * NTH * NPHI * H1; i += kThreads) {
-        const int mu2 = i % H1;
-        const T *line = o + (i / H1) * NPSI;
-        const V *tw = twpsi + mu2 * NPSI;
-        T re = 0, im = 0;
+template <int L, typename T> __device__ __forceinline__ void row_to_coefficients(T *row) {
+    using R = Rows<L>;
+    constexpr int NPHI = R::NPHI, NPSI = R::NPSI, H = R::H;
+    constexpr Turns<T, NPHI> tw;
+    constexpr Turns<T, NPSI> tp;
+    T g0[NPHI], gx[H > 0 ? H : 1][NPHI], gy[H > 0 ? H : 1][NPHI];
 #pragma unroll
-        for (int ipsi = 0; ipsi < NPSI; ipsi++) {
-            const T v = line[ipsi];
-            re += v * tw[ipsi].x;
-            im += v * tw[ipsi].y;
+    for (int j = 0; j < NPHI; j++) {
+        const T v0 = row[j * NPSI];
+        T s[H + 1], d[H + 1];
+        g0[j] = v0;
+#pragma unroll
+        for (int p = 1; p <= H; p++) {
+            const T a = row[j * NPSI + p], b = row[j * NPSI + NPSI - p];
+            s[p] = a + b;
+            d[p] = a - b;
+            g0[j] += s[p];
         }
-        G[i] = mk<V>(re, im);
-    }
-    __syncthreads();
-    for (int i = tid; i < npts * NTH * W * H1; i += kThreads) {
-        const int mu2 = i % H1;
-        const int rest = i / H1;
-        const int jm = rest % W;  // mup + L
-        const V *g = G + (rest / W) * NPHI * H1 + mu2;
-        const V *tw = twphi + jm * NPHI;
-        T re = 0, im = 0;
 #pragma unroll
-        for (int iphi = 0; iphi < NPHI; iphi++) {
-            const V v = g[iphi * H1], e = tw[iphi];
-            if constexpr (sizeof(T) == 4) {
-                // four multiply-adds per complex product (the plain expression compiles to six;
-                // in FP64 the plain form keeps the kernel's register count)
-                re = fma(v.x, e.x, re);
-                re = fma(-v.y, e.y, re);
-                im = fma(v.x, e.y, im);
-                im = fma(v.y, e.x, im);
-            } else {
-                re += v.x * e.x - v.y * e.y;
-                im += v.x * e.y + v.y * e.x;
+        for (int mu = 1; mu <= H; mu++) {
+            T x = v0, y = 0;
+#pragma unroll
+            for (int p = 1; p <= H; p++) {
+                x = fma(s[p], tp.c[(mu * p) % NPSI], x);
+                y = fma(d[p], tp.s[(mu * p) % NPSI], y);
             }
+            gx[mu - 1][j] = x;
+            gy[mu - 1][j] = y;
         }
-        F[i] = mk<V>(re, im);
     }
-    __syncthreads();
-    auto theta = [&](int pt, int ip) {
-        const V *f = F + (pt * NTH * W + (pmup[ip] + L)) * H1 + pmu2[ip];
-        const T *a = a2p + ip * NTH;
-        T re = 0, im = 0;
+    // mu2 = 0: real values, mup = 0 .. L
+    {
+        T x0 = g0[0], s[L + 1], d[L + 1];
 #pragma unroll
-        for (int it = 0; it < NTH; it++) {
-            const V v = f[it * W * H1];
-            re += v.x * a[it];
-            im += v.y * a[it];
+        for (int j = 1; j <= L; j++) {
+            s[j] = g0[j] + g0[NPHI - j];
+            d[j] = g0[j] - g0[NPHI - j];
+            x0 += s[j];
         }
-        return mk<V>(re * fmv[ip], im * fmv[ip]);
-    };
-    if constexpr (sizeof(T) == 4 && NP % 2 == 0) {
-        // FP32: two projections of a point per thread, one 16-byte store
-        for (int i = tid; i < npts * (NP / 2); i += kThreads) {
-            const int pt = i / (NP / 2), ip = 2 * (i - pt * (NP / 2));
-            const V u0 = theta(pt, ip), u1 = theta(pt, ip + 1);
-            reinterpret_cast<float4 *>(dst)[i] = make_float4(u0.x, u0.y, u1.x, u1.y);
+        row[0] = x0;
+        row[1] = x0;  // mup = 0 is real: its slot holds the value twice (see OutLane)
+#pragma unroll
+        for (int k = 1; k <= L; k++) {
+            T a = g0[0], b = 0;
+#pragma unroll
+            for (int j = 1; j <= L; j++) {
+                a = fma(s[j], tw.c[(j * k) % NPHI], a);
+                b = fma(d[j], tw.s[(j * k) % NPHI], b);
+            }
+            row[2 * k] = a;
+            row[2 * k + 1] = b;
         }
-    } else {
-        for (int i = tid; i < npts * NP; i += kThreads) {
-            const int pt = i / NP, ip = i - pt * NP;
-            dst[i] = theta(pt, ip);
+    }
+#pragma unroll
+    for (int mu = 0; mu < H; mu++) {
+        T ox[NPHI], oy[NPHI];
+        dft_odd<NPHI, T>(gx[mu], gy[mu], ox, oy);
+#pragma unroll
+        for (int k = 0; k < NPHI; k++) {
+            row[2 * (L + 1 + mu * NPHI + k)] = ox[k];
+            row[2 * (L + 1 + mu * NPHI + k) + 1] = oy[k];
         }
+    }
+}
+
+// One projection of the theta contraction: out = (sum_it ax[it] F_it.x, sum_it ay[it] F_it.y) with
+// F_it the coefficient at `item` of the rows of a point.  The signs of mup < 0 at mu2 = 0 (the
+// conjugate of mup > 0 times (-1)^mup) and all norms are in the weights.
+template <int L, typename T> struct OutLane {
+    T ax[L + 1], ay[L + 1];
+    int item;
+};
+
+template <int L, typename T>
+__global__ void out_lanes_build(OutLane<L, T> *__restrict__ out, AngTables t) {
+    using R = Rows<L>;
+    for (int ip = threadIdx.x; ip < R::NP; ip += blockDim.x) {
+        const int mup = t.pmup[ip], mu2 = t.pmu[ip] / 2;
+        const bool conj = mu2 == 0 && mup < 0;
+        OutLane<L, T> o;
+        for (int it = 0; it < R::NTH; it++) {
+            const double a = t.a2p[ip * R::NTH + it] * t.fm[ip] / (double)(R::NPHI * R::NPSI);
+            // d^m(mup, 0) already has the sign (-1)^mup of d^m(-mup, 0)
+            o.ax[it] = (T)a;
+            o.ay[it] = (T)(mu2 == 0 && mup == 0 ? 0.0 : (conj ? -a : a));
+        }
+        o.item = R::item(conj ? -mup : mup, mu2);
+        out[ip] = o;
     }
 }
 
@@ -482,59 +509,73 @@ __device__ inline void a2p_phases(const T *o, typename C2<T>::t *G, typename C2<
 // density guess xi and k0 = dv / 2: dF/dr / w for r = rho/rho0, whose angl2proj is the
 // adjoint of proj2angl up to a per-projection factor (the warm start's training gradient);
 // feat = 4: o = xi (the plain transform). k0 is rho0 for feat 0.
-template <int L, int PT, typename T>
-__global__ __launch_bounds__(kThreads) void angl2proj_t(const double *__restrict__ xi, typename C2<T>::t *__restrict__ proj,
-                                                       size_t N, AngTables t, double k0, int feat, double beta,
-                                                       const double *__restrict__ aux,
-                                                       const double *__restrict__ vsinv,
-                                                       const float *__restrict__ xi32,
-                                                       const A2pTab<L, T> *__restrict__ img) {
-    using D = Dims<L>;
+// Bound by HBM: at 128^3, mmax 5 it reads 5.5 GB of FP64 xi and writes 1.5 (FP32) or 3.0 GB (FP64
+// projections) in 1.22 and 1.79 ms, 5.7 and 4.8 TB/s.  (One thread per psi sum, per phi sum and per
+// projection, tables in LDS: 2.22 and 3.72 ms, the time of its reads of values and twiddles from LDS.)
+// The theta contraction gives a thread one projection, its weights in registers, and a group of
+// threads consecutive projections of a point, so the stores are whole records.
+template <int L, int PT, int TH, typename T>
+__global__ __launch_bounds__(TH) void angl2proj_t(const double *__restrict__ xi, typename C2<T>::t *__restrict__ proj,
+                                                 size_t N, AngTables t, double k0, int feat, double beta,
+                                                 const double *__restrict__ aux, const double *__restrict__ vsinv,
+                                                 const float *__restrict__ xi32,
+                                                 const OutLane<L, T> *__restrict__ lanes) {
+    using R = Rows<L>;
     using V = typename C2<T>::t;
-    constexpr int NO = D::NO, NP = D::NP, NTH = D::NTH, NPHI = D::NPHI, H1 = D::H1, W = D::W;
-    // o (read by the psi step) and F (written by the phi step, after the barrier that ends
-    // the psi step) share their LDS: the smaller footprint lets more workgroups share a CU
-    constexpr size_t kOB = sizeof(T) * PT * NO, kFB = sizeof(V) * PT * NTH * W * H1;
-    __shared__ __align__(16) unsigned char oF[kOB > kFB ? kOB : kFB];
-    __shared__ V G[PT * NTH * NPHI * H1];
-    __shared__ A2pTab<L, T> tb;
-    T *o = reinterpret_cast<T *>(oF);
-    V *F = reinterpret_cast<V *>(oF);
+    constexpr int NO = R::NO, NTH = R::NTH, NOUT = R::NP, ROW = R::ROW, RS = R::RS;
+    __shared__ T rows[NTH * PT * RS];  // row of (point, theta) at theta PT + point
+    __shared__ double sth[NTH];        // 1 / s of each theta (the weights, hence s, depend on theta only)
     const int tid = threadIdx.x;
     const size_t r0 = (size_t)blockIdx.x * PT;
     const int npts = (int)((N - r0) < (size_t)PT ? (N - r0) : (size_t)PT);
-    // the tile's FP64 input is loaded into registers before the tables are staged,
-    // so its HBM latency overlaps the staging
-    constexpr int NIT = (PT * NO + kThreads - 1) / kThreads;
+    // all of a thread's loads are issued before the first is used
+    constexpr int NIT = (PT * NO + TH - 1) / TH;
     const double *src = xi + r0 * NO;
-    double xr[NIT], sr[NIT];
+    double xr[NIT];
 #pragma unroll
     for (int q = 0; q < NIT; q++) {
-        const int i = tid + q * kThreads;
+        const int i = tid + q * TH;
         xr[q] = (i < npts * NO) ? (xi32 ? hold_f32(xi32[r0 * NO + i]) : src[i]) : 0.0;  // FP32 iterate: xi32
-        sr[q] = vsinv ? vsinv[i % NO] : 1.0;  // scaled variables: xi = u / s(io), loaded with the tile
     }
-    {
-        constexpr int n16 = (int)(sizeof(A2pTab<L, T>) / 16);
-        const uint4 *src16 = reinterpret_cast<const uint4 *>(img);
-        uint4 *dst16 = reinterpret_cast<uint4 *>(&tb);
-        for (int i = tid; i < n16; i += kThreads) dst16[i] = src16[i];
-    }
+    constexpr int G = TH / NOUT;  // groups of NOUT threads: each takes every G-th point of the theta contraction
+    static_assert(G >= 1, "a projection per thread");
+    const int grp = tid / NOUT, ip = tid - grp * NOUT;
+    const OutLane<L, T> ln = lanes[ip];
+    if (tid < NTH) sth[tid] = vsinv ? vsinv[tid * ROW] : 1.0;
+    __syncthreads();
 #pragma unroll
     for (int q = 0; q < NIT; q++) {
-        const int i = tid + q * kThreads;
+        const int i = tid + q * TH;
         if (i >= npts * NO) break;
+        const unsigned pt = DivC<NO, PT * NO>::q(i);
+        const unsigned io = i - mul24(pt, NO), it = DivC<ROW, NO>::q(io);
+        T &o = rows[mul24(mul24(it, PT) + pt, RS) + (io - mul24(it, ROW))];
         const double xv = xi32 ? held_f32(xr[q]) : xr[q];
-        const double x = vsinv ? xv * sr[q] : xv;
-        if (feat == 0) o[i] = (T)(k0 * (x * x - 1.0));
-        else if (feat == 1) o[i] = (T)(0.25 * fmin(fmax(-0.5 * beta * x, -4.0), 4.0));
-        else if (feat == 2) o[i] = (T)(x * x - 1.0);
-        else if (feat == 4) o[i] = (T)x;
-        else o[i] = (x * x > MDFT_WS_DENSITY_FLOOR * (1.0 + 1e-12)) ? (T)(k0 * aux[r0 * NO + i] / (x * t.w[i % NO]))
-                                                                   : (T)0;
+        const double x = vsinv ? xv * sth[it] : xv;  // scaled variables: xi = u / s
+        if (feat == 0) o = (T)(k0 * (x * x - 1.0));
+        else if (feat == 1) o = (T)(0.25 * fmin(fmax(-0.5 * beta * x, -4.0), 4.0));
+        else if (feat == 2) o = (T)(x * x - 1.0);
+        else if (feat == 4) o = (T)x;
+        else o = (x * x > MDFT_WS_DENSITY_FLOOR * (1.0 + 1e-12)) ? (T)(k0 * aux[r0 * NO + i] / (x * t.w[io])) : (T)0;
     }
     __syncthreads();
-    a2p_phases<L, PT, T>(o, G, F, tb, proj + r0 * NP, npts, tid);
+    // points past the end leave their rows unread: nothing of them is stored
+    for (int i = tid; i < NTH * PT; i += TH) row_to_coefficients<L, T>(rows + i * RS);
+    __syncthreads();
+    if (grp < G) {
+        const T *f0 = rows + 2 * ln.item;
+        V *dst = proj + r0 * NOUT + ip;
+        for (int pt = grp; pt < npts; pt += G) {
+            T re = 0, im = 0;
+#pragma unroll
+            for (int it = 0; it < NTH; it++) {
+                const T *f = f0 + (it * PT + pt) * RS;
+                re = fma(f[0], ln.ax[it], re);
+                im = fma(f[1], ln.ay[it], im);
+            }
+            dst[(size_t)pt * NOUT] = mk<V>(re, im);
+        }
+    }
 }
 
 // Persistent: each workgroup stages the tables once and then takes tiles blockIdx.x,
@@ -921,23 +962,33 @@ hipError_t ensure_partials(mdft_ctx *c, size_t nblocks) {
 
 }  // namespace
 
-template <int PT, typename T>
+// Points per workgroup and threads of angl2proj_t: about as many rows (L + 1 per point) as a
+// workgroup's threads can take in one round, in LDS that leaves three or more workgroups on a
+// compute unit.  Measured at 128^3, mmax 5, FP32 / FP64: 16 points, 256 threads 1.22 / 1.79 ms, 128
+// threads 1.26 / 2.47; 32 points 1.26 / 3.69 (one FP64 workgroup per compute unit); 8 points, 128
+// threads 1.27 / 1.78.  100^3, mmax 4, FP64: 192 threads 0.54, 256 0.64 ms.
+template <int L> struct A2pShape {
+    static constexpr int PT = L >= 4 ? 16 : L == 3 ? 32 : L == 2 ? 64 : L == 1 ? 128 : 256, TH = L == 4 ? 192 : 256;
+};
+
+template <typename T>
 bool launch_a2p_t(mdft_ctx *c, const double *xi, typename C2<T>::t *proj, int feat = 0, const double *aux = nullptr,
                   size_t npts = 0) {
     if (!npts) npts = c->N;
-    const size_t nb = (npts + PT - 1) / PT;
     const double beta = 1.0 / c->d.kT;
     const double k0 = (feat == 3) ? 0.5 * c->dv : c->rho0;
     void *&img = c->d_a2p_img[sizeof(T) == 8];
     switch (c->L) {
 #define A2P_CASE(LL) \
-    case LL: \
+    case LL: { \
+        using S = A2pShape<LL>; \
         if (!img) { \
-            if (hipMalloc(&img, sizeof(A2pTab<LL, T>)) != hipSuccess) { img = nullptr; return false; } \
-            hipLaunchKernelGGL((a2p_tab_build<LL, T>), dim3(1), dim3(kThreads), 0, c->stream, static_cast<A2pTab<LL, T> *>(img), c->ang); \
+            if (hipMalloc(&img, sizeof(OutLane<LL, T>) * Rows<LL>::NP) != hipSuccess) { img = nullptr; return false; } \
+            hipLaunchKernelGGL((out_lanes_build<LL, T>), dim3(1), dim3(128), 0, c->stream, static_cast<OutLane<LL, T> *>(img), c->ang); \
         } \
-        hipLaunchKernelGGL((angl2proj_t<LL, PT, T>), dim3((unsigned)nb), dim3(kThreads), 0, c->stream, xi, proj, npts, c->ang, k0, feat, beta, aux, feat == 0 ? c->vsinv : nullptr, feat == 0 ? c->xi32 : nullptr, static_cast<const A2pTab<LL, T> *>(img)); \
-        return true;
+        hipLaunchKernelGGL((angl2proj_t<LL, S::PT, S::TH, T>), dim3((unsigned)((npts + S::PT - 1) / S::PT)), dim3(S::TH), 0, c->stream, xi, proj, npts, c->ang, k0, feat, beta, aux, feat == 0 ? c->vsinv : nullptr, feat == 0 ? c->xi32 : nullptr, static_cast<const OutLane<LL, T> *>(img)); \
+        return true; \
+    }
         A2P_CASE(0) A2P_CASE(1) A2P_CASE(2) A2P_CASE(3) A2P_CASE(4) A2P_CASE(5)
 #undef A2P_CASE
         default: return false;
@@ -981,7 +1032,7 @@ constexpr int kPTt = 4;   // points per workgroup of the specialised kernels, FP
 constexpr int kPT32 = 4;  // the same for FP32 (8 measured slower at 128^3, mmax = 5)
 
 hipError_t launch_angl2proj_f64(mdft_ctx *c, const double *xi, double2 *proj) {
-    if (c->d.mrso == 2 && launch_a2p_t<kPTt, double>(c, xi, proj)) return hipGetLastError();
+    if (c->d.mrso == 2 && launch_a2p_t<double>(c, xi, proj)) return hipGetLastError();
     const size_t nb = (c->N + kPT - 1) / kPT;
     if (a2p_lds(c->ang) > c->lds_limit) return hipErrorInvalidConfiguration;
     hipLaunchKernelGGL(angl2proj_f64<kPT>, dim3((unsigned)nb), dim3(kThreads), a2p_lds(c->ang), c->stream, xi, proj,
@@ -1062,7 +1113,7 @@ FinalConsts final_consts(mdft_ctx *c) {
 }
 
 hipError_t launch_angl2proj_f32(mdft_ctx *c, const double *xi, float2 *proj) {
-    if (c->d.mrso != 2 || !launch_a2p_t<kPT32, float>(c, xi, proj)) return hipErrorNotSupported;
+    if (c->d.mrso != 2 || !launch_a2p_t<float>(c, xi, proj)) return hipErrorNotSupported;
     return hipGetLastError();
 }
 
@@ -1084,8 +1135,8 @@ hipError_t launch_angl2proj_feat(mdft_ctx *c, const double *src, int feat, const
     if (c->d.mrso != 2) return hipErrorNotSupported;
     if (!aux) aux = c->d_vext;
     bool ok = (c->d.precision == MDFT_PREC_FP64)
-                  ? launch_a2p_t<kPTt, double>(c, src, static_cast<double2 *>(c->d_proj), feat, aux)
-                  : launch_a2p_t<kPT32, float>(c, src, static_cast<float2 *>(c->d_proj), feat, aux);
+                  ? launch_a2p_t<double>(c, src, static_cast<double2 *>(c->d_proj), feat, aux)
+                  : launch_a2p_t<float>(c, src, static_cast<float2 *>(c->d_proj), feat, aux);
     return ok ? hipGetLastError() : hipErrorNotSupported;
 }
 
@@ -1093,7 +1144,7 @@ hipError_t launch_angl2proj_feat(mdft_ctx *c, const double *src, int feat, const
 // proj [npts][np] = angl2proj(f [npts][no]) and f = proj2angl(proj); mrso = 2 kernels.
 hipError_t launch_transform_f64(mdft_ctx *c, const double *f, double2 *proj, size_t npts, bool to_proj) {
     if (c->d.mrso != 2) return hipErrorNotSupported;
-    if (to_proj) return launch_a2p_t<kPTt, double>(c, f, proj, 4, nullptr, npts) ? hipGetLastError() : hipErrorNotSupported;
+    if (to_proj) return launch_a2p_t<double>(c, f, proj, 4, nullptr, npts) ? hipGetLastError() : hipErrorNotSupported;
     hipError_t e = ensure_partials(c, (npts + kPTt - 1) / kPTt);
     if (e != hipSuccess) return e;
     return launch_final_t<kPTt, double>(c, proj, nullptr, const_cast<double *>(f), 5, final_consts(c), npts)

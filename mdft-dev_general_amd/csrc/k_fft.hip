@@ -10,6 +10,7 @@
 // lines back.  Along y and z the columns of a workgroup may belong to two grid points,
 // so that every workgroup but the last has PB of them whatever np is.
 #include "mdft_internal.h"
+#include "turns.h"
 
 namespace {
 
@@ -104,38 +105,6 @@ struct Dft<8, V> {
         }
     }
 };
-
-// cos and sin of 2 pi k / n as compile-time constants: the angle is folded into [0, pi / 4]
-// by its index (exact), where the Taylor series to x^23 is correct to the last bits
-constexpr double kPi = 3.14159265358979323846;
-constexpr double taylor(double x, int first) {  // first 0: cos, 1: sin
-    double t = first ? x : 1.0, s = 0.0;
-    double terms[12] = {};
-    for (int i = 0; i < 12; i++) {
-        terms[i] = t;
-        t *= -x * x / (double)((2 * i + 1 + first) * (2 * i + 2 + first));
-    }
-    for (int i = 11; i >= 0; i--) s += terms[i];
-    return s;
-}
-constexpr double cos_turn(int k, int n);
-constexpr double sin_turn(int k, int n) {
-    k = ((k % n) + n) % n;
-    if (2 * k > n) return -sin_turn(n - k, n);
-    if (4 * k > n) return (4 * k == 2 * n) ? 0.0 : (n % 2 ? taylor(kPi * (n - 2 * k) / n, 1) : sin_turn(n / 2 - k, n));
-    if (8 * k > n) return taylor(kPi * (n - 4 * k) / (2.0 * n), 0);
-    return taylor(2.0 * kPi * k / n, 1);
-}
-constexpr double cos_turn(int k, int n) {
-    k = ((k % n) + n) % n;
-    if (2 * k > n) k = n - k;
-    if (4 * k > n) return -(n % 2 ? taylor(kPi * (n - 2 * k) / n, 0) : cos_turn(n / 2 - k, n));
-    if (8 * k > n) return taylor(kPi * (n - 4 * k) / (2.0 * n), 1);
-    return taylor(2.0 * kPi * k / n, 0);
-}
-static_assert(cos_turn(1, 8) - 0.70710678118654752440 < 2e-16 && cos_turn(1, 8) - 0.70710678118654752440 > -2e-16, "");
-static_assert(sin_turn(2, 5) - 0.58778525229247312917 < 2e-16 && sin_turn(2, 5) - 0.58778525229247312917 > -2e-16, "");
-static_assert(cos_turn(4, 9) + 0.93969262078590838405 < 2e-16 && cos_turn(4, 9) + 0.93969262078590838405 > -2e-16, "");
 
 // e^{s 2 pi i k / N} v for compile-time k
 template <int K, int N, typename V>

@@ -1,0 +1,45 @@
+"""GPU test of the angular kernels at the edges of their tiles: numbers of points just below,
+at and above a workgroup's, for every order, against the oracle.
+
+Tolerances: the projections are sums over the no orientations, exact to about sqrt(no) eps
+of their 2-norm (the FP32 kernel rounds its terms first): 4 sqrt(no) eps.  Energies and
+gradients: the engine's parity bars, 1e-10 in FP64 and 1e-5 in FP32."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+# 1, 15, 16, 18, 30, 32, 36, 64, 75, 125, 128, 135, 256, 270 points
+GRIDS = ((1, 1, 1), (5, 3, 1), (4, 2, 2), (3, 3, 2), (5, 2, 3), (4, 8, 1), (3, 3, 4), (4, 4, 4), (5, 5, 3), (5, 5, 5),
+         (16, 4, 2), (5, 9, 3), (16, 16, 1), (9, 5, 6))
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("mmax", range(6))
+def test_tiles_of_points(precision, mmax):
+    from mdft import ck
+    from mdft.gpu import Engine
+    from oracle import oracle as O
+    eps = np.finfo(np.float64 if precision == "fp64" else np.float32).eps
+    bar = 1e-10 if precision == "fp64" else 1e-5
+    table = ck.synthetic_ck(mmax, 512, 0.05, seed=11, n0=0.0333)
+    for n in GRIDS:
+        length = [0.5 * v for v in n]
+        print(f"[angular] {precision} mmax={mmax} {n}", flush=True)
+        eng = Engine(n, length, mmax, 2, 2.4777, 0.0333, precision)
+        ora = O.Oracle(n, length, mmax, 2, 2.4777, 0.0333)
+        for e in (eng, ora):
+            e.set_ck(table)
+        rng = np.random.default_rng(sum(n))
+        xi = 1.0 + 0.3 * rng.uniform(-1, 1, eng.N * eng.no)
+        vext = rng.uniform(-2.0, 5.0, eng.N * eng.no)
+        eng.set_vext(vext)
+        ref = ora.excess_stage(xi, 1).reshape(eng.N, -1)
+        got = eng.excess_stage(xi, 1)
+        assert np.linalg.norm(got - ref) <= 4.0 * np.sqrt(eng.no) * eps * np.linalg.norm(ref), n
+        parts, df = eng.energy_and_gradient(xi)
+        pref, dref = ora.energy_and_gradient(xi, vext)
+        # (F_id and F_ext are sums of terms of both signs: relative to the largest part)
+        assert np.abs(parts - pref).max() <= bar * np.abs(pref).max(), (n, parts, pref)
+        assert np.abs(df - dref).max() <= bar * np.abs(dref).max(), n
+        eng.close()

@@ -475,6 +475,52 @@ template <int L, typename T> __device__ __forceinline__ void row_to_coefficients
     }
 }
 
+// The phi synthesis of one (row, mu2), in place over its coefficients: mu2 = 0 (real values,
+// coefficients doubled for mup > 0): h(phi_j) at row[j]; mu2 > 0: h(phi_j) = sum_mup conj(f) e^{i mup
+// phi_j} at the item of mup = j - L.
+template <int L, typename T> __device__ __forceinline__ void phi_synthesis0(T *row) {
+    using R = Rows<L>;
+    constexpr int N = R::NPHI;
+    constexpr Turns<T, N> tw;
+    T x[L + 1], y[L + 1], h0 = row[0];
+    const T f0 = h0;
+#pragma unroll
+    for (int k = 1; k <= L; k++) {
+        x[k] = row[2 * k];
+        y[k] = row[2 * k + 1];
+        h0 += x[k];
+    }
+    row[0] = h0;
+#pragma unroll
+    for (int j = 1; j <= L; j++) {
+        T a = f0, b = 0;
+#pragma unroll
+        for (int k = 1; k <= L; k++) {
+            a = fma(x[k], tw.c[(j * k) % N], a);
+            b = fma(y[k], tw.s[(j * k) % N], b);
+        }
+        row[j] = a + b;
+        row[N - j] = a - b;
+    }
+}
+template <int L, typename T> __device__ __forceinline__ void phi_synthesis(T *f) {
+    constexpr int N = 2 * L + 1;
+    T x[N], y[N], ox[N], oy[N];
+#pragma unroll
+    for (int k = -L; k <= L; k++) {
+        const int at = k < 0 ? N + k : k;
+        x[at] = f[2 * (L + k)];
+        y[at] = -f[2 * (L + k) + 1];
+    }
+    dft_odd<N, T>(x, y, ox, oy);
+#pragma unroll
+    for (int j = 0; j < N; j++) {
+        const int at = j <= L ? L + j : j - L - 1;
+        f[2 * j] = ox[at];
+        f[2 * j + 1] = oy[at];
+    }
+}
+
 // One projection of the theta contraction: out = (sum_it ax[it] F_it.x, sum_it ay[it] F_it.y) with
 // F_it the coefficient at `item` of the rows of a point.  The signs of mup < 0 at mu2 = 0 (the
 // conjugate of mup > 0 times (-1)^mup) and all norms are in the weights.
@@ -578,79 +624,96 @@ __global__ __launch_bounds__(TH) void angl2proj_t(const double *__restrict__ xi,
     }
 }
 
+// Points per tile of final_t and its least waves per SIMD: elements for whole rounds of 256 threads
+// (330 x 6 = 7.7 rounds at mmax 5), as many as registers hold without spilling.  Measured, final
+// pass at 128^3, mmax 5: fast variant 4, 5, 6, 7, 8 points 3.58, 3.42, 3.38, 3.55, 4.52 ms; FP32
+// 4.54, 4.55, 3.85, 4.09, 3.97; FP64 5, 6, 7, 8 points 5.75, 5.59, 5.53, 5.81 ms (8 points at 3
+// waves); 100^3, mmax 4, FP64: 8 points at 4 waves 1.76, 9 at 3 waves 1.69 ms.
+template <int L, typename T> struct FinalShape {
+    static constexpr int PT32 = L == 5 ? 6 : L == 4 ? 9 : L == 3 ? 24 : L == 2 ? 32 : L == 1 ? 128 : 256;
+    static constexpr int PT64 = L == 5 ? 7 : L == 4 ? 9 : L == 3 ? 18 : L == 2 ? 32 : L == 1 ? 128 : 256;
+    static constexpr int PT = sizeof(T) == 4 ? PT32 : PT64;
+    static constexpr int WAVES = sizeof(T) == 8 && L == 4 ? 3 : 4;
+};
+
+// The fast variant is bound by HBM (15.3 GB at 128^3, mmax 5, in 3.38 ms: 4.5 TB/s; a plain copy
+// reaches 4.8).  FP64 (19.6 GB in 5.5 ms) is not: its logarithms and synthesis are 2.4 ms of vector
+// issue that 3 to 4 waves per SIMD do not hide wholly behind the loads.  The phi synthesis takes one
+// thread per (row, mu2), in place; with one thread per (row, phi, mu2), each reading 11 coefficients
+// and 11 twiddles from LDS for one output, the pass took 3.70 (fast) and 6.79 ms (FP64).
+//
 // Persistent: each workgroup stages the tables once and then takes tiles blockIdx.x,
 // blockIdx.x + gridDim.x, ...  A tile needs no barrier beyond its three: every LDS array a
 // tile writes was last read before a barrier that all threads have passed by then.  The
 // free-energy sums and gradient products accumulate over a workgroup's tiles and are
 // written once, one partial per workgroup.
 // DOT32: mode 0 with an FP32 iterate, forming the gradient products over FP32 vectors (the
-// evaluations of the fast minimiser), on full tiles only (N a multiple of PT).  Every load
-// of the tile is then issued on every path (the last partial round of a thread's elements
-// with its index clamped into the tile), and dF is stored on every path: the wait before
-// each use counts exactly the memory operations issued after it, so the product operands
-// loaded ahead stay in flight.
-template <int L, int PT, typename T, bool DOT32 = false>
-// DOT32: at least 5 waves per SIMD (at most 96 registers): the tile's iterate, vext and product
-// operands, loaded before the synthesis phases, stay in registers through them (measured faster
-// than 6 or 7 waves with fewer of them in flight); the general variant, with every mode's
-// branches, may take more registers rather than spill
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(DOT32 ? 5 : 4, 7))) void final_t(const typename C2<T>::t *__restrict__ proj, const double *__restrict__ xi,
-                                                   const double *__restrict__ vext, double *__restrict__ df,
-                                                   double *__restrict__ partials, size_t N, AngTables t,
-                                                   FinalConsts k, int mode, float *__restrict__ df32,
-                                                   const double *__restrict__ vsinv, DotArgs da,
-                                                   double *__restrict__ dpart, const float *__restrict__ xi32,
-                                                   const float *__restrict__ vext32) {
-    using D = Dims<L>;
+// evaluations of the fast minimiser), on at least PT points.  Every load of the tile is then
+// issued on every path (the last partial round of a thread's elements with its index clamped
+// into the tile), and dF is stored on every path: the wait before each use counts exactly the
+// memory operations issued after it, so the product operands loaded ahead stay in flight.  The
+// last tile of a grid that is not a whole number of tiles starts early, over points of the one
+// before it (whose dF is written twice, with the same values); those add nothing to the sums.
+template <int L, typename T, bool DOT32 = false>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FinalShape<L, T>::WAVES, 8))) void final_t(
+    const typename C2<T>::t *__restrict__ proj, const double *__restrict__ xi, const double *__restrict__ vext,
+    double *__restrict__ df, double *__restrict__ partials, size_t N, AngTables t, FinalConsts k, int mode,
+    float *__restrict__ df32, const double *__restrict__ vsinv, DotArgs da, double *__restrict__ dpart,
+    const float *__restrict__ xi32, const float *__restrict__ vext32) {
+    using R = Rows<L>;
     using V = typename C2<T>::t;
-    constexpr int NO = D::NO, NP = D::NP, NTH = D::NTH, NPHI = D::NPHI, NPSI = D::NPSI, H1 = D::H1, W = D::W;
+    constexpr int PT = FinalShape<L, T>::PT;
+    constexpr int NO = R::NO, NP = R::NP, NTH = R::NTH, NPSI = R::NPSI, H = R::H, W = R::W;
+    constexpr int ROW = R::ROW, RS = R::RS, NF = R::NF;
+    constexpr int NPS = NP | 1;  // odd: the records of consecutive points in different banks
     if constexpr (DOT32) mode = 0;
-    __shared__ __align__(16) V Gm[PT * NP];
-    __shared__ V f[PT * NTH * W * H1];
-    __shared__ V h[PT * NTH * NPHI * H1];
-    __shared__ V twphi[NPHI * W];   // (cos, sin)(2 pi mup iphi / nphi) at [iphi][mup + L]
-    __shared__ V twpsi[NPSI * H1];  // 2 (cos, sin)(2 pi mu2 ipsi / npsi) at [ipsi][mu2]
-    __shared__ T p2a[NP * NTH];
-    __shared__ double wq[NO];
-    __shared__ double sth[NTH];  // 1 / s of each theta (the weights, hence s, depend on theta only)
-    // projection index of (m, mup, mu2), as bytes: the loaded index is then known to be small and
-    // its products stay 24-bit multiplies (entries with m below the item's lowest m are never read)
+    __shared__ __align__(16) V Gm[PT * NPS];
+    __shared__ T rows[NTH * PT * RS];  // row of (point, theta) at theta PT + point
+    __shared__ V twpsi[NPSI * (H + 1)];  // (cos, sin)(2 pi mu2 ipsi / npsi) at [ipsi][mu2]
+    __shared__ T p2a[NP * NTH];          // twice the table's for mu2 > 0 (the weight of +-mu2 in the c2r)
+    __shared__ double wth[NTH];          // the weights depend on theta only
+    __shared__ double sth[NTH];          // 1 / s of each theta
+    // projection index of (m, mup, mu2) and (m, -mup, 0), as bytes: the loaded index is then known to be small
+    // and its products stay 24-bit multiplies (entries with m below the item's lowest m are never read)
     static_assert(NP <= 255, "projection indices are stored as bytes");
-    __shared__ unsigned char pidx[(L + 1) * W * H1];
-    __shared__ unsigned char ford[W * H1];  // the theta synthesis' (mup, mu2) items, longest m loop first
+    __shared__ unsigned char pidx[(L + 1) * NF], pneg[(L + 1) * (L + 1)];
+    __shared__ unsigned char ford[NF];  // the theta synthesis' (mup, mu2) items, longest m loop first
     const int tid = threadIdx.x;
-    for (int i = tid; i < (L + 1) * W * H1; i += kThreads) pidx[i] = (unsigned char)t.pidx[i];
+    auto mup_of = [](int it) { return it <= L ? it : (it - L - 1) % W - L; };
+    auto mu_of = [](int it) { return it <= L ? 0 : (it - L - 1) / W + 1; };
+    for (int i = tid; i < (L + 1) * NF; i += kThreads) {
+        const int m = i / NF, it = i % NF;
+        pidx[i] = (unsigned char)t.pidx[(m * W + mup_of(it) + L) * (H + 1) + mu_of(it)];
+    }
+    for (int i = tid; i < (L + 1) * (L + 1); i += kThreads)
+        pneg[i] = (unsigned char)t.pidx[((i / (L + 1)) * W - i % (L + 1) + L) * (H + 1)];
     {
-        // the item (mup + L) * H1 + mu2 sums over m = max(|mup|, 2 mu2) .. L; ranked by that
-        // length (ties by index), the lanes of a wave take loops of nearly one length
-        auto len = [](int it) {
-            const int a = it / H1 - L, b = 2 * (it % H1);
+        // an item sums over m = max(|mup|, 2 mu2) .. L; ranked by that length (ties by index),
+        // the lanes of a wave take loops of nearly one length
+        auto len = [&](int it) {
+            const int a = mup_of(it), b = 2 * mu_of(it);
             const int aa = a < 0 ? -a : a;
             return L + 1 - (aa > b ? aa : b);
         };
-        for (int i = tid; i < W * H1; i += kThreads) {
+        for (int i = tid; i < NF; i += kThreads) {
             const int li = len(i);
             int r = 0;
-            for (int j = 0; j < W * H1; j++) {
+            for (int j = 0; j < NF; j++) {
                 const int lj = len(j);
                 r += (lj > li || (lj == li && j < i)) ? 1 : 0;
             }
             ford[r] = (unsigned char)i;
         }
     }
-    for (int i = tid; i < NPHI * W; i += kThreads) {
-        const int iphi = i / W, mup = i % W - L;
-        int kk = (mup * iphi) % NPHI;
-        kk += (kk < 0) ? NPHI : 0;
-        twphi[i] = mk<V>((T)t.cph[kk], (T)t.sph[kk]);
+    for (int i = tid; i < NPSI * (H + 1); i += kThreads) {
+        const int kk = ((i % (H + 1)) * (i / (H + 1))) % NPSI;
+        twpsi[i] = mk<V>((T)t.cps[kk], (T)t.sps[kk]);
     }
-    for (int i = tid; i < NPSI * H1; i += kThreads) {
-        const int kk = ((i % H1) * (i / H1)) % NPSI;
-        twpsi[i] = mk<V>((T)(2.0 * t.cps[kk]), (T)(2.0 * t.sps[kk]));
+    for (int i = tid; i < NP * NTH; i += kThreads) p2a[i] = (T)(t.pmu[i / NTH] > 0 ? 2.0 * t.p2a[i] : t.p2a[i]);
+    for (int i = tid; i < NTH; i += kThreads) {
+        wth[i] = t.w[i * ROW];
+        sth[i] = vsinv ? vsinv[i * ROW] : 1.0;
     }
-    for (int i = tid; i < NP * NTH; i += kThreads) p2a[i] = (T)t.p2a[i];
-    for (int i = tid; i < NO; i += kThreads) wq[i] = t.w[i];
-    for (int i = tid; i < NTH; i += kThreads) sth[i] = vsinv ? vsinv[i * NPHI * NPSI] : 1.0;
     double fid = 0.0, fext = 0.0, fexc = 0.0;
     double d0 = 0.0, d1 = 0.0, d2 = 0.0;  // products of dF with the DotArgs vectors
     double dss = 0.0;                     // DOT32: the product of dF with itself
@@ -662,17 +725,26 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(DOT32 
         // all stay in registers (and spill)
         int tl = tid;
         asm volatile("" : "+v"(tl));
-        const size_t r0 = tile * PT;
+        const int skip = (DOT32 && (tile + 1) * PT > N) ? (int)((tile + 1) * PT - N) : 0;
+        const size_t r0 = tile * PT - skip;
         const int npts = DOT32 ? PT : (int)((N - r0) < (size_t)PT ? (N - r0) : (size_t)PT);
         // DOT32: the tile's base pointers (uniform), indexed by 32-bit element offsets
         const float *xi32t = DOT32 ? xi32 + r0 * NO : nullptr, *vx32t = DOT32 ? vext32 + r0 * NO : nullptr;
         float *df32t = DOT32 ? df32 + r0 * NO : nullptr;
         const V *src = proj + r0 * NP;
         if constexpr (sizeof(T) == 4 && NP % 2 == 0) {  // FP32: 16-byte loads, two projections each
-            for (int i = tl; i < npts * (NP / 2); i += kThreads)
-                reinterpret_cast<float4 *>(Gm)[i] = reinterpret_cast<const float4 *>(src)[i];
+            for (int i = tl; i < npts * (NP / 2); i += kThreads) {
+                const float4 v = reinterpret_cast<const float4 *>(src)[i];
+                const unsigned pt = DivC<NP / 2, PT * (NP / 2)>::q(i);
+                V *g = Gm + mul24(pt, NPS) + 2 * (i - mul24(pt, NP / 2));
+                g[0] = mk<V>(v.x, v.y);
+                g[1] = mk<V>(v.z, v.w);
+            }
         } else {
-            for (int i = tl; i < npts * NP; i += kThreads) Gm[i] = src[i];
+            for (int i = tl; i < npts * NP; i += kThreads) {
+                const unsigned pt = DivC<NP, PT * NP>::q(i);
+                Gm[mul24(pt, NPS) + (i - mul24(pt, NP))] = src[i];
+            }
         }
         // DOT32: the tile's FP32 iterate, FP32 vext and the FP32 operands of the first two
         // gradient products, loaded here so that their latency passes during the synthesis
@@ -695,26 +767,56 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(DOT32 
                 dq[1][q] = dp1t[ii];
             }
         }
+        // the general variant: the tile's xi and vext, all of a thread's loads issued together:
+        // before the synthesis phases where the registers allow it (FP32, and FP64 for mmax <= 3: 96^3,
+        // mmax 3: 0.577 -> 0.556 ms; FP64 at mmax 5 would spill), else before the loop that uses them
+        constexpr bool kEarly = sizeof(T) == 4 || L <= 3;
+        double xr[NIT], vr[NIT];
+        auto load_general = [&]() {
+    #pragma unroll
+            for (int q = 0; q < NIT; q++) {
+                const int i = tl + q * kThreads;
+                xr[q] = 0.0;
+                vr[q] = 0.0;
+                if (i < npts * NO) {
+                    const size_t g = r0 * NO + i;
+                    if (mode < 3) xr[q] = xi32 ? hold_f32(xi32[g]) : xi[g];  // FP32 iterate: xi32
+                    if (mode == 0 || mode == 3 || mode == 4) vr[q] = vext[g];
+                }
+            }
+        };
+        if constexpr (!DOT32 && kEarly) load_general();
         __syncthreads();
-        // f(theta, mu2, mup) = sum_m p(m, mup, mu2) d(theta) fm(m): one thread per
-        // (point, mup, mu2), all theta at once (each projection read once); items by rank of
-        // their loop length, the tile's points innermost
-        for (int i = tl; i < PT * W * H1; i += kThreads) {
+        // f(theta, mup, mu2) = sum_m p(m, mup, mu2) d(theta) fm(m): one thread per (point, mup, mu2),
+        // all theta at once (each projection read once); items by rank of their loop length, the
+        // tile's points innermost.  mu2 = 0: the psi step takes the real part of the sum over mup, so
+        // the items mup > 0 hold p(m, mup, 0) + (-1)^mup conj(p(m, -mup, 0)) and mup = 0 the real part
+        for (int i = tl; i < PT * NF; i += kThreads) {
             const int rk = i / PT, pt = i - rk * PT;
             if (pt >= npts) continue;
             const int item = ford[rk];
-            const int jm = (int)DivC<H1, W * H1>::q(item);
-            const int mu2 = item - jm * H1, mup = jm - L;
-            const int a = mup < 0 ? -mup : mup, b = 2 * mu2;
-            const int mlo = a > b ? a : b;
+            int mlo, neg = 0;  // lowest m; 1, 2: mu2 = 0 with mup > 0, = 0
+            if (item <= L) {
+                mlo = item;
+                neg = item > 0 ? 1 : 2;
+            } else {
+                const int rest = item - (L + 1), mu1 = (int)DivC<W, (H > 0 ? H : 1) * W>::q(rest);
+                const int mup = rest - mu1 * W - L, a = mup < 0 ? -mup : mup, b = 2 * mu1 + 2;
+                mlo = a > b ? a : b;
+            }
+            const T sg = (item & 1) ? (T)-1 : (T)1;
             T re[NTH], im[NTH];
     #pragma unroll
             for (int it = 0; it < NTH; it++) re[it] = im[it] = (T)0;
-            const unsigned char *pp = pidx + (mul24(jm, H1) + mu2);  // the item's entry of each m row
-            const V *gp = Gm + mul24(pt, NP);
+            const V *gp = Gm + mul24(pt, NPS);
             for (int m = mlo; m <= L; m++) {
-                const unsigned p = pp[m * (W * H1)];
-                const V v = gp[p];
+                const unsigned p = pidx[m * NF + item];
+                V v = gp[p];
+                if (neg == 1) {
+                    const V u = gp[pneg[m * (L + 1) + item]];
+                    v.x = fma(sg, u.x, v.x);
+                    v.y = fma(-sg, u.y, v.y);
+                }
                 const T *c = p2a + p * NTH;
     #pragma unroll
                 for (int it = 0; it < NTH; it++) {
@@ -722,67 +824,24 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(DOT32 
                     im[it] += v.y * c[it];
                 }
             }
-            V *fo = f + (mul24(mul24(pt, NTH * W) + jm, H1) + mu2);
+            T *fo = rows + (mul24(pt, RS) + 2 * item);
     #pragma unroll
-            for (int it = 0; it < NTH; it++) fo[it * (W * H1)] = mk<V>(re[it], im[it]);
-        }
-        __syncthreads();
-        // h(theta, phi, mu2): the sum over mup of f(theta, mu2, mup) with the phi twiddles; items
-        // mu2-major, so that whole waves take mu2 = 0, whose imaginary part the psi synthesis
-        // below never reads
-        constexpr int NL = PT * NTH * NPHI;  // (point, theta, phi) lines of a full tile
-        for (int i = tl; i < NL * H1; i += kThreads) {
-            const int mu2 = (int)DivC<NL, NL * H1>::q(i), line = i - mu2 * NL;
-            if (line >= npts * NTH * NPHI) continue;
-            const int rest = (int)DivC<NPHI, NL>::q(line), iphi = line - rest * NPHI;
-            const V *fr = f + (mul24(rest, W * H1) + mu2);
-            const V *tw = twphi + mul24(iphi, W);
-            T re = 0, im = 0;
-            if (mu2 == 0) {
-    #pragma unroll
-                for (int j = 0; j < W; j++) {
-                    const V v = fr[j * H1], e = tw[j];
-                    if constexpr (sizeof(T) == 4) {
-                        re = fma(v.x, e.x, re);
-                        re = fma(v.y, e.y, re);
-                    } else {
-                        re += v.x * e.x + v.y * e.y;
-                    }
-                }
-            } else {
-    #pragma unroll
-                for (int j = 0; j < W; j++) {
-                    const V v = fr[j * H1], e = tw[j];
-                    if constexpr (sizeof(T) == 4) {  // four multiply-adds (FP32 only, as in angl2proj_t)
-                        re = fma(v.x, e.x, re);
-                        re = fma(v.y, e.y, re);
-                        im = fma(v.x, e.y, im);
-                        im = fma(-v.y, e.x, im);
-                    } else {
-                        re += v.x * e.x + v.y * e.y;
-                        im += v.x * e.y - v.y * e.x;
-                    }
-                }
-            }
-            h[mul24(line, H1) + mu2] = mk<V>(re, im);
-        }
-        __syncthreads();
-        // the general variant: the tile's xi and vext, all of a thread's loads issued together
-        // for the loop below; the other workgroups on the compute unit cover their latency
-        // (loaded before the synthesis phases, these FP64 values would hold twice the registers)
-        double xr[NIT], vr[NIT];
-    #pragma unroll
-        for (int q = 0; q < NIT; q++) {
-            if constexpr (DOT32) continue;
-            const int i = tl + q * kThreads;
-            xr[q] = 0.0;
-            vr[q] = 0.0;
-            if (i < npts * NO) {
-                const size_t g = r0 * NO + i;
-                if (mode < 3) xr[q] = xi32 ? hold_f32(xi32[g]) : xi[g];  // FP32 iterate: xi32
-                if (mode == 0 || mode == 3 || mode == 4) vr[q] = vext[g];
+            for (int it = 0; it < NTH; it++) {
+                fo[it * (PT * RS)] = re[it];
+                fo[it * (PT * RS) + 1] = neg == 2 ? (T)0 : im[it];
             }
         }
+        __syncthreads();
+        // h(theta, phi, mu2), one thread per (row, mu2), in place; mu2-major, so that whole waves
+        // take mu2 = 0 (points past the end: their rows are never read)
+        for (int i = tl; i < NTH * PT * (H + 1); i += kThreads) {
+            const int mu2 = (int)DivC<NTH * PT, NTH * PT * (H + 1)>::q(i), row = i - mu2 * (NTH * PT);
+            T *f = rows + mul24(row, RS);
+            if (mu2 == 0) phi_synthesis0<L, T>(f);
+            else phi_synthesis<L, T>(f + 2 * (L + 1) + mul24(mu2 - 1, 2 * W));
+        }
+        __syncthreads();
+        if constexpr (!DOT32 && !kEarly) load_general();
         // FP32 path: the free-energy terms of a thread's elements in this tile, summed in FP32
         // and added to the FP64 sums once per tile
         float fexc_t = 0.0f, fid_t = 0.0f, fext_t = 0.0f;
@@ -802,15 +861,16 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(DOT32 
             }
             // LDS offsets by 24-bit products: every operand here is small and non-negative
             const unsigned pt = DivC<NO, PT * NO>::q(i);
-            const int io = i - (int)mul24(pt, NO);
-            const unsigned line = DivC<NPSI, NO>::q(io), ipsi = io - mul24(line, NPSI);  // line = it*NPHI + iphi
-            const V *hr = h + mul24(mul24(pt, NTH * NPHI) + line, H1);
-            const V *tp = twpsi + mul24(ipsi, H1);
-            T vt = hr[0].x;
+            const unsigned io = i - mul24(pt, NO), it = DivC<ROW, NO>::q(io);
+            const unsigned col = io - mul24(it, ROW), iphi = DivC<NPSI, ROW>::q(col), ipsi = col - mul24(iphi, NPSI);
+            const T *hr = rows + mul24(mul24(it, PT) + pt, RS);
+            const V *tp = twpsi + mul24(ipsi, H + 1);
+            T vt = hr[iphi];
+            hr += 2 * (L + 1) + 2 * iphi;
     #pragma unroll
-            for (int mu2 = 1; mu2 < H1; mu2++) {
-                if constexpr (sizeof(T) == 4) vt = fma(-hr[mu2].y, tp[mu2].y, fma(hr[mu2].x, tp[mu2].x, vt));
-                else vt += hr[mu2].x * tp[mu2].x - hr[mu2].y * tp[mu2].y;
+            for (int mu2 = 1; mu2 <= H; mu2++) {
+                const T hx = hr[(mu2 - 1) * 2 * W], hy = hr[(mu2 - 1) * 2 * W + 1];
+                vt = fma(-hy, tp[mu2].y, fma(hx, tp[mu2].x, vt));
             }
             const size_t g = r0 * NO + i;
             if constexpr (sizeof(T) == 4) {
@@ -819,14 +879,15 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(DOT32 
                     // are FP32 already), summed in FP32 over the thread's elements of the tile
                     // and in FP64 over the tiles; rho/rho0 - 1 is formed in FP64 first so that
                     // the excess term keeps its small deviations from the bulk
-                    const double si = vsinv ? sth[DivC<NPHI * NPSI, NO>::q(io)] : 1.0;  // scaled variables: xi = u / s, dF/du = dF/dxi / s
+                    const double si = vsinv ? sth[it] : 1.0;  // scaled variables: xi = u / s, dF/du = dF/dxi / s
                     const double x = xq * si;
                     const double xx = x * x;
-                    const float wf = (float)wq[io];
+                    const float wf = (float)wth[it];
+                    const float ws = DOT32 && (int)pt < skip ? 0.0f : wf;  // weight in the sums
                     const float vexcf = (float)k.prefactor * wf * vt;
                     const float drf = (float)(xx - 1.0);
                     const float rho0f = (float)rho0, x2 = (float)xx, xf = (float)x;
-                    fexc_t += rho0f * drf * vexcf;
+                    fexc_t += rho0f * drf * ((float)k.prefactor * ws * vt);
                     float gid = 0.0f;
                     if (xx * rho0 > DBL_EPSILON) {
                         // ln(rho / rho0) from the hardware base-2 logarithm: x2 > 6e-15 here (rho > DBL_EPSILON),
@@ -835,16 +896,16 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(DOT32 
                         const float lg = __builtin_amdgcn_logf(x2) * 0.693147181f;
                         const float ve = DOT32 ? ve32 : (float)vr[q];
                         const float kTf = (float)kT, dvf = (float)dv;
-                        fid_t += kTf * dvf * wf * rho0f * (x2 * lg - drf);
-                        fext_t += dvf * wf * rho0f * x2 * ve;
+                        fid_t += kTf * dvf * ws * rho0f * (x2 * lg - drf);
+                        fext_t += dvf * ws * rho0f * x2 * ve;
                         gid = wf * 2.0f * rho0f * xf * (kTf * lg + ve);
                     } else {
-                        fid_t += (float)(kT * dv * rho0) * wf;
+                        fid_t += (float)(kT * dv * rho0) * ws;
                     }
                     const float gv = (gid + 2.0f * rho0f * xf * vexcf) * (float)si;
                     if constexpr (DOT32) {
                         df32t[i] = gv;
-                        const double gd = (double)gv;
+                        const double gd = (int)pt < skip ? 0.0 : (double)gv;
                         // the empty asm keeps the conversions here: hoisted next to the loads above,
                         // they would make each load wait
                         float o0 = dq[0][q], o1 = dq[1][q];
@@ -869,9 +930,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(DOT32 
             }
             // from here on FP64: free-energy reductions, rho ln rho and the gradient
             const double v = (double)vt;
-            const double wio = wq[io];
+            const double wio = wth[it];
             const double vexc = k.prefactor * wio * v;
-            const double si = (mode == 0 && vsinv) ? sth[DivC<NPHI * NPSI, NO>::q(io)] : 1.0;  // scaled variables (mode 0)
+            const double si = (mode == 0 && vsinv) ? sth[it] : 1.0;  // scaled variables (mode 0)
             const double x = xq * si;
             const double rho = x * x * rho0;
             fexc += (x * x * rho0 - rho0) * vexc;
@@ -922,14 +983,14 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(DOT32 
     }
 }
 
+constexpr size_t kMinTile = 4;  // the specialised kernels take at least as many points per workgroup
 constexpr int kPT = 4;  // points per workgroup tile (keeps the LDS tile under 64 KB at mmax = 5)
 
 // Workgroups of a persistent kernel, never more than the tiles.  resident_grid: as many as
 // the compute units hold at once (registers and LDS of that kernel); a larger grid leaves
 // workgroups waiting for a slot until others have finished all their tiles.  The fast final
-// pass runs faster so (3.85 -> 3.77 ms at 128^3, mmax 5); the general final pass, at 3 (FP64,
-// the LDS limit) or 4 (FP32) resident workgroups per compute unit, runs faster with 8 per
-// compute unit (FP64 6.4 against 6.9 ms), the later ones taking the slots of the first to finish.
+// pass runs faster so; the general final pass runs faster with 8 per compute unit (about twice the
+// resident number), the later ones taking the slots of the first to finish.
 template <typename K>
 size_t resident_grid(const mdft_ctx *c, K kernel, size_t ntiles) {
     int per_cu = 0;
@@ -995,11 +1056,10 @@ bool launch_a2p_t(mdft_ctx *c, const double *xi, typename C2<T>::t *proj, int fe
     }
 }
 
-template <int PT, typename T>
+template <typename T>
 bool launch_final_t(mdft_ctx *c, const typename C2<T>::t *proj, const double *xi, double *df, int mode, FinalConsts k,
                     size_t npts = 0, size_t *grid_out = nullptr) {
     if (!npts) npts = c->N;
-    const size_t ntiles = (npts + PT - 1) / PT;
     DotArgs da{};
     if (mode == 0 && c->dot_k > 0) {
         da.k = c->dot_k;
@@ -1008,28 +1068,29 @@ bool launch_final_t(mdft_ctx *c, const typename C2<T>::t *proj, const double *xi
         for (int j = 0; j < 3; j++) da.p[j] = c->dot_vec[j];
     }
     // the FP32 kernel forming products over FP32 vectors (dF then FP32 too) has its own variant
-    const bool dot32 = sizeof(T) == 4 && mode == 0 && da.k > 0 && da.f32 && c->xi32 && c->vext32_ok && npts % PT == 0;
+    const bool dot32 = sizeof(T) == 4 && mode == 0 && da.k > 0 && da.f32 && c->xi32 && c->vext32_ok;
     switch (c->L) {
 #define FIN_CASE(LL) \
-    case LL: \
-        if (dot32) { \
-            const size_t nb = resident_grid(c, final_t<LL, PT, T, sizeof(T) == 4>, ntiles); \
+    case LL: { \
+        constexpr int PT = FinalShape<LL, T>::PT; \
+        const size_t ntiles = (npts + PT - 1) / PT; \
+        if (dot32 && npts >= PT) { \
+            const size_t nb = resident_grid(c, final_t<LL, T, sizeof(T) == 4>, ntiles); \
             if (grid_out) *grid_out = nb; \
-            hipLaunchKernelGGL((final_t<LL, PT, T, sizeof(T) == 4>), dim3((unsigned)nb), dim3(kThreads), 0, c->stream, proj, xi, c->d_vext, df, c->d_partials, npts, c->ang, k, mode, c->df32, c->vsinv, da, c->d_dpart, c->xi32, c->d_vext32); \
+            hipLaunchKernelGGL((final_t<LL, T, sizeof(T) == 4>), dim3((unsigned)nb), dim3(kThreads), 0, c->stream, proj, xi, c->d_vext, df, c->d_partials, npts, c->ang, k, mode, c->df32, c->vsinv, da, c->d_dpart, c->xi32, c->d_vext32); \
         } else { \
             const size_t nb = oversubscribed_grid(c, ntiles); \
             if (grid_out) *grid_out = nb; \
-            hipLaunchKernelGGL((final_t<LL, PT, T>), dim3((unsigned)nb), dim3(kThreads), 0, c->stream, proj, xi, c->d_vext, df, c->d_partials, npts, c->ang, k, mode, mode == 0 ? c->df32 : nullptr, mode == 0 ? c->vsinv : nullptr, da, c->d_dpart, mode == 0 ? c->xi32 : nullptr, nullptr); \
+            hipLaunchKernelGGL((final_t<LL, T>), dim3((unsigned)nb), dim3(kThreads), 0, c->stream, proj, xi, c->d_vext, df, c->d_partials, npts, c->ang, k, mode, mode == 0 ? c->df32 : nullptr, mode == 0 ? c->vsinv : nullptr, da, c->d_dpart, mode == 0 ? c->xi32 : nullptr, nullptr); \
         } \
-        return true;
+        return true; \
+    }
         FIN_CASE(0) FIN_CASE(1) FIN_CASE(2) FIN_CASE(3) FIN_CASE(4) FIN_CASE(5)
 #undef FIN_CASE
         default: return false;
     }
 }
 
-constexpr int kPTt = 4;   // points per workgroup of the specialised kernels, FP64
-constexpr int kPT32 = 4;  // the same for FP32 (8 measured slower at 128^3, mmax = 5)
 
 hipError_t launch_angl2proj_f64(mdft_ctx *c, const double *xi, double2 *proj) {
     if (c->d.mrso == 2 && launch_a2p_t<double>(c, xi, proj)) return hipGetLastError();
@@ -1054,10 +1115,10 @@ hipError_t launch_final_f64(mdft_ctx *c, const double2 *proj, const double *xi, 
     const double fourpisq = 4.0 * pi * pi;
     k.prefactor = -c->d.kT * 2.0 * fourpisq / c->d.mrso / c->d.n0;  // cproj_mrso.f90:728
     if (c->d.mrso == 2) {
-        const size_t nbt = (c->N + kPTt - 1) / kPTt;
+        const size_t nbt = (c->N + kMinTile - 1) / kMinTile;
         if ((e = ensure_partials(c, nbt)) != hipSuccess) return e;
         size_t grid = 0;
-        if (launch_final_t<kPTt, double>(c, proj, xi, df, mode, k, 0, &grid)) {
+        if (launch_final_t<double>(c, proj, xi, df, mode, k, 0, &grid)) {
             *nblocks_out = (int)grid;
             return hipGetLastError();
         }
@@ -1118,11 +1179,11 @@ hipError_t launch_angl2proj_f32(mdft_ctx *c, const double *xi, float2 *proj) {
 }
 
 hipError_t launch_final_f32(mdft_ctx *c, const float2 *proj, const double *xi, double *df, int mode, int *nblocks_out) {
-    const size_t nbt = (c->N + kPT32 - 1) / kPT32;
+    const size_t nbt = (c->N + kMinTile - 1) / kMinTile;
     hipError_t e = ensure_partials(c, nbt);
     if (e != hipSuccess) return e;
     size_t grid = 0;
-    if (c->d.mrso != 2 || !launch_final_t<kPT32, float>(c, proj, xi, df, mode, final_consts(c), 0, &grid))
+    if (c->d.mrso != 2 || !launch_final_t<float>(c, proj, xi, df, mode, final_consts(c), 0, &grid))
         return hipErrorNotSupported;
     *nblocks_out = (int)grid;
     return hipGetLastError();
@@ -1145,9 +1206,9 @@ hipError_t launch_angl2proj_feat(mdft_ctx *c, const double *src, int feat, const
 hipError_t launch_transform_f64(mdft_ctx *c, const double *f, double2 *proj, size_t npts, bool to_proj) {
     if (c->d.mrso != 2) return hipErrorNotSupported;
     if (to_proj) return launch_a2p_t<double>(c, f, proj, 4, nullptr, npts) ? hipGetLastError() : hipErrorNotSupported;
-    hipError_t e = ensure_partials(c, (npts + kPTt - 1) / kPTt);
+    hipError_t e = ensure_partials(c, (npts + kMinTile - 1) / kMinTile);
     if (e != hipSuccess) return e;
-    return launch_final_t<kPTt, double>(c, proj, nullptr, const_cast<double *>(f), 5, final_consts(c), npts)
+    return launch_final_t<double>(c, proj, nullptr, const_cast<double *>(f), 5, final_consts(c), npts)
                ? hipGetLastError()
                : hipErrorNotSupported;
 }

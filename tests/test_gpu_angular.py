@@ -43,3 +43,46 @@ def test_tiles_of_points(precision, mmax):
         assert np.abs(parts - pref).max() <= bar * np.abs(pref).max(), (n, parts, pref)
         assert np.abs(df - dref).max() <= bar * np.abs(dref).max(), n
         eng.close()
+
+
+@pytest.mark.parametrize("mmax", range(6))
+def test_fast_step_on_partial_tiles(mmax):
+    """The fast minimiser's evaluation (FP32 iterate of the scaled variables, FP32 gradient, products
+    of the gradient) where the last tile is not full, against the oracle.  The products are FP64
+    sums over the gradient as stored: exact to about sqrt(n) eps of their terms' 2-norm."""
+    import ctypes as C
+    from mdft import ck
+    from mdft.gpu import DEVICE_PTRS, DF_FP32, SCALED_VARS, XI_FP32, DeviceBuffer, Engine
+    from oracle import oracle as O
+    table = ck.synthetic_ck(mmax, 512, 0.05, seed=11, n0=0.0333)
+    dp = C.POINTER(C.c_double)
+    for n in GRIDS:
+        length = [0.5 * v for v in n]
+        print(f"[angular] step mmax={mmax} {n}", flush=True)
+        eng = Engine(n, length, mmax, 2, 2.4777, 0.0333, "fp32")
+        ora = O.Oracle(n, length, mmax, 2, 2.4777, 0.0333)
+        for e in (eng, ora):
+            e.set_ck(table)
+        rng = np.random.default_rng(sum(n))
+        vext = rng.uniform(-2.0, 5.0, eng.N * eng.no)
+        eng.set_vext(vext)
+        w = eng.quadrature()[2]
+        s = np.tile(np.sqrt(w / w.mean()), eng.N)
+        u = (s * (1.0 + 0.3 * rng.uniform(-1, 1, eng.N * eng.no))).astype(np.float32)
+        vecs = [rng.standard_normal(u.size).astype(np.float32) for _ in range(2)]
+        du, dg, *dv = (DeviceBuffer(eng, 4 * u.size) for _ in range(4))
+        for b, v in ((du, u), (dv[0], vecs[0]), (dv[1], vecs[1])):
+            b.upload(v)
+        parts, dots = np.zeros(3), np.zeros(3)
+        ptrs = (C.c_void_p * 3)(dv[0].ptr, dg.ptr, dv[1].ptr)
+        eng._check(eng.lib.mdft_energy_and_gradient_dots(eng._h, du.ptr, parts.ctypes.data_as(dp), dg.ptr,
+                                                         DEVICE_PTRS | DF_FP32 | SCALED_VARS | XI_FP32, 3, ptrs,
+                                                         dots.ctypes.data_as(dp)))
+        df = dg.download(np.float32).astype(np.float64)
+        pref, dref = ora.energy_and_gradient(u.astype(np.float64) / s, vext)
+        dref = dref / s
+        assert np.abs(parts - pref).max() <= 1e-5 * np.abs(pref).max(), (n, parts, pref)
+        assert np.abs(df - dref).max() <= 1e-5 * np.abs(dref).max(), n
+        for got, v in zip(dots, (vecs[0].astype(np.float64), df, vecs[1].astype(np.float64))):
+            assert abs(got - df @ v) <= 1e-15 * np.sqrt(df.size) * (np.abs(df) @ np.abs(v)), (n, got, df @ v)
+        eng.close()

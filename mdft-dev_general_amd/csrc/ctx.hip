@@ -275,14 +275,15 @@ int run_excess_pipeline(mdft_ctx *c, const double *xi, int stage, bool timers) {
     HIPCHK(c, bf16 ? launch_angl2proj_bf16(c, xi, p32)
                    : (f32 ? launch_angl2proj_f32(c, xi, p32) : launch_angl2proj_f64(c, xi, p64)));
     if (timers) HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
-    if (stage >= 2) HIPCHK(c, f32 ? launch_fft3d_f32(c, p32, +1) : launch_fft3d_f64(c, p64, +1));
+    const int nf = c->packed ? c->npk : c->np;
+    if (stage >= 2) HIPCHK(c, f32 ? launch_fft3d_f32(c, p32, +1, nf) : launch_fft3d_f64(c, p64, +1, nf));
     if (timers) HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
     if (stage >= 3) {
         if (ozm_supported(c)) HIPCHK(c, f32 ? launch_ozm_f32(c, p32) : launch_ozm_f64(c, p64));
         else HIPCHK(c, f32 ? launch_oz32(c, p32) : launch_oz_f64(c, p64));
     }
     if (timers) HIPCHK(c, hipEventRecord(c->ev[3], c->stream));
-    if (stage >= 4) HIPCHK(c, f32 ? launch_fft3d_f32(c, p32, -1) : launch_fft3d_f64(c, p64, -1));
+    if (stage >= 4) HIPCHK(c, f32 ? launch_fft3d_f32(c, p32, -1, nf) : launch_fft3d_f64(c, p64, -1, nf));
     if (timers) HIPCHK(c, hipEventRecord(c->ev[4], c->stream));
     return MDFT_OK;
 }
@@ -486,6 +487,10 @@ int mdft_ctx_create(const mdft_desc *desc, mdft_ctx **out) {
             return bad(MDFT_ENOMEM, "device allocation failed");
     }
     if (ozm_setup(c) != MDFT_OK) return bad(MDFT_ENOMEM, "matrix-core q-space tables");
+    if (d.mrso == 2 && c->L <= 5 && d.precision != MDFT_PREC_BF16 && ozm_supported(c)) {
+        const int npk[6] = {Packed<0>::np, Packed<1>::np, Packed<2>::np, Packed<3>::np, Packed<4>::np, Packed<5>::np};
+        c->npk = npk[c->L];
+    }
     AngTables &t = c->ang;
     t.ntheta = c->ntheta;
     t.nphi = c->nphi;
@@ -521,7 +526,7 @@ void mdft_ctx_destroy(mdft_ctx *c) {
                     c->d_partials, c->d_slices, c->d_sums, c->d_vpart, c->d_mpart, c->d_oz32_ftab, c->d_oz32_lanerow,
                     c->d_ozm_frag, c->d_ozm_frag16, c->d_ozm_col, c->d_ozm_ftab, c->d_ozm_units, c->d_ozm_rlen,
                     c->d_bf16_M, c->d_bf16_Q, c->d_chscale, c->d_adjscale, c->d_vscale, c->d_dpart, c->d_vext32,
-                    c->d_a2p_img[0], c->d_a2p_img[1]};
+                    c->d_a2p_img[0], c->d_a2p_img[1], c->d_a2p_img[2], c->d_a2p_img[3], c->d_ozm_pack};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
     free_pairs(c->pairs);
@@ -750,10 +755,14 @@ static int evaluate(mdft_ctx *c, const double *xi, double *df, int flags, int mo
     }
     c->vsinv = scaled ? c->d_vscale + c->no : nullptr;
     c->xi32 = x32 ? reinterpret_cast<const float *>(xi) : nullptr;
+    // the field of an evaluation is real: its transforms need only the packed projections.  (BF16
+    // contexts and orders above 5 have dense or generic angular kernels, over all projections.)
+    c->packed = c->npk > 0;
     rc = run_excess_pipeline(c, xd, 4, timers);
     if (rc) {
         c->vsinv = nullptr;
         c->xi32 = nullptr;
+        c->packed = false;
         return rc;
     }
     int nb = 0;
@@ -766,6 +775,7 @@ static int evaluate(mdft_ctx *c, const double *xi, double *df, int flags, int mo
     c->vsinv = nullptr;
     c->xi32 = nullptr;
     c->dot_k = 0;
+    c->packed = false;
     HIPCHK(c, fe);
     if (fused_dots) {
         HIPCHK(c, launch_reduce3_buf(c, c->d_dpart, nb, c->d_sums + 5));

@@ -523,27 +523,60 @@ template <int L, typename T> __device__ __forceinline__ void phi_synthesis(T *f)
 
 // One projection of the theta contraction: out = (sum_it ax[it] F_it.x, sum_it ay[it] F_it.y) with
 // F_it the coefficient at `item` of the rows of a point.  The signs of mup < 0 at mu2 = 0 (the
-// conjugate of mup > 0 times (-1)^mup) and all norms are in the weights.
+// conjugate of mup > 0 times (-1)^mup), the pairs of real projections and all norms are in the weights.
 template <int L, typename T> struct OutLane {
     T ax[L + 1], ay[L + 1];
     int item;
 };
 
-template <int L, typename T>
+// (m, mup, mu2) of packed entry e; of a pair of real projections m = 2 j and mup = 0
+template <int L> __device__ inline void packed_entry(int e, int &m, int &mup, int &mu2) {
+    using P = Packed<L>;
+    m = mup = mu2 = 0;
+    if (e >= P::pair0) {
+        m = 2 * (e - P::pair0);
+        return;
+    }
+    for (int it = 1; it < Rows<L>::NF; it++) {
+        const int k = it <= L ? it : (it - L - 1) % P::W - L, u = it <= L ? 0 : (it - L - 1) / P::W + 1;
+        const int o = P::off(k, u), lo = P::mlo(k, u);
+        if (lo <= L && e >= o && e < o + L + 1 - lo) {
+            m = lo + e - o;
+            mup = k;
+            mu2 = u;
+            return;
+        }
+    }
+}
+
+// weights of the projections in the context's order, or (PACK) of the packed entries
+template <int L, typename T, bool PACK>
 __global__ void out_lanes_build(OutLane<L, T> *__restrict__ out, AngTables t) {
     using R = Rows<L>;
-    for (int ip = threadIdx.x; ip < R::NP; ip += blockDim.x) {
-        const int mup = t.pmup[ip], mu2 = t.pmu[ip] / 2;
-        const bool conj = mu2 == 0 && mup < 0;
+    constexpr int NOUT = PACK ? Packed<L>::np : R::NP;
+    const double nrm = 1.0 / (double)(R::NPHI * R::NPSI);
+    for (int i = threadIdx.x; i < NOUT; i += blockDim.x) {
+        int m, mup, mu2, ip = i;
+        if (PACK) {
+            packed_entry<L>(i, m, mup, mu2);
+            ip = t.pidx[(m * R::W + mup + L) * (R::H + 1) + mu2];
+        } else {
+            m = t.pm[ip];
+            mup = t.pmup[ip];
+            mu2 = t.pmu[ip] / 2;
+        }
+        const bool conj = mu2 == 0 && mup < 0, real = mu2 == 0 && mup == 0;
+        const int ip2 = (PACK && real && m < L) ? t.pidx[((m + 1) * R::W + L) * (R::H + 1)] : -1;
         OutLane<L, T> o;
         for (int it = 0; it < R::NTH; it++) {
-            const double a = t.a2p[ip * R::NTH + it] * t.fm[ip] / (double)(R::NPHI * R::NPSI);
             // d^m(mup, 0) already has the sign (-1)^mup of d^m(-mup, 0)
+            const double a = t.a2p[ip * R::NTH + it] * t.fm[ip] * nrm;
+            const double a2 = ip2 < 0 ? 0.0 : t.a2p[ip2 * R::NTH + it] * t.fm[ip2] * nrm;
             o.ax[it] = (T)a;
-            o.ay[it] = (T)(mu2 == 0 && mup == 0 ? 0.0 : (conj ? -a : a));
+            o.ay[it] = (T)(real ? a2 : (conj ? -a : a));
         }
         o.item = R::item(conj ? -mup : mup, mu2);
-        out[ip] = o;
+        out[i] = o;
     }
 }
 
@@ -560,7 +593,7 @@ __global__ void out_lanes_build(OutLane<L, T> *__restrict__ out, AngTables t) {
 // projection, tables in LDS: 2.22 and 3.72 ms, the time of its reads of values and twiddles from LDS.)
 // The theta contraction gives a thread one projection, its weights in registers, and a group of
 // threads consecutive projections of a point, so the stores are whole records.
-template <int L, int PT, int TH, typename T>
+template <int L, int PT, int TH, typename T, bool PACK>
 __global__ __launch_bounds__(TH) void angl2proj_t(const double *__restrict__ xi, typename C2<T>::t *__restrict__ proj,
                                                  size_t N, AngTables t, double k0, int feat, double beta,
                                                  const double *__restrict__ aux, const double *__restrict__ vsinv,
@@ -568,7 +601,7 @@ __global__ __launch_bounds__(TH) void angl2proj_t(const double *__restrict__ xi,
                                                  const OutLane<L, T> *__restrict__ lanes) {
     using R = Rows<L>;
     using V = typename C2<T>::t;
-    constexpr int NO = R::NO, NTH = R::NTH, NOUT = R::NP, ROW = R::ROW, RS = R::RS;
+    constexpr int NO = R::NO, NTH = R::NTH, NOUT = PACK ? Packed<L>::np : R::NP, ROW = R::ROW, RS = R::RS;
     __shared__ T rows[NTH * PT * RS];  // row of (point, theta) at theta PT + point
     __shared__ double sth[NTH];        // 1 / s of each theta (the weights, hence s, depend on theta only)
     const int tid = threadIdx.x;
@@ -654,7 +687,7 @@ template <int L, typename T> struct FinalShape {
 // memory operations issued after it, so the product operands loaded ahead stay in flight.  The
 // last tile of a grid that is not a whole number of tiles starts early, over points of the one
 // before it (whose dF is written twice, with the same values); those add nothing to the sums.
-template <int L, typename T, bool DOT32 = false>
+template <int L, typename T, bool DOT32, bool PACK>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FinalShape<L, T>::WAVES, 8))) void final_t(
     const typename C2<T>::t *__restrict__ proj, const double *__restrict__ xi, const double *__restrict__ vext,
     double *__restrict__ df, double *__restrict__ partials, size_t N, AngTables t, FinalConsts k, int mode,
@@ -663,30 +696,45 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FinalS
     using R = Rows<L>;
     using V = typename C2<T>::t;
     constexpr int PT = FinalShape<L, T>::PT;
-    constexpr int NO = R::NO, NP = R::NP, NTH = R::NTH, NPSI = R::NPSI, H = R::H, W = R::W;
+    constexpr int NO = R::NO, NP = PACK ? Packed<L>::np : R::NP, NTH = R::NTH, NPSI = R::NPSI, H = R::H, W = R::W;
+    constexpr int NW = PACK ? Packed<L>::pair0 + L + 1 : NP;  // rows of the theta weights
     constexpr int ROW = R::ROW, RS = R::RS, NF = R::NF;
     constexpr int NPS = NP | 1;  // odd: the records of consecutive points in different banks
     if constexpr (DOT32) mode = 0;
     __shared__ __align__(16) V Gm[PT * NPS];
     __shared__ T rows[NTH * PT * RS];  // row of (point, theta) at theta PT + point
     __shared__ V twpsi[NPSI * (H + 1)];  // (cos, sin)(2 pi mu2 ipsi / npsi) at [ipsi][mu2]
-    __shared__ T p2a[NP * NTH];          // twice the table's for mu2 > 0 (the weight of +-mu2 in the c2r)
+    // theta weights, twice the table's for mu2 > 0 (the weight of +-mu2 in the c2r) and, packed, for mup > 0
+    // of mu2 = 0 (mup and -mup); by projection, or by packed entry with one row per m of the real ones
+    __shared__ T p2a[NW * NTH];
     __shared__ double wth[NTH];          // the weights depend on theta only
     __shared__ double sth[NTH];          // 1 / s of each theta
-    // projection index of (m, mup, mu2) and (m, -mup, 0), as bytes: the loaded index is then known to be small
+    // projection index or packed entry of (m, mup, mu2), projection index of (m, -mup, 0), as bytes: the loaded index is then known to be small
     // and its products stay 24-bit multiplies (entries with m below the item's lowest m are never read)
-    static_assert(NP <= 255, "projection indices are stored as bytes");
+    static_assert(R::NP <= 255, "projection indices are stored as bytes");
     __shared__ unsigned char pidx[(L + 1) * NF], pneg[(L + 1) * (L + 1)];
     __shared__ unsigned char ford[NF];  // the theta synthesis' (mup, mu2) items, longest m loop first
     const int tid = threadIdx.x;
     auto mup_of = [](int it) { return it <= L ? it : (it - L - 1) % W - L; };
     auto mu_of = [](int it) { return it <= L ? 0 : (it - L - 1) / W + 1; };
     for (int i = tid; i < (L + 1) * NF; i += kThreads) {
-        const int m = i / NF, it = i % NF;
-        pidx[i] = (unsigned char)t.pidx[(m * W + mup_of(it) + L) * (H + 1) + mu_of(it)];
+        const int m = i / NF, it = i % NF, mup = mup_of(it), mu2 = mu_of(it), lo = Packed<L>::mlo(mup, mu2);
+        const int ip = t.pidx[(m * W + mup + L) * (H + 1) + mu2];
+        if (m < lo) continue;
+        int row = ip;
+        if constexpr (PACK) {
+            row = it == 0 ? Packed<L>::pair0 + m : Packed<L>::off(mup, mu2) + m - lo;
+            pidx[i] = (unsigned char)(it == 0 ? Packed<L>::pair0 + m / 2 : row);
+        } else {
+            pidx[i] = (unsigned char)ip;
+        }
+        const double f = (mu2 > 0 || (PACK && it != 0)) ? 2.0 : 1.0;
+        for (int th = 0; th < NTH; th++) p2a[row * NTH + th] = (T)(f * t.p2a[ip * NTH + th]);
     }
-    for (int i = tid; i < (L + 1) * (L + 1); i += kThreads)
-        pneg[i] = (unsigned char)t.pidx[((i / (L + 1)) * W - i % (L + 1) + L) * (H + 1)];
+    if constexpr (!PACK) {  // (mu2 = 0, mup < 0 has the weights of mup > 0 in its sum)
+        for (int i = tid; i < (L + 1) * (L + 1); i += kThreads)
+            pneg[i] = (unsigned char)t.pidx[((i / (L + 1)) * W - i % (L + 1) + L) * (H + 1)];
+    }
     {
         // an item sums over m = max(|mup|, 2 mu2) .. L; ranked by that length (ties by index),
         // the lanes of a wave take loops of nearly one length
@@ -709,7 +757,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FinalS
         const int kk = ((i % (H + 1)) * (i / (H + 1))) % NPSI;
         twpsi[i] = mk<V>((T)t.cps[kk], (T)t.sps[kk]);
     }
-    for (int i = tid; i < NP * NTH; i += kThreads) p2a[i] = (T)(t.pmu[i / NTH] > 0 ? 2.0 * t.p2a[i] : t.p2a[i]);
     for (int i = tid; i < NTH; i += kThreads) {
         wth[i] = t.w[i * ROW];
         sth[i] = vsinv ? vsinv[i * ROW] : 1.0;
@@ -790,7 +837,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FinalS
         // f(theta, mup, mu2) = sum_m p(m, mup, mu2) d(theta) fm(m): one thread per (point, mup, mu2),
         // all theta at once (each projection read once); items by rank of their loop length, the
         // tile's points innermost.  mu2 = 0: the psi step takes the real part of the sum over mup, so
-        // the items mup > 0 hold p(m, mup, 0) + (-1)^mup conj(p(m, -mup, 0)) and mup = 0 the real part
+        // the items mup > 0 hold p(m, mup, 0) + (-1)^mup conj(p(m, -mup, 0)), packed twice p(m, mup, 0),
+        // and mup = 0 the real part
         for (int i = tl; i < PT * NF; i += kThreads) {
             const int rk = i / PT, pt = i - rk * PT;
             if (pt >= npts) continue;
@@ -804,7 +852,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FinalS
                 const int mup = rest - mu1 * W - L, a = mup < 0 ? -mup : mup, b = 2 * mu1 + 2;
                 mlo = a > b ? a : b;
             }
-            const T sg = (item & 1) ? (T)-1 : (T)1;
+            [[maybe_unused]] const T sg = (item & 1) ? (T)-1 : (T)1;
             T re[NTH], im[NTH];
     #pragma unroll
             for (int it = 0; it < NTH; it++) re[it] = im[it] = (T)0;
@@ -812,12 +860,17 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FinalS
             for (int m = mlo; m <= L; m++) {
                 const unsigned p = pidx[m * NF + item];
                 V v = gp[p];
-                if (neg == 1) {
+                const T *c = p2a + p * NTH;
+                if constexpr (PACK) {
+                    if (neg == 2) {
+                        if (m & 1) v.x = v.y;
+                        c = p2a + (Packed<L>::pair0 + m) * NTH;
+                    }
+                } else if (neg == 1) {
                     const V u = gp[pneg[m * (L + 1) + item]];
                     v.x = fma(sg, u.x, v.x);
                     v.y = fma(-sg, u.y, v.y);
                 }
-                const T *c = p2a + p * NTH;
     #pragma unroll
                 for (int it = 0; it < NTH; it++) {
                     re[it] += v.x * c[it];
@@ -1032,22 +1085,22 @@ template <int L> struct A2pShape {
     static constexpr int PT = L >= 4 ? 16 : L == 3 ? 32 : L == 2 ? 64 : L == 1 ? 128 : 256, TH = L == 4 ? 192 : 256;
 };
 
-template <typename T>
+template <typename T, bool PACK = false>
 bool launch_a2p_t(mdft_ctx *c, const double *xi, typename C2<T>::t *proj, int feat = 0, const double *aux = nullptr,
                   size_t npts = 0) {
     if (!npts) npts = c->N;
     const double beta = 1.0 / c->d.kT;
     const double k0 = (feat == 3) ? 0.5 * c->dv : c->rho0;
-    void *&img = c->d_a2p_img[sizeof(T) == 8];
+    void *&img = c->d_a2p_img[(sizeof(T) == 8) + 2 * PACK];
     switch (c->L) {
 #define A2P_CASE(LL) \
     case LL: { \
         using S = A2pShape<LL>; \
         if (!img) { \
             if (hipMalloc(&img, sizeof(OutLane<LL, T>) * Rows<LL>::NP) != hipSuccess) { img = nullptr; return false; } \
-            hipLaunchKernelGGL((out_lanes_build<LL, T>), dim3(1), dim3(128), 0, c->stream, static_cast<OutLane<LL, T> *>(img), c->ang); \
+            hipLaunchKernelGGL((out_lanes_build<LL, T, PACK>), dim3(1), dim3(128), 0, c->stream, static_cast<OutLane<LL, T> *>(img), c->ang); \
         } \
-        hipLaunchKernelGGL((angl2proj_t<LL, S::PT, S::TH, T>), dim3((unsigned)((npts + S::PT - 1) / S::PT)), dim3(S::TH), 0, c->stream, xi, proj, npts, c->ang, k0, feat, beta, aux, feat == 0 ? c->vsinv : nullptr, feat == 0 ? c->xi32 : nullptr, static_cast<const OutLane<LL, T> *>(img)); \
+        hipLaunchKernelGGL((angl2proj_t<LL, S::PT, S::TH, T, PACK>), dim3((unsigned)((npts + S::PT - 1) / S::PT)), dim3(S::TH), 0, c->stream, xi, proj, npts, c->ang, k0, feat, beta, aux, feat == 0 ? c->vsinv : nullptr, feat == 0 ? c->xi32 : nullptr, static_cast<const OutLane<LL, T> *>(img)); \
         return true; \
     }
         A2P_CASE(0) A2P_CASE(1) A2P_CASE(2) A2P_CASE(3) A2P_CASE(4) A2P_CASE(5)
@@ -1056,7 +1109,7 @@ bool launch_a2p_t(mdft_ctx *c, const double *xi, typename C2<T>::t *proj, int fe
     }
 }
 
-template <typename T>
+template <typename T, bool PACK = false>
 bool launch_final_t(mdft_ctx *c, const typename C2<T>::t *proj, const double *xi, double *df, int mode, FinalConsts k,
                     size_t npts = 0, size_t *grid_out = nullptr) {
     if (!npts) npts = c->N;
@@ -1068,21 +1121,23 @@ bool launch_final_t(mdft_ctx *c, const typename C2<T>::t *proj, const double *xi
         for (int j = 0; j < 3; j++) da.p[j] = c->dot_vec[j];
     }
     // the FP32 kernel forming products over FP32 vectors (dF then FP32 too) has its own variant
-    const bool dot32 = sizeof(T) == 4 && mode == 0 && da.k > 0 && da.f32 && c->xi32 && c->vext32_ok;
+    [[maybe_unused]] const bool dot32 = sizeof(T) == 4 && mode == 0 && da.k > 0 && da.f32 && c->xi32 && c->vext32_ok;
     switch (c->L) {
 #define FIN_CASE(LL) \
     case LL: { \
         constexpr int PT = FinalShape<LL, T>::PT; \
         const size_t ntiles = (npts + PT - 1) / PT; \
-        if (dot32 && npts >= PT) { \
-            const size_t nb = resident_grid(c, final_t<LL, T, sizeof(T) == 4>, ntiles); \
-            if (grid_out) *grid_out = nb; \
-            hipLaunchKernelGGL((final_t<LL, T, sizeof(T) == 4>), dim3((unsigned)nb), dim3(kThreads), 0, c->stream, proj, xi, c->d_vext, df, c->d_partials, npts, c->ang, k, mode, c->df32, c->vsinv, da, c->d_dpart, c->xi32, c->d_vext32); \
-        } else { \
-            const size_t nb = oversubscribed_grid(c, ntiles); \
-            if (grid_out) *grid_out = nb; \
-            hipLaunchKernelGGL((final_t<LL, T>), dim3((unsigned)nb), dim3(kThreads), 0, c->stream, proj, xi, c->d_vext, df, c->d_partials, npts, c->ang, k, mode, mode == 0 ? c->df32 : nullptr, mode == 0 ? c->vsinv : nullptr, da, c->d_dpart, mode == 0 ? c->xi32 : nullptr, nullptr); \
+        if constexpr (PACK && sizeof(T) == 4) { \
+            if (dot32 && npts >= PT) { \
+                const size_t nb = resident_grid(c, final_t<LL, T, true, true>, ntiles); \
+                if (grid_out) *grid_out = nb; \
+                hipLaunchKernelGGL((final_t<LL, T, true, true>), dim3((unsigned)nb), dim3(kThreads), 0, c->stream, proj, xi, c->d_vext, df, c->d_partials, npts, c->ang, k, mode, c->df32, c->vsinv, da, c->d_dpart, c->xi32, c->d_vext32); \
+                return true; \
+            } \
         } \
+        const size_t nb = oversubscribed_grid(c, ntiles); \
+        if (grid_out) *grid_out = nb; \
+        hipLaunchKernelGGL((final_t<LL, T, false, PACK>), dim3((unsigned)nb), dim3(kThreads), 0, c->stream, proj, xi, c->d_vext, df, c->d_partials, npts, c->ang, k, mode, mode == 0 ? c->df32 : nullptr, mode == 0 ? c->vsinv : nullptr, da, c->d_dpart, mode == 0 ? c->xi32 : nullptr, nullptr); \
         return true; \
     }
         FIN_CASE(0) FIN_CASE(1) FIN_CASE(2) FIN_CASE(3) FIN_CASE(4) FIN_CASE(5)
@@ -1093,6 +1148,7 @@ bool launch_final_t(mdft_ctx *c, const typename C2<T>::t *proj, const double *xi
 
 
 hipError_t launch_angl2proj_f64(mdft_ctx *c, const double *xi, double2 *proj) {
+    if (c->packed) return launch_a2p_t<double, true>(c, xi, proj) ? hipGetLastError() : hipErrorNotSupported;
     if (c->d.mrso == 2 && launch_a2p_t<double>(c, xi, proj)) return hipGetLastError();
     const size_t nb = (c->N + kPT - 1) / kPT;
     if (a2p_lds(c->ang) > c->lds_limit) return hipErrorInvalidConfiguration;
@@ -1118,7 +1174,8 @@ hipError_t launch_final_f64(mdft_ctx *c, const double2 *proj, const double *xi, 
         const size_t nbt = (c->N + kMinTile - 1) / kMinTile;
         if ((e = ensure_partials(c, nbt)) != hipSuccess) return e;
         size_t grid = 0;
-        if (launch_final_t<double>(c, proj, xi, df, mode, k, 0, &grid)) {
+        if (c->packed ? launch_final_t<double, true>(c, proj, xi, df, mode, k, 0, &grid)
+                      : launch_final_t<double>(c, proj, xi, df, mode, k, 0, &grid)) {
             *nblocks_out = (int)grid;
             return hipGetLastError();
         }
@@ -1174,6 +1231,7 @@ FinalConsts final_consts(mdft_ctx *c) {
 }
 
 hipError_t launch_angl2proj_f32(mdft_ctx *c, const double *xi, float2 *proj) {
+    if (c->packed) return launch_a2p_t<float, true>(c, xi, proj) ? hipGetLastError() : hipErrorNotSupported;
     if (c->d.mrso != 2 || !launch_a2p_t<float>(c, xi, proj)) return hipErrorNotSupported;
     return hipGetLastError();
 }
@@ -1183,7 +1241,8 @@ hipError_t launch_final_f32(mdft_ctx *c, const float2 *proj, const double *xi, d
     hipError_t e = ensure_partials(c, nbt);
     if (e != hipSuccess) return e;
     size_t grid = 0;
-    if (c->d.mrso != 2 || !launch_final_t<float>(c, proj, xi, df, mode, final_consts(c), 0, &grid))
+    if (c->d.mrso != 2 || !(c->packed ? launch_final_t<float, true>(c, proj, xi, df, mode, final_consts(c), 0, &grid)
+                                      : launch_final_t<float>(c, proj, xi, df, mode, final_consts(c), 0, &grid)))
         return hipErrorNotSupported;
     *nblocks_out = (int)grid;
     return hipGetLastError();

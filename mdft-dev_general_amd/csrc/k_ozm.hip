@@ -200,6 +200,7 @@ template <typename T> struct OzmArgs {
     int ntiles, per;
     const TilePair *tpair;      // [tile][8] the tiles' pairs
     const int *pmup;            // mup of each projection
+    const int *pack;            // packed entries: projection | second << 8 | kind << 16 | (mup + 16) << 20
     const T *frag;              // [interval][nfrag][64] B fragments of (c[iq], c[iq+1])
     const bf16x8 *frag16;       // BF16 contexts: [interval][nfrag32][64] B fragments, 8 values per lane
     const int *colent;          // [2 L + 1][32] OZ column entries (entry << 1 | own side) of each block
@@ -512,9 +513,91 @@ __device__ __forceinline__ void oz_wave(Lds<T, L> &s, const OzmArgs<T> &a, size_
     }
 }
 
+// ---- packed records (packed.h).  kind 0: one projection; 1: p(m, mup, 0), mup > 0, which gives
+// p(m, -mup, 0)(q) = (-1)^mup conj p(m, mup, 0)(-q) as well; 2: p(m, 0, 0) + i p(m + 1, 0, 0).
+// Into the rows of q and -q of pair pr, in FP32 times exp(-i mup phi) (see rot_class).
+template <typename T, int L>
+__device__ __forceinline__ void unpack(int d, typename Ty<T>::c xq, typename Ty<T>::c xm, Lds<T, L> &s, int pr) {
+    using C = typename Ty<T>::c;
+    const int ip = d & 255, ip2 = (d >> 8) & 255, kind = (d >> 16) & 3, mup = (d >> 20) - 16;
+    if (kind == 2) {  // mup = 0: no phase
+        C e, o;
+        e.x = (T)0.5 * (xq.x + xm.x);
+        e.y = (T)0.5 * (xq.y - xm.y);
+        o.x = (T)0.5 * (xq.y + xm.y);
+        o.y = (T)-0.5 * (xq.x - xm.x);
+        s.xs[pr][ip] = e;
+        e.y = -e.y;
+        s.xs[8 + pr][ip] = e;
+        if (ip2 != 255) {
+            s.xs[pr][ip2] = o;
+            o.y = -o.y;
+            s.xs[8 + pr][ip2] = o;
+        }
+        return;
+    }
+    if constexpr (sizeof(T) == 4) {
+        const C z = s.ph[pr][mup < 0 ? -mup : mup];
+        const T ex = z.x, ey = mup < 0 ? z.y : -z.y;
+        const C u = xq, v = xm;
+        xq.x = u.x * ex - u.y * ey;
+        xq.y = u.x * ey + u.y * ex;
+        xm.x = v.x * ex - v.y * ey;
+        xm.y = v.x * ey + v.y * ex;
+    }
+    s.xs[pr][ip] = xq;
+    s.xs[8 + pr][ip] = xm;
+    if (kind == 1) {
+        const T sg = (mup & 1) ? (T)-1 : (T)1;
+        C c;
+        c.x = sg * xm.x;
+        c.y = -sg * xm.y;
+        s.xs[pr][ip2] = c;
+        c.x = sg * xq.x;
+        c.y = -sg * xq.y;
+        s.xs[8 + pr][ip2] = c;
+    }
+}
+
+// The part of the rotated-back outputs that the final pass reads, i.e. the projections of the real
+// part: p(m, mup, 0) <- (p(m, mup, 0)(q) + (-1)^mup conj p(m, -mup, 0)(-q)) / 2.  rq, rm: the rows
+// of q and -q, both the second's where q == -q (the store rule).
+template <typename T, int L>
+__device__ __forceinline__ void pack_out(int d, typename Ty<T>::c &oq, typename Ty<T>::c &om, const Lds<T, L> &s,
+                                         int rq, int rm) {
+    using C = typename Ty<T>::c;
+    const int ip = d & 255, ip2 = (d >> 8) & 255, kind = (d >> 16) & 3, mup = (d >> 20) - 16;
+    oq = s.xs[rq][ip];
+    om = s.xs[rm][ip];
+    if (kind == 1) {
+        const T sg = (mup & 1) ? (T)-1 : (T)1;
+        const C u = s.xs[rm][ip2], v = s.xs[rq][ip2];
+        oq.x = (T)0.5 * (oq.x + sg * u.x);
+        oq.y = (T)0.5 * (oq.y - sg * u.y);
+        om.x = (T)0.5 * (om.x + sg * v.x);
+        om.y = (T)0.5 * (om.y - sg * v.y);
+    } else if (kind == 2) {
+        C o1, o2;
+        o1.x = o1.y = o2.x = o2.y = (T)0;
+        if (ip2 != 255) {
+            o1 = s.xs[rq][ip2];
+            o2 = s.xs[rm][ip2];
+        }
+        C e, o;  // of q; conjugated, of -q
+        e.x = (T)0.5 * (oq.x + om.x);
+        e.y = (T)0.5 * (oq.y - om.y);
+        o.x = (T)0.5 * (o1.x + o2.x);
+        o.y = (T)0.5 * (o1.y - o2.y);
+        oq.x = e.x - o.y;
+        oq.y = e.y + o.x;
+        om.x = e.x + o.y;
+        om.y = o.x - e.y;
+    }
+}
+
 // FP32: at least 7 waves per SIMD (72 registers, no spills; at the compiler's own choice of 88
 // registers, 5 waves and 2.13 against 2.01 ms at 128^3, mmax 5)
-template <typename T, int L, bool BF>
+template <typename T, int L, bool BF, bool PACK>
 __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 7 : 1, 8))) void ozm(typename Ty<T>::c *__restrict__ proj, OzmArgs<T> a) {
     using P = Plan<L>;
     using C = typename Ty<T>::c;
@@ -528,9 +611,27 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(siz
     const int b = blockIdx.x;
     const int tile = (b & 7) * a.per + (b >> 3);
     if (tile >= a.ntiles) return;
-    const int iq = a.tpair[(size_t)tile * 8].iq;  // the same for the tile's pairs
+    const TilePair *tps = a.tpair + (size_t)tile * 8;
+    const int iq = tps[0].iq;  // the same for the tile's pairs
+    // PACK: the records of q and -q, two entries (FP32, whole 16-byte words) or one per access, all
+    // of a thread's loads issued before the angles are formed
+    constexpr int NPK = PACK ? Packed<L>::np : 1, VE = (sizeof(T) == 4 && NPK % 2 == 0) ? 2 : 1;
+    constexpr int NPV = NPK / VE, NIT = (8 * NPV + 64 * kWaves - 1) / (64 * kWaves);
+    struct alignas(VE * sizeof(C)) Vec {
+        C v[VE];
+    };
+    [[maybe_unused]] Vec pa[NIT], pb[NIT];
+    if constexpr (PACK) {
+#pragma unroll
+        for (int k = 0; k < NIT; k++) {
+            const int i = tid + k * 64 * kWaves, ii = i < 8 * NPV ? i : 8 * NPV - 1;
+            const int pr = ii / NPV, e = ii - pr * NPV;
+            pa[k] = reinterpret_cast<const Vec *>(proj + (size_t)tps[pr].gq * NPK)[e];
+            pb[k] = reinterpret_cast<const Vec *>(proj + (size_t)tps[pr].gmq * NPK)[e];
+        }
+    }
     if (tid < 8) {
-        const TilePair tp = a.tpair[(size_t)tile * 8 + tid];
+        const TilePair tp = tps[tid];
         s.g[tid] = tp.gq;
         s.g[8 + tid] = tp.gmq;
         s.flag[tid] = tp.flag;
@@ -555,43 +656,55 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(siz
         }
     }
     __syncthreads();
-    // X of the 16 (side, pair) rows, each row one contiguous record; in FP32 times
-    // exp(-i mup phi) for the factored rotation, two elements per 16-byte access when the
-    // records are a whole number of 16-byte words
-    if constexpr (sizeof(T) == 4 && NP % 2 == 0) {
-        constexpr int NP2 = NP / 2;
-        for (int i = tid; i < 16 * NP2; i += 64 * kWaves) {
-            const int r = i / NP2, e = 2 * (i - r * NP2);
-            const float4 x2 = reinterpret_cast<const float4 *>(proj + (size_t)s.g[r] * NP)[e / 2];
-            C out[2];
+    if constexpr (PACK) {
 #pragma unroll
-            for (int h = 0; h < 2; h++) {
-                const int mup = a.pmup[e + h];
-                const C z = s.ph[r & 7][mup < 0 ? -mup : mup];
-                const T ex = z.x, ey = mup < 0 ? z.y : -z.y;
-                const T ux = h ? x2.z : x2.x, uy = h ? x2.w : x2.y;
-                out[h].x = ux * ex - uy * ey;
-                out[h].y = ux * ey + uy * ex;
-            }
-            s.xs[r][e] = out[0];
-            s.xs[r][e + 1] = out[1];
+        for (int k = 0; k < NIT; k++) {
+            const int i = tid + k * 64 * kWaves;
+            if (i >= 8 * NPV) break;
+            const int pr = i / NPV, e = (i - pr * NPV) * VE;
+#pragma unroll
+            for (int h = 0; h < VE; h++) unpack(a.pack[e + h], pa[k].v[h], pb[k].v[h], s, pr);
         }
+        __syncthreads();
     } else {
-        for (int i = tid; i < 16 * NP; i += 64 * kWaves) {
-            const int r = i / NP, e = i - r * NP;
-            C x = proj[(size_t)s.g[r] * NP + e];
-            if constexpr (sizeof(T) == 4) {
-                const int mup = a.pmup[e];
-                const C z = s.ph[r & 7][mup < 0 ? -mup : mup];
-                const T ex = z.x, ey = mup < 0 ? z.y : -z.y;
-                const C u = x;
-                x.x = u.x * ex - u.y * ey;
-                x.y = u.x * ey + u.y * ex;
+        // X of the 16 (side, pair) rows, each row one contiguous record; in FP32 times
+        // exp(-i mup phi) for the factored rotation, two elements per 16-byte access when the
+        // records are a whole number of 16-byte words
+        if constexpr (sizeof(T) == 4 && NP % 2 == 0) {
+            constexpr int NP2 = NP / 2;
+            for (int i = tid; i < 16 * NP2; i += 64 * kWaves) {
+                const int r = i / NP2, e = 2 * (i - r * NP2);
+                const float4 x2 = reinterpret_cast<const float4 *>(proj + (size_t)s.g[r] * NP)[e / 2];
+                C out[2];
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    const int mup = a.pmup[e + h];
+                    const C z = s.ph[r & 7][mup < 0 ? -mup : mup];
+                    const T ex = z.x, ey = mup < 0 ? z.y : -z.y;
+                    const T ux = h ? x2.z : x2.x, uy = h ? x2.w : x2.y;
+                    out[h].x = ux * ex - uy * ey;
+                    out[h].y = ux * ey + uy * ex;
+                }
+                s.xs[r][e] = out[0];
+                s.xs[r][e + 1] = out[1];
             }
-            s.xs[r][e] = x;
+        } else {
+            for (int i = tid; i < 16 * NP; i += 64 * kWaves) {
+                const int r = i / NP, e = i - r * NP;
+                C x = proj[(size_t)s.g[r] * NP + e];
+                if constexpr (sizeof(T) == 4) {
+                    const int mup = a.pmup[e];
+                    const C z = s.ph[r & 7][mup < 0 ? -mup : mup];
+                    const T ex = z.x, ey = mup < 0 ? z.y : -z.y;
+                    const C u = x;
+                    x.x = u.x * ex - u.y * ey;
+                    x.y = u.x * ey + u.y * ex;
+                }
+                s.xs[r][e] = x;
+            }
         }
+        __syncthreads();
     }
-    __syncthreads();
     rot_all<T, L, P::nclass, false>(a, s, w, p, j);
     __syncthreads();
     {
@@ -603,6 +716,18 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(siz
     rot_all<T, L, P::nclass, true>(a, s, w, p, j);
     __syncthreads();
     // store rule (:648-656): both sides of real pairs; for q == -q only the -q side
+    if constexpr (PACK) {
+        for (int i = tid; i < 8 * NPV; i += 64 * kWaves) {
+            const int pr = i / NPV, e = (i - pr * NPV) * VE, f = s.flag[pr];
+            if (f & 4) continue;
+            Vec oq, om;
+#pragma unroll
+            for (int h = 0; h < VE; h++) pack_out(a.pack[e + h], oq.v[h], om.v[h], s, (f & 1) ? 8 + pr : pr, 8 + pr);
+            if (!(f & 1)) reinterpret_cast<Vec *>(proj + (size_t)s.g[pr] * NPK)[e / VE] = oq;
+            reinterpret_cast<Vec *>(proj + (size_t)s.g[8 + pr] * NPK)[e / VE] = om;
+        }
+        return;
+    }
     if constexpr (sizeof(T) == 4 && NP % 2 == 0) {
         constexpr int NP2 = NP / 2;
         for (int i = tid; i < 16 * NP2; i += 64 * kWaves) {
@@ -679,12 +804,13 @@ HostPlan host_plan_of(int L) {
     }
 }
 
-template <typename T, int L, bool BF> hipError_t launch_ozm_t(mdft_ctx *c, typename Ty<T>::c *proj) {
+template <typename T, int L, bool BF, bool PACK = false> hipError_t launch_ozm_t(mdft_ctx *c, typename Ty<T>::c *proj) {
     OzmArgs<T> a;
     a.ntiles = c->pairs.ntiles;
     a.per = (c->pairs.ntiles + 7) / 8;
     a.tpair = c->pairs.tpair;
     a.pmup = c->d_pmup;
+    a.pack = c->d_ozm_pack;
     a.frag = static_cast<const T *>(c->d_ozm_frag);
     a.frag16 = static_cast<const bf16x8 *>(c->d_ozm_frag16);
     a.colent = c->d_ozm_col;
@@ -700,11 +826,22 @@ template <typename T, int L, bool BF> hipError_t launch_ozm_t(mdft_ctx *c, typen
     if (a.ntiles == 0) return hipSuccess;
     const size_t lds = sizeof(Lds<T, L>);
     if (lds > c->lds_limit) return hipErrorInvalidConfiguration;
-    hipLaunchKernelGGL((ozm<T, L, BF>), dim3((unsigned)(8 * a.per)), dim3(64 * kWaves), lds, c->stream, proj, a);
+    hipLaunchKernelGGL((ozm<T, L, BF, PACK>), dim3((unsigned)(8 * a.per)), dim3(64 * kWaves), lds, c->stream, proj, a);
     return hipGetLastError();
 }
 
 template <typename T, bool BF> hipError_t launch_ozm_any(mdft_ctx *c, typename Ty<T>::c *proj) {
+    if constexpr (!BF) {
+        if (c->packed) switch (c->L) {
+                case 0: return launch_ozm_t<T, 0, false, true>(c, proj);
+                case 1: return launch_ozm_t<T, 1, false, true>(c, proj);
+                case 2: return launch_ozm_t<T, 2, false, true>(c, proj);
+                case 3: return launch_ozm_t<T, 3, false, true>(c, proj);
+                case 4: return launch_ozm_t<T, 4, false, true>(c, proj);
+                case 5: return launch_ozm_t<T, 5, false, true>(c, proj);
+                default: return hipErrorInvalidConfiguration;
+            }
+    }
     switch (c->L) {
         case 0: return launch_ozm_t<T, 0, BF>(c, proj);
         case 1: return launch_ozm_t<T, 1, BF>(c, proj);
@@ -860,6 +997,21 @@ int ozm_setup(mdft_ctx *c) {
     if (hipMemcpy(c->d_ozm_units, units.data(), sizeof(int) * units.size(), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(c->d_ozm_rlen, rlen.data(), sizeof(int) * rlen.size(), hipMemcpyHostToDevice) != hipSuccess)
         return MDFT_EHIP;
+    if (L <= 5) {  // packed entries
+        std::vector<int> pk;
+        auto item = [&](int mup, int mu2) {
+            for (int m = std::max(std::abs(mup), 2 * mu2); m <= L; m++)
+                pk.push_back(pidx(m, mup, mu2) | (mu2 == 0 ? pidx(m, -mup, 0) | 1 << 8 : 255) << 8 | (mup + 16) << 20);
+        };
+        for (int mup = 1; mup <= L; mup++) item(mup, 0);
+        for (int mu2 = 1; mu2 <= L / 2; mu2++)
+            for (int mup = -L; mup <= L; mup++) item(mup, mu2);
+        for (int m = 0; m <= L; m += 2)
+            pk.push_back(pidx(m, 0, 0) | (m < L ? pidx(m + 1, 0, 0) : 255) << 8 | 2 << 16 | 16 << 20);
+        if (hipMalloc((void **)&c->d_ozm_pack, sizeof(int) * pk.size()) != hipSuccess) return MDFT_ENOMEM;
+        if (hipMemcpy(c->d_ozm_pack, pk.data(), sizeof(int) * pk.size(), hipMemcpyHostToDevice) != hipSuccess)
+            return MDFT_EHIP;
+    }
     // OZ column entries of each block (entry << 1 | own side; padding columns read entry 0), 32 per block
     std::vector<int> colent;
     for (int khi = -L; khi <= L; khi++)

@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "mdft_gpu.h"
+#include "packed.h"
 
 #define MDFT_MAX_MMAX 6
 #define MDFT_VEC_MAX 16  // vectors per multi-dot / combine pass
@@ -121,7 +122,10 @@ struct mdft_ctx {
     const void *dot_vec[3] = {nullptr, nullptr, nullptr};
     double *d_dpart = nullptr;    // [blocks][3] their block partials
     float *d_vext32 = nullptr;    // FP32 copy of vext read by the fast minimiser's final pass
-    void *d_a2p_img[2] = {nullptr, nullptr};  // angl2proj_t's LDS table image, FP32 and FP64
+    void *d_a2p_img[4] = {};      // angl2proj_t's weights: FP32, FP64, packed FP32, packed FP64
+    bool packed = false;          // set during an evaluation whose projection field is packed (packed.h)
+    int npk = 0;                  // packed projections per point
+    int *d_ozm_pack = nullptr;    // packed entries of the q-space kernel
     bool vext32_ok = false;       // d_vext32 holds the current vext
     size_t dpart_cap = 0;
     float *d_chscale = nullptr;   // per-channel input scale of the warm-start features [2 np]

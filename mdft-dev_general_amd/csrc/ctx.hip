@@ -907,23 +907,85 @@ int mdft_compute_vext_ex(mdft_ctx *c, int natom, const double *atoms, int nsite,
         sp[3 * s + 2] = sites[6 * s + 5];
     }
     for (int i = 0; i < natom * 6; i++) at[i] = atoms[i];
-    double *d_off = nullptr, *d_sp = nullptr, *d_at = nullptr;
-    HIPCHK(c, upload(c, &d_off, off.data(), off.size()));
-    HIPCHK(c, upload(c, &d_sp, sp.data(), sp.size()));
-    HIPCHK(c, upload(c, &d_at, at.data(), at.size()));
-    // the clip at qfact/2 (src/module_vext.f90:638-640) follows the sum of all terms
     const bool direct = electrostatics == MDFT_ELEC_DIRECT, poisson = electrostatics == MDFT_ELEC_POISSON;
-    hipError_t e = launch_vext(c, natom, d_at, nsite, d_sp, d_off, rcut, qfact, poisson ? HUGE_VAL : qfact / 2.0, direct);
+    // sites with a potential, and the distinct places where each stands over the orientations
+    std::vector<int> live, col((size_t)c->no * nsite, -1), col_site;
+    std::vector<double> col_pos;
+    for (int s = 0; s < nsite; s++) {
+        bool any = false;
+        for (int i = 0; i < natom; i++)
+            any = any || sites[6 * s + 5] * at[6 * i + 5] > 0.0 || (direct && sites[6 * s + 3] * at[6 * i + 3] != 0.0);
+        if (!any) continue;
+        std::map<std::tuple<double, double, double>, int> place;
+        std::vector<int> at_place(c->no);
+        for (int io = 0; io < c->no; io++) {
+            const double *o = &off[((size_t)io * nsite + s) * 3];
+            at_place[io] = place.emplace(std::make_tuple(o[0] + 0.0, o[1] + 0.0, o[2] + 0.0), (int)place.size()).first->second;
+        }
+        // a place costs a column of N values and its sum over the atoms; from four orientations per
+        // place on that is less than the sum for each orientation
+        if (place.size() > 1 && 4 * place.size() > (size_t)c->no) {
+            live.push_back(s);
+            continue;
+        }
+        const int c0 = (int)col_site.size();
+        col_site.resize(c0 + place.size(), s);
+        col_pos.resize(3 * col_site.size());
+        for (auto &p : place) {
+            col_pos[3 * (c0 + p.second)] = std::get<0>(p.first);
+            col_pos[3 * (c0 + p.second) + 1] = std::get<1>(p.first);
+            col_pos[3 * (c0 + p.second) + 2] = std::get<2>(p.first);
+        }
+        for (int io = 0; io < c->no; io++) col[(size_t)io * nsite + s] = c0 + at_place[io];
+    }
+    // (the place table of the sites that have any)
+    std::vector<int> placed, pcol;
+    for (int s = 0; s < nsite; s++)
+        if (col[s] >= 0) placed.push_back(s);
+    for (int io = 0; io < c->no; io++)
+        for (int s : placed) pcol.push_back(col[(size_t)io * nsite + s]);
+    VextPlaces pl{(int)col_site.size(), (int)placed.size(), nullptr, nullptr};
+    double *d_off = nullptr, *d_sp = nullptr, *d_at = nullptr, *d_S = nullptr, *d_cpos = nullptr;
+    int *d_col = nullptr, *d_csite = nullptr, *d_live = nullptr;
+    if (pl.ncols > 0 && hipMalloc((void **)&d_S, sizeof(double) * c->N * pl.ncols) != hipSuccess) {
+        // no room for the places: their sites are summed per orientation
+        (void)hipGetLastError();
+        d_S = nullptr;
+        live.insert(live.end(), placed.begin(), placed.end());
+        pl.ncols = pl.nsite = 0;
+    }
+    hipError_t e = upload(c, &d_off, off.data(), off.size());
+    if (e == hipSuccess) e = upload(c, &d_sp, sp.data(), sp.size());
+    if (e == hipSuccess) e = upload(c, &d_at, at.data(), at.size());
+    if (e == hipSuccess && !live.empty()) e = upload(c, &d_live, live.data(), live.size());
+    if (e == hipSuccess && pl.ncols > 0) {
+        e = upload(c, &d_col, pcol.data(), pcol.size());
+        if (e == hipSuccess) e = upload(c, &d_cpos, col_pos.data(), col_pos.size());
+        if (e == hipSuccess) e = upload(c, &d_csite, col_site.data(), col_site.size());
+        if (e == hipSuccess)
+            e = launch_site_potential(c, natom, d_at, nsite, d_sp, rcut, qfact, direct, pl.ncols, d_cpos, d_csite, d_S);
+        pl.S = d_S;
+        pl.col = d_col;
+    }
+    // the clip at qfact/2 (src/module_vext.f90:638-640) follows the sum of all terms.  Where every site
+    // stands at few places, the Poisson path adds them as it writes vext
+    const double clip = qfact / 2.0;
+    if (e == hipSuccess && !live.empty())
+        e = launch_vext(c, natom, d_at, nsite, d_sp, d_off, rcut, qfact, poisson ? HUGE_VAL : clip, direct, pl,
+                        (int)live.size(), d_live);
+    bool done = false;
     if (e == hipSuccess && poisson) {
         std::vector<double> sq(nsite);
         for (int s = 0; s < nsite; s++) sq[s] = sites[6 * s + 3];
-        e = launch_poisson_vext(c, natom, at.data(), nsite, sq.data(), d_off, qfact);
-        if (e == hipSuccess) e = launch_vext_clip(c, qfact / 2.0);
+        VextPlaces base = pl;
+        if (!live.empty()) base.ncols = -1;
+        e = launch_poisson_vext(c, natom, at.data(), nsite, sq.data(), off.data(), d_off, qfact, base, clip, &done);
+        if (e == hipSuccess && !done && !live.empty()) e = launch_vext_clip(c, clip);
     }
+    if (e == hipSuccess && live.empty() && !done) e = launch_vext_from_places(c, pl, clip);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    (void)hipFree(d_off);
-    (void)hipFree(d_sp);
-    (void)hipFree(d_at);
+    void *tmp[] = {d_off, d_sp, d_at, d_S, d_cpos, d_col, d_csite, d_live};
+    for (void *p : tmp) (void)hipFree(p);
     HIPCHK(c, e);
     c->have_vext = true;
     c->vext32_ok = false;

@@ -201,8 +201,21 @@ hipError_t vec_combine_step32x(mdft_ctx *c, size_t n, int k, const double *coef,
 hipError_t vec_axpy32x(mdft_ctx *c, size_t n, double a, const float *z, const float *x, float *y);
 hipError_t vec_narrow(mdft_ctx *c, size_t n, const double *in, float *out);
 hipError_t vec_scale_orient(mdft_ctx *c, size_t n, int no, const double *fac, const void *in, bool in_f32, double *out);
+// Potentials of nsite solvent sites at the few places where each stands: S [N][ncols], and the
+// column of each (orientation, site).
+struct VextPlaces {
+    int ncols, nsite;
+    const double *S;
+    const int *col;  // [no][nsite]
+};
+hipError_t launch_site_potential(mdft_ctx *c, int natom, const double *d_atoms, int nsite, const double *d_site_p,
+                                 double rcut, double qfact, bool coulomb, int ncols, const double *d_col_pos,
+                                 const int *d_col_site, double *S);
+hipError_t launch_vext_from_places(mdft_ctx *c, const VextPlaces &b, double clip);
 hipError_t launch_vext(mdft_ctx *c, int natom, const double *d_atoms, int nsite, const double *d_site_p,
-                       const double *d_site_off, double rcut, double qfact, double clip, bool coulomb = true);
+                       const double *d_site_off, double rcut, double qfact, double clip, bool coulomb,
+                       const VextPlaces &b, int nlive, const int *d_sites);
 hipError_t launch_poisson_vext(mdft_ctx *c, int natom, const double *h_atoms, int nsite, const double *h_site_q,
-                               const double *d_site_off, double qfact);
+                               const double *h_site_off, const double *d_site_off, double qfact,
+                               const VextPlaces &places, double clip, bool *done);
 hipError_t launch_vext_clip(mdft_ctx *c, double clip);

@@ -263,7 +263,9 @@ int mdft_regrid_trilinear(mdft_ctx *ctx, const double *d_prev, const int *n_prev
                           double outside, double *d_xi);
 
 /* Device memory owned by the caller, for device-resident fields
- * (MDFT_DEVICE_PTRS) and the device L-BFGS vectors. */
+ * (MDFT_DEVICE_PTRS) and the device L-BFGS vectors.  Freeing waits for the device; freed
+ * memory is kept for the next allocation of its size, at most 2 GiB per device, until the
+ * device's last context is destroyed. */
 int mdft_device_alloc(mdft_ctx *ctx, size_t bytes, void **dptr);
 int mdft_device_free(mdft_ctx *ctx, void *dptr);
 int mdft_memcpy_h2d(mdft_ctx *ctx, void *dst, const void *src, size_t bytes);

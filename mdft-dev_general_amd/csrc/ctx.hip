@@ -118,22 +118,22 @@ int mq(int i, int n) { return i == 0 ? 0 : n - i; }  // module_grid.f90:384-418
 
 template <typename T>
 hipError_t upload(mdft_ctx *c, T **dst, const T *src, size_t n) {
-    hipError_t e = hipMalloc((void **)dst, sizeof(T) * (n ? n : 1));
+    hipError_t e = dev_malloc(dst, sizeof(T) * (n ? n : 1));
     if (e != hipSuccess) return e;
     if (n) e = hipMemcpy(*dst, src, sizeof(T) * n, hipMemcpyHostToDevice);
     return e;
 }
 
 void free_pairs(PairSchedule &p) {
-    (void)hipFree(p.pq);
-    (void)hipFree(p.pmq);
-    (void)hipFree(p.pflag);
-    (void)hipFree(p.cstart);
-    (void)hipFree(p.ccount);
-    (void)hipFree(p.ciq);
-    (void)hipFree(p.tstart);
-    (void)hipFree(p.tinfo);
-    (void)hipFree(p.tpair);
+    (void)dev_free(p.pq);
+    (void)dev_free(p.pmq);
+    (void)dev_free(p.pflag);
+    (void)dev_free(p.cstart);
+    (void)dev_free(p.ccount);
+    (void)dev_free(p.ciq);
+    (void)dev_free(p.tstart);
+    (void)dev_free(p.tinfo);
+    (void)dev_free(p.tpair);
     p = PairSchedule{};
 }
 
@@ -262,7 +262,7 @@ hipError_t launch_final(mdft_ctx *c, const double *xi, double *df, int mode, int
 
 hipError_t ensure_stage(mdft_ctx *c, double **buf) {
     if (*buf) return hipSuccess;
-    return hipMalloc((void **)buf, sizeof(double) * c->N * c->no);
+    return dev_malloc(buf, sizeof(double) * c->N * c->no);
 }
 
 // Runs the excess-term projection pipeline up to `stage` (1..4) on device xi.
@@ -354,6 +354,7 @@ int mdft_ctx_create(const mdft_desc *desc, mdft_ctx **out) {
     }
     mdft_ctx *c = new mdft_ctx();
     c->d = d;
+    dev_context(d.device, +1);
     c->L = d.mmax;
     c->H = d.mmax / d.mrso;
     c->ntheta = d.mmax + 1;
@@ -469,9 +470,9 @@ int mdft_ctx_create(const mdft_desc *desc, mdft_ctx **out) {
               upload(c, &c->d_ky, c->ky.data(), c->ky.size()) == hipSuccess &&
               upload(c, &c->d_kz, c->kz.data(), c->kz.size()) == hipSuccess;
     c->ia0_h = ia0;
-    ok = ok && hipMalloc(&c->d_proj, proj_elem_bytes(c) * c->N * np) == hipSuccess;
-    ok = ok && hipMalloc(&c->d_vext, sizeof(double) * c->N * c->no) == hipSuccess;
-    ok = ok && hipMalloc(&c->d_sums, sizeof(double) * 8) == hipSuccess;
+    ok = ok && dev_malloc(&c->d_proj, proj_elem_bytes(c) * c->N * np) == hipSuccess;
+    ok = ok && dev_malloc(&c->d_vext, sizeof(double) * c->N * c->no) == hipSuccess;
+    ok = ok && dev_malloc(&c->d_sums, sizeof(double) * 8) == hipSuccess;
     ok = ok && hipHostMalloc(&c->h_sums, sizeof(double) * 8, hipHostMallocDefault) == hipSuccess;
     if (!ok) return bad(MDFT_ENOMEM, "device allocation failed");
     if (d.precision == MDFT_PREC_BF16) {
@@ -519,7 +520,7 @@ int mdft_ctx_create(const mdft_desc *desc, mdft_ctx **out) {
 void mdft_ctx_destroy(mdft_ctx *c) {
     if (!c) return;
     if (c->stream) (void)hipStreamSynchronize(c->stream);
-    for (auto &f : c->fft) (void)hipFree(f.tw);
+    for (auto &f : c->fft) (void)dev_free(f.tw);
     void *bufs[] = {c->d_w,   c->d_a2p,  c->d_p2a,  c->d_fm,   c->d_cph,      c->d_sph,        c->d_cps,
                     c->d_sps, c->d_pidx, c->d_pm,   c->d_pmup, c->d_pmu,      c->d_ia0,        c->d_kx,
                     c->d_ky,  c->d_kz,   c->d_ck,   c->d_vext, c->d_proj,     c->d_xi_stage,   c->d_df_stage,
@@ -528,12 +529,13 @@ void mdft_ctx_destroy(mdft_ctx *c) {
                     c->d_bf16_M, c->d_bf16_Q, c->d_chscale, c->d_adjscale, c->d_vscale, c->d_dpart, c->d_vext32,
                     c->d_a2p_img[0], c->d_a2p_img[1], c->d_a2p_img[2], c->d_a2p_img[3], c->d_ozm_pack};
     for (void *b : bufs)
-        if (b) (void)hipFree(b);
+        if (b) (void)dev_free(b);
     free_pairs(c->pairs);
     if (c->h_sums) (void)hipHostFree(c->h_sums);
     if (c->timers_ready)
         for (auto &e : c->ev) (void)hipEventDestroy(e);
     if (c->stream) (void)hipStreamDestroy(c->stream);
+    dev_context(c->d.device, -1);
     delete c;
 }
 
@@ -619,7 +621,7 @@ int mdft_set_ck(mdft_ctx *c, int np_file, const int *m, const int *n, const int 
             // conj (cproj_mrso.f90:415) then the sign folding (:420-429)
             tab[(size_t)iq * npc + ia] = make_double2(sgn[ia] * v[0], sgn[ia] * -v[1]);
         }
-    if (c->d_ck) (void)hipFree(c->d_ck);
+    if (c->d_ck) (void)dev_free(c->d_ck);
     c->d_ck = nullptr;
     HIPCHK(c, upload(c, &c->d_ck, tab.data(), tab.size()));
     {
@@ -681,7 +683,7 @@ static int ensure_vscale(mdft_ctx *c) {
         h[io] = sqrt(c->w[io] / wm);
         h[no + io] = 1.0 / h[io];
     }
-    HIPCHK(c, hipMalloc(&c->d_vscale, sizeof(double) * h.size()));
+    HIPCHK(c, dev_malloc(&c->d_vscale, sizeof(double) * h.size()));
     HIPCHK(c, hipMemcpy(c->d_vscale, h.data(), sizeof(double) * h.size(), hipMemcpyHostToDevice));
     return MDFT_OK;
 }
@@ -718,10 +720,10 @@ static int evaluate(mdft_ctx *c, const double *xi, double *df, int flags, int mo
                                         "molecular symmetry order 2 and an FP64 or FP32 context");
         const size_t need = 3 * ((c->N + 3) / 4);
         if (c->dpart_cap < need) {
-            if (c->d_dpart) HIPCHK(c, hipFree(c->d_dpart));
+            if (c->d_dpart) HIPCHK(c, dev_free(c->d_dpart));
             c->d_dpart = nullptr;
             c->dpart_cap = 0;
-            HIPCHK(c, hipMalloc(&c->d_dpart, sizeof(double) * need));
+            HIPCHK(c, dev_malloc(&c->d_dpart, sizeof(double) * need));
             c->dpart_cap = need;
         }
         c->dot_self = 0;
@@ -749,7 +751,7 @@ static int evaluate(mdft_ctx *c, const double *xi, double *df, int flags, int mo
     if (x32 && df32 && dot_k > 0 && c->d.precision == MDFT_PREC_FP32 && !c->vext32_ok) {
         // the fast minimiser's final pass reads vext in FP32 (its FP32 terms round vext to FP32
         // first, so the copy changes no result): made once per vext
-        if (!c->d_vext32) HIPCHK(c, hipMalloc(&c->d_vext32, sizeof(float) * c->N * c->no));
+        if (!c->d_vext32) HIPCHK(c, dev_malloc(&c->d_vext32, sizeof(float) * c->N * c->no));
         HIPCHK(c, vec_narrow(c, c->N * c->no, c->d_vext, c->d_vext32));
         c->vext32_ok = true;
     }
@@ -947,7 +949,7 @@ int mdft_compute_vext_ex(mdft_ctx *c, int natom, const double *atoms, int nsite,
     VextPlaces pl{(int)col_site.size(), (int)placed.size(), nullptr, nullptr};
     double *d_off = nullptr, *d_sp = nullptr, *d_at = nullptr, *d_S = nullptr, *d_cpos = nullptr;
     int *d_col = nullptr, *d_csite = nullptr, *d_live = nullptr;
-    if (pl.ncols > 0 && hipMalloc((void **)&d_S, sizeof(double) * c->N * pl.ncols) != hipSuccess) {
+    if (pl.ncols > 0 && dev_malloc(&d_S, sizeof(double) * c->N * pl.ncols) != hipSuccess) {
         // no room for the places: their sites are summed per orientation
         (void)hipGetLastError();
         d_S = nullptr;
@@ -985,7 +987,7 @@ int mdft_compute_vext_ex(mdft_ctx *c, int natom, const double *atoms, int nsite,
     if (e == hipSuccess && live.empty() && !done) e = launch_vext_from_places(c, pl, clip);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     void *tmp[] = {d_off, d_sp, d_at, d_S, d_cpos, d_col, d_csite, d_live};
-    for (void *p : tmp) (void)hipFree(p);
+    for (void *p : tmp) (void)dev_free(p, e == hipSuccess);
     HIPCHK(c, e);
     c->have_vext = true;
     c->vext32_ok = false;
@@ -1159,12 +1161,12 @@ int mdft_pressure_correction(mdft_ctx *c, const double *xi, int flags, double *o
     const double dN = n_without - n_with;
     // bulk grand potential: the functional of the empty box, xi = 0 (:115-119)
     double *zero = nullptr;
-    HIPCHK(c, hipMalloc(&zero, nbytes));
+    HIPCHK(c, dev_malloc(&zero, nbytes));
     hipError_t e = hipMemsetAsync(zero, 0, nbytes, c->stream);
     double sums[3] = {0.0, 0.0, 0.0};
     if (e == hipSuccess) rc = evaluate(c, zero, nullptr, MDFT_DEVICE_PTRS, 0, sums);
     (void)hipStreamSynchronize(c->stream);
-    (void)hipFree(zero);
+    (void)dev_free(zero);
     if (e != hipSuccess) return fail(c, MDFT_EHIP, std::string("hipMemsetAsync: ") + hipGetErrorString(e));
     if (rc) return rc;
     const double f_empty = sums[0] + sums[1] + sums[2];
@@ -1237,13 +1239,13 @@ int mdft_phase_times(const mdft_ctx *c, double *ms, int n) {
 
 int mdft_device_alloc(mdft_ctx *c, size_t bytes, void **dptr) {
     if (!c || !dptr) return MDFT_EINVAL;
-    HIPCHK(c, hipMalloc(dptr, bytes ? bytes : 1));
+    HIPCHK(c, dev_malloc(dptr, bytes ? bytes : 1));
     return MDFT_OK;
 }
 
 int mdft_device_free(mdft_ctx *c, void *dptr) {
     if (!c) return MDFT_EINVAL;
-    if (dptr) HIPCHK(c, hipFree(dptr));
+    if (dptr) HIPCHK(c, dev_free(dptr));
     return MDFT_OK;
 }
 
@@ -1275,7 +1277,7 @@ int mdft_ws_features(mdft_ctx *c, float *d_feat, const float *h_scale) {
     if (c->d.mrso != 2) return fail(c, MDFT_EINVAL, "the warm start needs molecular symmetry order 2");
     if (h_scale) {
         const size_t bytes = sizeof(float) * 2 * c->np;
-        if (!c->d_chscale) HIPCHK(c, hipMalloc(&c->d_chscale, bytes));
+        if (!c->d_chscale) HIPCHK(c, dev_malloc(&c->d_chscale, bytes));
         HIPCHK(c, hipMemcpyAsync(c->d_chscale, h_scale, bytes, hipMemcpyHostToDevice, c->stream));
     }
     HIPCHK(c, launch_angl2proj_feat(c, c->d_vext, 1));
@@ -1349,7 +1351,7 @@ int mdft_ws_start_gradient(mdft_ctx *c, const double *d_xi, const double *d_df, 
                     h[2 * ip + 1] = (mup == 0 && mu == 0) ? 0.0f : (float)f;
                 }
         if (ip != (size_t)c->np) return fail(c, MDFT_EINVAL, "projection count mismatch");
-        HIPCHK(c, hipMalloc(&c->d_adjscale, sizeof(float) * h.size()));
+        HIPCHK(c, dev_malloc(&c->d_adjscale, sizeof(float) * h.size()));
         HIPCHK(c, hipMemcpy(c->d_adjscale, h.data(), sizeof(float) * h.size(), hipMemcpyHostToDevice));
     }
     HIPCHK(c, launch_angl2proj_feat(c, d_xi, 3, d_df));
@@ -1411,14 +1413,14 @@ int mdft_regrid_trilinear(mdft_ctx *c, const double *d_prev, const int *n_prev, 
     }
     int *d_cell = nullptr;
     double *d_wgt = nullptr;
-    HIPCHK(c, hipMalloc(&d_cell, sizeof(int) * cell.size()));
-    hipError_t e = hipMalloc(&d_wgt, sizeof(double) * wgt.size());
+    HIPCHK(c, dev_malloc(&d_cell, sizeof(int) * cell.size()));
+    hipError_t e = dev_malloc(&d_wgt, sizeof(double) * wgt.size());
     if (e == hipSuccess) e = hipMemcpy(d_cell, cell.data(), sizeof(int) * cell.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(d_wgt, wgt.data(), sizeof(double) * wgt.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = launch_regrid(c, d_prev, n_prev[0], n_prev[1], d_cell, d_wgt, outside, d_xi);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    (void)hipFree(d_cell);
-    (void)hipFree(d_wgt);
+    (void)dev_free(d_cell);
+    (void)dev_free(d_wgt);
     if (e != hipSuccess) return fail(c, MDFT_EHIP, std::string("regrid: ") + hipGetErrorString(e));
     return MDFT_OK;
 }

@@ -1,0 +1,93 @@
+// devmem.hip -- device memory of short-lived vectors and tables.
+//
+// A solve allocates its vectors and a potential its tables and fields anew on every call;
+// hipMalloc and hipFree of a few hundred MB take 0.1 to several ms each, more than the small
+// solves' kernels.  Freed blocks are therefore kept for the next allocation of their size, at
+// most kKeep bytes per device, the oldest given back first; all are given back when the last
+// context of the device is destroyed, and when any allocation here fails.  A block is kept only
+// after the device has finished all work (as hipFree does; or its caller has waited for all that
+// used it), so its next owner may use it on any stream; the list is locked, so contexts in several threads share it.
+#include <list>
+#include <mutex>
+#include <unordered_map>
+
+#include "mdft_internal.h"
+
+namespace {
+
+constexpr size_t kKeep = (size_t)2 << 30;
+
+struct Block {
+    void *p;
+    size_t bytes;
+    int device;
+};
+// (never destroyed: a context may be destroyed while the program ends)
+std::mutex &lock = *new std::mutex;
+std::unordered_map<void *, Block> &live = *new std::unordered_map<void *, Block>;  // allocated through dev_malloc
+std::list<Block> &idle = *new std::list<Block>;                                    // oldest first
+std::unordered_map<int, int> &users = *new std::unordered_map<int, int>;           // contexts per device
+
+// gives back idle blocks of a device, oldest first, until at most `keep` bytes of it are idle
+void trim(int device, size_t keep) {
+    size_t n = 0;
+    for (const Block &b : idle)
+        if (b.device == device) n += b.bytes;
+    for (auto it = idle.begin(); it != idle.end() && n > keep;) {
+        if (it->device != device) {
+            ++it;
+            continue;
+        }
+        n -= it->bytes;
+        (void)hipFree(it->p);
+        it = idle.erase(it);
+    }
+}
+
+}  // namespace
+
+hipError_t dev_malloc_bytes(void **p, size_t bytes) {
+    *p = nullptr;
+    if (bytes == 0) bytes = 1;
+    int device = 0;
+    hipError_t e = hipGetDevice(&device);
+    if (e != hipSuccess) return e;
+    const std::lock_guard<std::mutex> hold(lock);
+    for (auto it = idle.begin(); it != idle.end(); ++it)
+        if (it->device == device && it->bytes == bytes) {
+            *p = it->p;
+            live[it->p] = *it;
+            idle.erase(it);
+            return hipSuccess;
+        }
+    e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        trim(device, 0);
+        e = hipMalloc(p, bytes);
+    }
+    if (e == hipSuccess) live[*p] = Block{*p, bytes, device};
+    else *p = nullptr;
+    return e;
+}
+
+hipError_t dev_free(void *p, bool synced) {
+    if (!p) return hipSuccess;
+    const std::lock_guard<std::mutex> hold(lock);
+    const auto it = live.find(p);
+    if (it == live.end()) return hipFree(p);  // not from dev_malloc
+    const Block b = it->second;
+    live.erase(it);
+    int device = 0;
+    if (b.bytes > kKeep || hipGetDevice(&device) != hipSuccess || device != b.device || !users[b.device] ||
+        (!synced && hipDeviceSynchronize() != hipSuccess))
+        return hipFree(p);
+    trim(device, kKeep - b.bytes);
+    idle.push_back(b);
+    return hipSuccess;
+}
+
+void dev_context(int device, int change) {
+    const std::lock_guard<std::mutex> hold(lock);
+    if ((users[device] += change) <= 0) trim(device, 0);
+}

@@ -1067,9 +1067,9 @@ size_t final_lds(const AngTables &t) {
 
 hipError_t ensure_partials(mdft_ctx *c, size_t nblocks) {
     if (c->partials_cap >= nblocks * 3) return hipSuccess;
-    if (c->d_partials) (void)hipFree(c->d_partials);
+    if (c->d_partials) (void)dev_free(c->d_partials);
     c->d_partials = nullptr;
-    hipError_t e = hipMalloc(&c->d_partials, sizeof(double) * nblocks * 3);
+    hipError_t e = dev_malloc(&c->d_partials, sizeof(double) * nblocks * 3);
     if (e == hipSuccess) c->partials_cap = nblocks * 3;
     return e;
 }
@@ -1097,7 +1097,7 @@ bool launch_a2p_t(mdft_ctx *c, const double *xi, typename C2<T>::t *proj, int fe
     case LL: { \
         using S = A2pShape<LL>; \
         if (!img) { \
-            if (hipMalloc(&img, sizeof(OutLane<LL, T>) * Rows<LL>::NP) != hipSuccess) { img = nullptr; return false; } \
+            if (dev_malloc(&img, sizeof(OutLane<LL, T>) * Rows<LL>::NP) != hipSuccess) { img = nullptr; return false; } \
             hipLaunchKernelGGL((out_lanes_build<LL, T, PACK>), dim3(1), dim3(128), 0, c->stream, static_cast<OutLane<LL, T> *>(img), c->ang); \
         } \
         hipLaunchKernelGGL((angl2proj_t<LL, S::PT, S::TH, T, PACK>), dim3((unsigned)((npts + S::PT - 1) / S::PT)), dim3(S::TH), 0, c->stream, xi, proj, npts, c->ang, k0, feat, beta, aux, feat == 0 ? c->vsinv : nullptr, feat == 0 ? c->xi32 : nullptr, static_cast<const OutLane<LL, T> *>(img)); \
@@ -1210,7 +1210,7 @@ hipError_t launch_reduce3_buf(mdft_ctx *c, const double *part, int nblocks, doub
         return hipGetLastError();
     }
     if (!c->d_slices) {
-        hipError_t e = hipMalloc(&c->d_slices, sizeof(double) * 3 * kSlices);
+        hipError_t e = dev_malloc(&c->d_slices, sizeof(double) * 3 * kSlices);
         if (e != hipSuccess) return e;
     }
     hipLaunchKernelGGL(reduce3, dim3(kSlices), dim3(kThreads), 0, c->stream, part, nblocks, c->d_slices);

@@ -258,8 +258,8 @@ int bf16_tables(mdft_ctx *c, const std::vector<double> &a2p, const std::vector<d
             }
     (void)H1;
     std::vector<__bf16> Mf = to_fragments(M, no, 2 * np), Qf = to_fragments(Q, 2 * np, no);
-    if (hipMalloc(&c->d_bf16_M, Mf.size() * sizeof(__bf16)) != hipSuccess ||
-        hipMalloc(&c->d_bf16_Q, Qf.size() * sizeof(__bf16)) != hipSuccess)
+    if (dev_malloc(&c->d_bf16_M, Mf.size() * sizeof(__bf16)) != hipSuccess ||
+        dev_malloc(&c->d_bf16_Q, Qf.size() * sizeof(__bf16)) != hipSuccess)
         return MDFT_ENOMEM;
     if (hipMemcpy(c->d_bf16_M, Mf.data(), Mf.size() * sizeof(__bf16), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(c->d_bf16_Q, Qf.data(), Qf.size() * sizeof(__bf16), hipMemcpyHostToDevice) != hipSuccess)
@@ -285,10 +285,10 @@ hipError_t launch_final_bf16(mdft_ctx *c, const float2 *proj, const double *xi, 
                              int *nblocks_out) {
     const int nb = blocks_for(c);
     if (c->partials_cap < (size_t)nb * 3) {
-        (void)hipFree(c->d_partials);
+        (void)dev_free(c->d_partials);
         c->d_partials = nullptr;
         c->partials_cap = 0;
-        hipError_t e = hipMalloc(&c->d_partials, sizeof(double) * 3 * nb);
+        hipError_t e = dev_malloc(&c->d_partials, sizeof(double) * 3 * nb);
         if (e != hipSuccess) return e;
         c->partials_cap = 3 * (size_t)nb;
     }

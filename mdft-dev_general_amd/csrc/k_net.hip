@@ -388,10 +388,10 @@ int ws_fail(mdft_wsnet *n, int code, const std::string &msg) {
     } while (0)
 
 void free_acts(mdft_wsnet *n) {
-    for (float *p : n->act) (void)hipFree(p);
+    for (float *p : n->act) (void)dev_free(p);
     n->act.clear();
-    (void)hipFree(n->gA);
-    (void)hipFree(n->gB);
+    (void)dev_free(n->gA);
+    (void)dev_free(n->gB);
     n->gA = n->gB = nullptr;
     n->nx = n->ny = n->nz = 0;
 }
@@ -405,9 +405,9 @@ int ensure_grid(mdft_wsnet *n, int nx, int ny, int nz) {
     int cmax = 0;
     for (int c : n->ch) cmax = std::max(cmax, c);
     n->act.assign(n->nl + 1, nullptr);
-    for (int l = 1; l <= n->nl; l++) WSCHK(n, hipMalloc(&n->act[l], sizeof(float) * N * n->ch[l]));
-    WSCHK(n, hipMalloc(&n->gA, sizeof(float) * N * cmax));
-    WSCHK(n, hipMalloc(&n->gB, sizeof(float) * N * cmax));
+    for (int l = 1; l <= n->nl; l++) WSCHK(n, dev_malloc(&n->act[l], sizeof(float) * N * n->ch[l]));
+    WSCHK(n, dev_malloc(&n->gA, sizeof(float) * N * cmax));
+    WSCHK(n, dev_malloc(&n->gB, sizeof(float) * N * cmax));
     n->nx = nx;
     n->ny = ny;
     n->nz = nz;
@@ -469,9 +469,9 @@ int backward(mdft_wsnet *n, const float *d_in, float *d_gin) {
     for (int l = 0; l < L; l++)
         need = std::max(need, (size_t)nblk * ((size_t)n->ch[l + 1] * n->ch[l] * n->taps[l] + n->ch[l + 1]));
     if (need > n->part_cap) {
-        (void)hipFree(n->part);
+        (void)dev_free(n->part);
         n->part = nullptr;
-        WSCHK(n, hipMalloc(&n->part, sizeof(float) * need));
+        WSCHK(n, dev_malloc(&n->part, sizeof(float) * need));
         n->part_cap = need;
     }
     float *gcur = n->gA, *gnext = n->gB;
@@ -576,11 +576,11 @@ int mdft_wsnet_create(int nlayers, const int *channels, const int *ksize, const 
         }
     }
     bool ok = hipStreamCreate(&n->stream) == hipSuccess;
-    ok = ok && hipMalloc(&n->params, sizeof(float) * off) == hipSuccess;
-    ok = ok && hipMalloc(&n->grads, sizeof(float) * off) == hipSuccess;
-    ok = ok && hipMalloc(&n->m1, sizeof(float) * off) == hipSuccess;
-    ok = ok && hipMalloc(&n->m2, sizeof(float) * off) == hipSuccess;
-    ok = ok && hipMalloc(&n->dpart, sizeof(double) * 4096) == hipSuccess;
+    ok = ok && dev_malloc(&n->params, sizeof(float) * off) == hipSuccess;
+    ok = ok && dev_malloc(&n->grads, sizeof(float) * off) == hipSuccess;
+    ok = ok && dev_malloc(&n->m1, sizeof(float) * off) == hipSuccess;
+    ok = ok && dev_malloc(&n->m2, sizeof(float) * off) == hipSuccess;
+    ok = ok && dev_malloc(&n->dpart, sizeof(double) * 4096) == hipSuccess;
     ok = ok && hipHostMalloc(&n->hpart, sizeof(double) * 4096, hipHostMallocDefault) == hipSuccess;
     ok = ok && hipMemcpy(n->params, h.data(), sizeof(float) * off, hipMemcpyHostToDevice) == hipSuccess;
     ok = ok && hipMemset(n->grads, 0, sizeof(float) * off) == hipSuccess;
@@ -599,12 +599,12 @@ void mdft_wsnet_destroy(mdft_wsnet *n) {
     if (!n) return;
     if (n->stream) (void)hipStreamSynchronize(n->stream);
     free_acts(n);
-    (void)hipFree(n->params);
-    (void)hipFree(n->grads);
-    (void)hipFree(n->m1);
-    (void)hipFree(n->m2);
-    (void)hipFree(n->part);
-    (void)hipFree(n->dpart);
+    (void)dev_free(n->params);
+    (void)dev_free(n->grads);
+    (void)dev_free(n->m1);
+    (void)dev_free(n->m2);
+    (void)dev_free(n->part);
+    (void)dev_free(n->dpart);
     if (n->hpart) (void)hipHostFree(n->hpart);
     if (n->stream) (void)hipStreamDestroy(n->stream);
     delete n;

@@ -856,9 +856,9 @@ template <typename T, bool BF> hipError_t launch_ozm_any(mdft_ctx *c, typename T
 
 template <typename T> int upload_t(mdft_ctx *c, void **dst, const std::vector<double> &src) {
     std::vector<T> v(src.begin(), src.end());
-    if (*dst) (void)hipFree(*dst);
+    if (*dst) (void)dev_free(*dst);
     *dst = nullptr;
-    if (hipMalloc(dst, sizeof(T) * (v.size() ? v.size() : 1)) != hipSuccess) return MDFT_ENOMEM;
+    if (dev_malloc(dst, sizeof(T) * (v.size() ? v.size() : 1)) != hipSuccess) return MDFT_ENOMEM;
     if (!v.empty() && hipMemcpy(*dst, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice) != hipSuccess)
         return MDFT_EHIP;
     return MDFT_OK;
@@ -991,8 +991,8 @@ int ozm_setup(mdft_ctx *c) {
     int rc = c->d.precision == MDFT_PREC_FP64 ? upload_t<double>(c, &c->d_ozm_ftab, ftab)
                                                 : upload_t<float>(c, &c->d_ozm_ftab, ftab);
     if (rc != MDFT_OK) return rc;
-    if (hipMalloc((void **)&c->d_ozm_units, sizeof(int) * units.size()) != hipSuccess ||
-        hipMalloc((void **)&c->d_ozm_rlen, sizeof(int) * rlen.size()) != hipSuccess)
+    if (dev_malloc(&c->d_ozm_units, sizeof(int) * units.size()) != hipSuccess ||
+        dev_malloc(&c->d_ozm_rlen, sizeof(int) * rlen.size()) != hipSuccess)
         return MDFT_ENOMEM;
     if (hipMemcpy(c->d_ozm_units, units.data(), sizeof(int) * units.size(), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(c->d_ozm_rlen, rlen.data(), sizeof(int) * rlen.size(), hipMemcpyHostToDevice) != hipSuccess)
@@ -1008,7 +1008,7 @@ int ozm_setup(mdft_ctx *c) {
             for (int mup = -L; mup <= L; mup++) item(mup, mu2);
         for (int m = 0; m <= L; m += 2)
             pk.push_back(pidx(m, 0, 0) | (m < L ? pidx(m + 1, 0, 0) : 255) << 8 | 2 << 16 | 16 << 20);
-        if (hipMalloc((void **)&c->d_ozm_pack, sizeof(int) * pk.size()) != hipSuccess) return MDFT_ENOMEM;
+        if (dev_malloc(&c->d_ozm_pack, sizeof(int) * pk.size()) != hipSuccess) return MDFT_ENOMEM;
         if (hipMemcpy(c->d_ozm_pack, pk.data(), sizeof(int) * pk.size(), hipMemcpyHostToDevice) != hipSuccess)
             return MDFT_EHIP;
     }
@@ -1016,7 +1016,7 @@ int ozm_setup(mdft_ctx *c) {
     std::vector<int> colent;
     for (int khi = -L; khi <= L; khi++)
         for (int cc = 0; cc < 32; cc++) colent.push_back(cc < h.ncol[khi + L] ? h.col[khi + L][cc] : 1);
-    if (hipMalloc((void **)&c->d_ozm_col, sizeof(int) * colent.size()) != hipSuccess) return MDFT_ENOMEM;
+    if (dev_malloc(&c->d_ozm_col, sizeof(int) * colent.size()) != hipSuccess) return MDFT_ENOMEM;
     if (hipMemcpy(c->d_ozm_col, colent.data(), sizeof(int) * colent.size(), hipMemcpyHostToDevice) != hipSuccess)
         return MDFT_EHIP;
     return MDFT_OK;
@@ -1075,9 +1075,9 @@ int ozm_frags(mdft_ctx *c, const std::vector<double2> &tab, int nq, int npc, con
                         }
                 }
         }
-    if (c->d_ozm_frag16) (void)hipFree(c->d_ozm_frag16);
+    if (c->d_ozm_frag16) (void)dev_free(c->d_ozm_frag16);
     c->d_ozm_frag16 = nullptr;
-    if (hipMalloc(&c->d_ozm_frag16, sizeof(__bf16) * f16.size()) != hipSuccess) return MDFT_ENOMEM;
+    if (dev_malloc(&c->d_ozm_frag16, sizeof(__bf16) * f16.size()) != hipSuccess) return MDFT_ENOMEM;
     if (hipMemcpy(c->d_ozm_frag16, f16.data(), sizeof(__bf16) * f16.size(), hipMemcpyHostToDevice) != hipSuccess)
         return MDFT_EHIP;
     return MDFT_OK;

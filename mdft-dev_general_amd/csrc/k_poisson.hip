@@ -289,13 +289,13 @@ hipError_t launch_poisson_vext(mdft_ctx *c, int natom, const double *h_atoms, in
     long long *d_idx = nullptr;
     double *d_val = nullptr, *d_q = nullptr;
     int *d_qsite = nullptr;
-    hipError_t e = hipMalloc(&X, sizeof(double2) * N);
-    if (e == hipSuccess) e = hipMalloc(&Z, sizeof(double2) * N * B);
-    if (e == hipSuccess) e = hipMalloc(&ph, sizeof(double2) * nph);
-    if (e == hipSuccess) e = hipMalloc(&d_idx, sizeof(long long) * idx.size());
-    if (e == hipSuccess) e = hipMalloc(&d_val, sizeof(double) * val.size());
-    if (e == hipSuccess) e = hipMalloc(&d_q, sizeof(double) * (qs.size() + 1));
-    if (e == hipSuccess) e = hipMalloc(&d_qsite, sizeof(int) * (qs.size() + 1));
+    hipError_t e = dev_malloc(&X, sizeof(double2) * N);
+    if (e == hipSuccess) e = dev_malloc(&Z, sizeof(double2) * N * B);
+    if (e == hipSuccess) e = dev_malloc(&ph, sizeof(double2) * nph);
+    if (e == hipSuccess) e = dev_malloc(&d_idx, sizeof(long long) * idx.size());
+    if (e == hipSuccess) e = dev_malloc(&d_val, sizeof(double) * val.size());
+    if (e == hipSuccess) e = dev_malloc(&d_q, sizeof(double) * (qs.size() + 1));
+    if (e == hipSuccess) e = dev_malloc(&d_qsite, sizeof(int) * (qs.size() + 1));
     if (e == hipSuccess) e = hipMemcpy(d_idx, idx.data(), sizeof(long long) * idx.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(d_val, val.data(), sizeof(double) * val.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess && !qs.empty()) e = hipMemcpy(d_q, qs.data(), sizeof(double) * qs.size(), hipMemcpyHostToDevice);
@@ -349,12 +349,12 @@ hipError_t launch_poisson_vext(mdft_ctx *c, int natom, const double *h_atoms, in
         }
     }
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    (void)hipFree(X);
-    (void)hipFree(Z);
-    (void)hipFree(ph);
-    (void)hipFree(d_qsite);
-    (void)hipFree(d_idx);
-    (void)hipFree(d_val);
-    (void)hipFree(d_q);
+    (void)dev_free(X, e == hipSuccess);
+    (void)dev_free(Z, e == hipSuccess);
+    (void)dev_free(ph, e == hipSuccess);
+    (void)dev_free(d_qsite, e == hipSuccess);
+    (void)dev_free(d_idx, e == hipSuccess);
+    (void)dev_free(d_val, e == hipSuccess);
+    (void)dev_free(d_q, e == hipSuccess);
     return e;
 }

@@ -486,7 +486,7 @@ unsigned resident_blocks(const mdft_ctx *c, K kernel, size_t n) {
 
 hipError_t ensure_vec_partials(mdft_ctx *c) {
     if (c->d_vpart) return hipSuccess;
-    return hipMalloc(&c->d_vpart, sizeof(double) * (kMaxBlocks + 8));
+    return dev_malloc(&c->d_vpart, sizeof(double) * (kMaxBlocks + 8));
 }
 
 hipError_t finish_sum(mdft_ctx *c, unsigned nb, double *out) {
@@ -536,7 +536,7 @@ hipError_t launch_widen_f32(mdft_ctx *c, const float2 *in, double2 *out, size_t 
 
 hipError_t vec_multi_dot(mdft_ctx *c, size_t n, int k, const double *const *vecs, const double *x, double *out) {
     if (!c->d_mpart) {
-        hipError_t e = hipMalloc(&c->d_mpart, sizeof(double) * ((size_t)kMaxBlocks * MDFT_VEC_MAX + MDFT_VEC_MAX));
+        hipError_t e = dev_malloc(&c->d_mpart, sizeof(double) * ((size_t)kMaxBlocks * MDFT_VEC_MAX + MDFT_VEC_MAX));
         if (e != hipSuccess) return e;
     }
     VecSet v{};
@@ -650,7 +650,7 @@ hipError_t vec_multi_dot_noalloc(mdft_ctx *c, size_t n, int k, const double *con
 
 hipError_t vec_multi_dot32(mdft_ctx *c, size_t n, int k, const float *const *vecs, const float *x, double *out) {
     if (!c->d_mpart) {
-        hipError_t e = hipMalloc(&c->d_mpart, sizeof(double) * ((size_t)kMaxBlocks * MDFT_VEC_MAX + MDFT_VEC_MAX));
+        hipError_t e = dev_malloc(&c->d_mpart, sizeof(double) * ((size_t)kMaxBlocks * MDFT_VEC_MAX + MDFT_VEC_MAX));
         if (e != hipSuccess) return e;
     }
     VecSet32 v{};
@@ -744,10 +744,10 @@ hipError_t vec_scale_orient(mdft_ctx *c, size_t n, int no, const double *fac, co
 hipError_t launch_density_integrals(mdft_ctx *c, const double *xi, double cav, int *nblocks_out) {
     const unsigned nb = 2048;
     if (c->partials_cap < 3 * (size_t)nb) {
-        (void)hipFree(c->d_partials);
+        (void)dev_free(c->d_partials);
         c->d_partials = nullptr;
         c->partials_cap = 0;
-        hipError_t e = hipMalloc(&c->d_partials, sizeof(double) * 3 * nb);
+        hipError_t e = dev_malloc(&c->d_partials, sizeof(double) * 3 * nb);
         if (e != hipSuccess) return e;
         c->partials_cap = 3 * (size_t)nb;
     }

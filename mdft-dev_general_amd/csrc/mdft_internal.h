@@ -143,6 +143,12 @@ struct mdft_ctx {
     std::string err;
 };
 
+// ---- device memory (devmem.hip): hipMalloc and hipFree that keep freed blocks for the next allocation
+hipError_t dev_malloc_bytes(void **p, size_t bytes);
+template <typename T> hipError_t dev_malloc(T **p, size_t bytes) { return dev_malloc_bytes(reinterpret_cast<void **>(p), bytes); }
+hipError_t dev_free(void *p, bool synced = false);  // synced: all work that used it has ended
+void dev_context(int device, int change);  // a context of the device created (+1) or destroyed (-1)
+
 // ---- launchers (return hipError_t of the launch) ----
 hipError_t launch_angl2proj_f64(mdft_ctx *c, const double *xi, double2 *proj);
 // mode: 0 = energy_and_gradient (df overwritten with ideal+exc gradient),

@@ -279,7 +279,8 @@ int run_excess_pipeline(mdft_ctx *c, const double *xi, int stage, bool timers) {
     if (stage >= 2) HIPCHK(c, f32 ? launch_fft3d_f32(c, p32, +1, nf) : launch_fft3d_f64(c, p64, +1, nf));
     if (timers) HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
     if (stage >= 3) {
-        if (ozm_supported(c)) HIPCHK(c, f32 ? launch_ozm_f32(c, p32) : launch_ozm_f64(c, p64));
+        if (c->packed && c->L <= 2) HIPCHK(c, f32 ? launch_ozp_f32(c, p32) : launch_ozp_f64(c, p64));
+        else if (ozm_supported(c)) HIPCHK(c, f32 ? launch_ozm_f32(c, p32) : launch_ozm_f64(c, p64));
         else HIPCHK(c, f32 ? launch_oz32(c, p32) : launch_oz_f64(c, p64));
     }
     if (timers) HIPCHK(c, hipEventRecord(c->ev[3], c->stream));

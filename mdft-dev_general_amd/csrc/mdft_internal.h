@@ -167,6 +167,8 @@ hipError_t launch_oz_f64(mdft_ctx *c, double2 *proj);
 bool ozm_supported(const mdft_ctx *c);
 int ozm_setup(mdft_ctx *c);
 int ozm_frags(mdft_ctx *c, const std::vector<double2> &tab, int nq, int npc, const std::vector<int> &ia0);
+hipError_t launch_ozp_f64(mdft_ctx *c, double2 *proj);  // packed projections, mmax <= 2
+hipError_t launch_ozp_f32(mdft_ctx *c, float2 *proj);
 hipError_t launch_ozm_f64(mdft_ctx *c, double2 *proj);
 hipError_t launch_ozm_f32(mdft_ctx *c, float2 *proj);
 hipError_t launch_widen_f32(mdft_ctx *c, const float2 *in, double2 *out, size_t n);

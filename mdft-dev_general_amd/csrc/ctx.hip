@@ -289,9 +289,8 @@ int run_excess_pipeline(mdft_ctx *c, const double *xi, int stage, bool timers) {
     return MDFT_OK;
 }
 
-int read_sums(mdft_ctx *c, int nblocks, double *out3) {
-    HIPCHK(c, launch_reduce3(c, nblocks));
-    HIPCHK(c, hipMemcpyAsync(c->h_sums, c->d_sums, sizeof(double) * 3, hipMemcpyDeviceToHost, c->stream));
+int read_sums(mdft_ctx *c, int nblocks, double *out3, bool products = false) {
+    HIPCHK(c, launch_reduce3(c, nblocks, c->h_sums, products ? c->h_sums + 5 : nullptr));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     out3[0] = c->h_sums[0];
     out3[1] = c->h_sums[1];
@@ -473,7 +472,6 @@ int mdft_ctx_create(const mdft_desc *desc, mdft_ctx **out) {
     c->ia0_h = ia0;
     ok = ok && dev_malloc(&c->d_proj, proj_elem_bytes(c) * c->N * np) == hipSuccess;
     ok = ok && dev_malloc(&c->d_vext, sizeof(double) * c->N * c->no) == hipSuccess;
-    ok = ok && dev_malloc(&c->d_sums, sizeof(double) * 8) == hipSuccess;
     ok = ok && hipHostMalloc(&c->h_sums, sizeof(double) * 8, hipHostMallocDefault) == hipSuccess;
     if (!ok) return bad(MDFT_ENOMEM, "device allocation failed");
     if (d.precision == MDFT_PREC_BF16) {
@@ -525,7 +523,7 @@ void mdft_ctx_destroy(mdft_ctx *c) {
     void *bufs[] = {c->d_w,   c->d_a2p,  c->d_p2a,  c->d_fm,   c->d_cph,      c->d_sph,        c->d_cps,
                     c->d_sps, c->d_pidx, c->d_pm,   c->d_pmup, c->d_pmu,      c->d_ia0,        c->d_kx,
                     c->d_ky,  c->d_kz,   c->d_ck,   c->d_vext, c->d_proj,     c->d_xi_stage,   c->d_df_stage,
-                    c->d_partials, c->d_slices, c->d_sums, c->d_vpart, c->d_mpart, c->d_oz32_ftab, c->d_oz32_lanerow,
+                    c->d_partials, c->d_slices, c->d_vpart, c->d_mpart, c->d_oz32_ftab, c->d_oz32_lanerow,
                     c->d_ozm_frag, c->d_ozm_frag16, c->d_ozm_col, c->d_ozm_ftab, c->d_ozm_units, c->d_ozm_rlen,
                     c->d_bf16_M, c->d_bf16_Q, c->d_chscale, c->d_adjscale, c->d_vscale, c->d_dpart, c->d_vext32,
                     c->d_a2p_img[0], c->d_a2p_img[1], c->d_a2p_img[2], c->d_a2p_img[3], c->d_ozm_pack};
@@ -780,12 +778,8 @@ static int evaluate(mdft_ctx *c, const double *xi, double *df, int flags, int mo
     c->dot_k = 0;
     c->packed = false;
     HIPCHK(c, fe);
-    if (fused_dots) {
-        HIPCHK(c, launch_reduce3_buf(c, c->d_dpart, nb, c->d_sums + 5));
-        HIPCHK(c, hipMemcpyAsync(c->h_sums + 5, c->d_sums + 5, sizeof(double) * 3, hipMemcpyDeviceToHost, c->stream));
-    }
     if (timers) HIPCHK(c, hipEventRecord(c->ev[5], c->stream));
-    rc = read_sums(c, nb, sums);
+    rc = read_sums(c, nb, sums, fused_dots);
     if (rc) return rc;
     if (timers) {
         HIPCHK(c, hipEventRecord(c->ev[6], c->stream));

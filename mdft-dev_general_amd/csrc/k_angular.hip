@@ -284,36 +284,41 @@ __global__ __launch_bounds__(kThreads) void ideal_f64(const double *__restrict__
     block_reduce3(fid, fext, zero, partials);
 }
 
-// Sums of the per-workgroup (F_id, F_ext, F_exc) partials in a fixed order (so
-// repeated evaluations are bitwise identical): each workgroup of the first
-// pass sums one contiguous slice, one workgroup sums the slices.
-__global__ __launch_bounds__(kThreads) void reduce3(const double *__restrict__ partials, int nblocks,
-                                                   double *__restrict__ out) {
+// Sums of the per-workgroup (F_id, F_ext, F_exc) partials in a fixed order (so repeated
+// evaluations are bitwise identical).  Workgroup (b, y) sums the b-th contiguous slice of array y
+// (the gradient products are a second array of the same length) into out[y].
+constexpr int kReduce = 1024;
+struct ReduceArgs {
+    const double *part[2];
+    double *out[2];
+};
+__global__ __launch_bounds__(kReduce) void reduce3(ReduceArgs r, int nblocks) {
     const int per = (nblocks + gridDim.x - 1) / gridDim.x;
     const int lo = blockIdx.x * per, hi = min(nblocks, lo + per);
+    const double *partials = r.part[blockIdx.y];
     double a = 0.0, b = 0.0, c = 0.0;
-    for (int i = lo + threadIdx.x; i < hi; i += kThreads) {
+    for (int i = lo + threadIdx.x; i < hi; i += kReduce) {
         a += partials[3 * i + 0];
         b += partials[3 * i + 1];
         c += partials[3 * i + 2];
     }
-    __shared__ double red[3][kThreads];
-    red[0][threadIdx.x] = a;
-    red[1][threadIdx.x] = b;
-    red[2][threadIdx.x] = c;
-    __syncthreads();
-    for (int s = kThreads / 2; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) {
-            red[0][threadIdx.x] += red[0][threadIdx.x + s];
-            red[1][threadIdx.x] += red[1][threadIdx.x + s];
-            red[2][threadIdx.x] += red[2][threadIdx.x + s];
-        }
-        __syncthreads();
+    __shared__ double red[3][kReduce / 64];
+    for (int off = 32; off > 0; off >>= 1) {
+        a += __shfl_down(a, off, 64);
+        b += __shfl_down(b, off, 64);
+        c += __shfl_down(c, off, 64);
     }
-    if (threadIdx.x == 0) {
-        out[3 * blockIdx.x + 0] = red[0][0];
-        out[3 * blockIdx.x + 1] = red[1][0];
-        out[3 * blockIdx.x + 2] = red[2][0];
+    const int wv = threadIdx.x >> 6;
+    if ((threadIdx.x & 63) == 0) {
+        red[0][wv] = a;
+        red[1][wv] = b;
+        red[2][wv] = c;
+    }
+    __syncthreads();
+    if (threadIdx.x < 3) {
+        double s = 0.0;
+        for (int w = 0; w < kReduce / 64; w++) s += red[threadIdx.x][w];
+        r.out[blockIdx.y][3 * blockIdx.x + threadIdx.x] = s;
     }
 }
 
@@ -1203,22 +1208,27 @@ hipError_t launch_ideal_f64(mdft_ctx *c, const double *xi, double *df, int *nblo
     return hipGetLastError();
 }
 
-hipError_t launch_reduce3_buf(mdft_ctx *c, const double *part, int nblocks, double *out) {
+// out[0..2] <- the sums of d_partials and, where products is set, prod_out[0..2] <- those of d_dpart.  The
+// outputs are pinned host memory, written by the kernel itself: a copy after it, and a reduction of
+// its own for the products, made the end of an evaluation 20 us where this takes 8.
+hipError_t launch_reduce3(mdft_ctx *c, int nblocks, double *out, double *prod_out) {
     constexpr int kSlices = 512;
-    if (nblocks <= 4 * kThreads) {
-        hipLaunchKernelGGL(reduce3, dim3(1), dim3(kThreads), 0, c->stream, part, nblocks, out);
-        return hipGetLastError();
+    ReduceArgs r{{c->d_partials, c->d_dpart}, {out, prod_out}};
+    const unsigned arrays = prod_out ? 2 : 1;
+    if (nblocks > 8 * kReduce) {  // (the specialised final passes have at most 8 workgroups per compute unit)
+        if (!c->d_slices) {
+            hipError_t e = dev_malloc(&c->d_slices, sizeof(double) * 6 * kSlices);
+            if (e != hipSuccess) return e;
+        }
+        ReduceArgs s{{c->d_partials, c->d_dpart}, {c->d_slices, c->d_slices + 3 * kSlices}};
+        hipLaunchKernelGGL(reduce3, dim3(kSlices, arrays), dim3(kReduce), 0, c->stream, s, nblocks);
+        r.part[0] = c->d_slices;
+        r.part[1] = c->d_slices + 3 * kSlices;
+        nblocks = kSlices;
     }
-    if (!c->d_slices) {
-        hipError_t e = dev_malloc(&c->d_slices, sizeof(double) * 3 * kSlices);
-        if (e != hipSuccess) return e;
-    }
-    hipLaunchKernelGGL(reduce3, dim3(kSlices), dim3(kThreads), 0, c->stream, part, nblocks, c->d_slices);
-    hipLaunchKernelGGL(reduce3, dim3(1), dim3(kThreads), 0, c->stream, c->d_slices, kSlices, out);
+    hipLaunchKernelGGL(reduce3, dim3(1, arrays), dim3(kReduce), 0, c->stream, r, nblocks);
     return hipGetLastError();
 }
-
-hipError_t launch_reduce3(mdft_ctx *c, int nblocks) { return launch_reduce3_buf(c, c->d_partials, nblocks, c->d_sums); }
 
 FinalConsts final_consts(mdft_ctx *c) {
     FinalConsts k;

@@ -109,8 +109,7 @@ struct mdft_ctx {
     double *d_xi_stage = nullptr; // staging for host xi
     double *d_df_stage = nullptr; // staging for host df
     double *d_partials = nullptr; // block partial sums
-    double *d_slices = nullptr;   // [3 * 512] first-pass sums of d_partials
-    double *d_sums = nullptr;     // [8] final reductions
+    double *d_slices = nullptr;   // [2][3 * 512] first-pass sums of d_partials and d_dpart
     double *d_vpart = nullptr;    // vector-op block partials
     double *d_mpart = nullptr;    // multi-dot block partials [blocks][MDFT_VEC_MAX] + result
     float *df32 = nullptr;        // set during an evaluation with MDFT_DF_FP32: dF goes here, rounded to FP32
@@ -130,7 +129,7 @@ struct mdft_ctx {
     size_t dpart_cap = 0;
     float *d_chscale = nullptr;   // per-channel input scale of the warm-start features [2 np]
     float *d_adjscale = nullptr;  // per-channel factor of the adjoint of proj2angl [2 np]
-    double *h_sums = nullptr;     // pinned mirror of d_sums
+    double *h_sums = nullptr;     // [8] reductions, pinned host memory that the kernels write
     size_t partials_cap = 0;
     bool have_vext = false, have_ck = false;
     hipStream_t stream = nullptr;
@@ -160,7 +159,7 @@ hipError_t launch_angl2proj_f32(mdft_ctx *c, const double *xi, float2 *proj);
 hipError_t launch_final_f32(mdft_ctx *c, const float2 *proj, const double *xi, double *df, int mode, int *nblocks_out);
 hipError_t launch_oz32(mdft_ctx *c, float2 *proj);
 int oz32_tables(mdft_ctx *c, std::vector<float> &ftab, std::vector<int> &itab);
-hipError_t launch_reduce3(mdft_ctx *c, int nblocks);
+hipError_t launch_reduce3(mdft_ctx *c, int nblocks, double *out, double *prod_out);
 hipError_t launch_fft3d_f64(mdft_ctx *c, double2 *proj, int sign, int batch = 0);  // batch 0: np
 hipError_t launch_fft3d_f32(mdft_ctx *c, float2 *proj, int sign, int batch = 0);
 hipError_t launch_oz_f64(mdft_ctx *c, double2 *proj);
@@ -178,7 +177,6 @@ hipError_t launch_regrid(mdft_ctx *c, const double *prev, int pnx, int pny, cons
                          double outside, double *xi);
 hipError_t launch_proj_to_channels(mdft_ctx *c, float *out, float scale, const float *chscale = nullptr);
 hipError_t launch_channels_to_proj(mdft_ctx *c, const float *in);
-hipError_t launch_reduce3_buf(mdft_ctx *c, const double *part, int nblocks, double *out);
 hipError_t launch_cold_start(mdft_ctx *c, double *xi, bool boltzmann = false);
 hipError_t launch_density_mix(mdft_ctx *c, size_t total, double lam, const double *xa, const double *xb,
                               double *out);

@@ -21,17 +21,18 @@
 // |q|, and their c(k) fragments share that die's L2.  Per tile:
 //  0. the 16 projection records X (np complex each) are copied into LDS with
 //     whole-record coalesced loads;
-//  1. rotation to the q frame on the vector ALUs, lanes over pairs: lane
-//     (pair p = l & 7, slot j = l >> 3) takes rotation units (m, khi) from a
-//     host-built round table (units of equal m/2 + 1 in a round, so the lanes
-//     run one instruction stream; rounds balanced over the four waves), forms
-//     R^m(mup, khi) = exp(-i mup phi_q) d^m(mup, khi)(theta_q) once per unit
-//     entry (d^m from its Fourier series in theta, coefficients host-built and
-//     read one iteration ahead) and uses it for both sides and every mu:
+//  1. rotation to the q frame,
 //       A_q(m, khi, mu) = sum_mup X_q(m, mup, mu) R(mup, khi)
-//       A_-q(m, -khi, mu) = (-1)^m sum_mup X_-q(m, mup, mu) R(mup, khi);
-//     in FP32 the phase e^{-i mup phi} is applied once per element of X as it
-//     enters LDS and once per output, so the unit loops multiply by real d^m;
+//       A_-q(m, -khi, mu) = (-1)^m sum_mup X_-q(m, mup, mu) R(mup, khi),
+//     FP32: R as two products with the constant d^m(pi/2) and two phases, on the
+//     matrix cores (rot_item); FP64, whose R the reference chops entry by entry:
+//     on the vector ALUs, lanes over pairs: lane (pair p = l & 7, slot j = l >> 3)
+//     takes rotation units (m, khi) from a host-built round table (units of equal
+//     m/2 + 1 in a round, so the lanes run one instruction stream; rounds balanced
+//     over the four waves), forms R^m(mup, khi) = exp(-i mup phi_q)
+//     d^m(mup, khi)(theta_q) once per unit entry (d^m from its Fourier series in
+//     theta, coefficients host-built and read one iteration ahead) and uses it for
+//     both sides and every mu;
 //  2. OZ contraction (OZ blocks khi spread over the four waves): for each khi
 //     the rows (m, mu) of both sides are
 //       gamma_s(m, khi, mu) = sum_{(n, nu)} c_{m mu; n nu}^{khi}(|q|) V_s(n, nu)
@@ -43,7 +44,7 @@
 //     order the matrix instruction reads them (ozm_frags, at c(k) upload);
 //     alpha and 1 - alpha are applied per row after the product, the result
 //     transposed through LDS to the (side, pair) rows;
-//  3. rotation back on the vector ALUs, units (m, mup):
+//  3. rotation back, on the same units,
 //       out_q(m, mup, mu) = sum_khi gamma_q(m, khi, mu) conj(R(mup, khi))
 //       out_-q(m, mup, mu) = (-1)^m sum_khi gamma_-q(m, khi, mu) conj(R(mup, -khi))
 //     into LDS, then copied out record by record (coalesced).
@@ -207,6 +208,7 @@ template <typename T> struct OzmArgs {
     const T *ftab;              // [entry][kp] Fourier coefficients of d^m(theta)
     const int4 *units;          // [round][8] rotation units
     const int *rlen;            // [round] iterations of each round
+    const float *jtab;          // FP32: [wave][RotPlan::NJ][64] entries of d^m(pi/2) in operand order
     int cr0[2][kWaves][4], cnr[2][kWaves][4];  // first round and count per (direction, wave, class)
 };
 
@@ -234,7 +236,7 @@ template <typename T, int L> struct Lds {
     int flag[8];                // pair flags; bit 2: padding pair of a partial tile
 };
 
-// ---- rotations: one class of units (m/2 + 1 = NMU) ----------------------------------
+// ---- FP64 rotations: one class of units (m/2 + 1 = NMU) -------------------------------
 // rotation in: X from s.xs, A to s.buf; rotation back: gamma from s.buf, the outputs
 // (sign, Nyquist conjugate applied) to s.xs
 template <typename T, int L, int NMU, bool BACK>
@@ -242,9 +244,6 @@ __device__ __forceinline__ void rot_class(const OzmArgs<T> &a, Lds<T, L> &s, int
     using C = typename Ty<T>::c;
     constexpr int KP = Plan<L>::kp;
     constexpr int KC = (2 * NMU < KP) ? 2 * NMU : KP;  // coefficients that can be nonzero for m <= 2 NMU - 1
-    // FP32 (no chop to honour): R = exp(-i mup phi) d factored, X carries the phase from its
-    // load into LDS, the rotation back applies it once per output; real d products in between
-    constexpr bool FACT = sizeof(T) == 4;
     const T *ct = s.trig[p][0], *st = s.trig[p][1];
     const C *xq = s.xs[p], *xmq = s.xs[8 + p];
     const C *gq = s.buf[p], *gmq = s.buf[8 + p];
@@ -291,18 +290,6 @@ __device__ __forceinline__ void rot_class(const OzmArgs<T> &a, Lds<T, L> &s, int
             for (int k = 0; k < KC / 2; k++) {
                 v += o.f[k].x * tg[2 * k];
                 v += o.f[k].y * tg[2 * k + 1];
-            }
-            if constexpr (FACT) {
-#pragma unroll
-                for (int i = 0; i < NMU; i++) {
-                    const C y1 = BACK ? gq[x0 + t * NMU + i] : xq[x0 + t * NMU + i];
-                    const C y2 = BACK ? gmq[x0 + (2 * m - t) * NMU + i] : xmq[x0 + t * NMU + i];
-                    acq[i].x = fma(y1.x, v, acq[i].x);
-                    acq[i].y = fma(y1.y, v, acq[i].y);
-                    acm[i].x = fma(y2.x, v, acm[i].x);
-                    acm[i].y = fma(y2.y, v, acm[i].y);
-                }
-                return;
             }
             C e;
             if (BACK) {
@@ -352,16 +339,6 @@ __device__ __forceinline__ void rot_class(const OzmArgs<T> &a, Lds<T, L> &s, int
         }
         if (w > 0) {
             const T sg = (m & 1) ? (T)-1 : (T)1;
-            if (FACT && BACK) {  // exp(+i mup phi) = conj(eph)
-#pragma unroll
-                for (int i = 0; i < NMU; i++) {
-                    const C u = acq[i], v = acm[i];
-                    acq[i].x = u.x * eph.x + u.y * eph.y;
-                    acq[i].y = u.y * eph.x - u.x * eph.y;
-                    acm[i].x = v.x * eph.x + v.y * eph.y;
-                    acm[i].y = v.y * eph.x - v.x * eph.y;
-                }
-            }
 #pragma unroll
             for (int i = 0; i < NMU; i++) {
                 C o;
@@ -386,6 +363,149 @@ template <typename T, int L, int NMU, bool BACK>
 __device__ __forceinline__ void rot_all(const OzmArgs<T> &a, Lds<T, L> &s, int w, int p, int j) {
     rot_class<T, L, NMU, BACK>(a, s, a.cr0[BACK][w][NMU - 1], a.cnr[BACK][w][NMU - 1], p, j);
     if constexpr (NMU > 1) rot_all<T, L, NMU - 1, BACK>(a, s, w, p, j);
+}
+
+// ---- FP32 rotations on the matrix cores ------------------------------------------------
+// d^m(theta) = i^(a - b) sum_k J_ka J_kb exp(-i k theta) with the constant J = d^m(pi/2), so a rotation is
+//   A(b) i^b = sum_k J_kb exp(-i k theta) sum_a J_ka X(a) exp(-i a phi'),   phi' = phi - pi/2:
+// two products with one matrix for all pairs, X the 16 (side, pair) rows, and two phases.  (The factors
+// i^b cancel between the rotation in and the rotation back: V of an OZ block has one common factor, the
+// sums being linear in V.)  For one (m, mu2), real and imaginary parts apart, with the rows as columns of
+// the B operand: the index of the sum, position a + L = 4 step + (l >> 4), and of the result, register r of
+// lane l, position 4 r + (l >> 4), are laid out alike, so the first product's registers, times their
+// phases, are the second's B operands without leaving the lane.  (On the vector ALUs, R formed per pair
+// and entry in both directions, the kernel took 1.99 against 1.63 ms at 128^3, mmax 5, 0.67 against 0.51 at
+// 100^3, mmax 4.)
+template <int L> struct RotPlan {
+    static constexpr int s0(int m) { return (L - m) / 4; }
+    static constexpr int ns(int m) { return (L + m) / 4 - (L - m) / 4 + 1; }
+    static constexpr int RN = 2 * L / 4 + 1;  // registers with positions up to 2 L
+    // items (m, mu2), m = L .. 1, longest first onto the least loaded wave
+    static constexpr int NI = [] {
+        int n = 0;
+        for (int m = 1; m <= L; m++) n += m / 2 + 1;
+        return n;
+    }();
+    static constexpr int item_m(int i) {
+        for (int m = L; m >= 1; m--) {
+            if (i < m / 2 + 1) return m;
+            i -= m / 2 + 1;
+        }
+        return 0;
+    }
+    static constexpr int item_u(int i) {
+        for (int m = L; m >= 1; m--) {
+            if (i < m / 2 + 1) return i;
+            i -= m / 2 + 1;
+        }
+        return 0;
+    }
+    static constexpr int owner(int item) {
+        int load[kWaves] = {};
+        for (int i = 0; i < NI; i++) {
+            int best = 0;
+            for (int w = 1; w < kWaves; w++)
+                if (load[w] < load[best]) best = w;
+            load[best] += ns(item_m(i));
+            if (i == item) return best;
+        }
+        return 0;
+    }
+    // J entries of a wave: those of its orders, descending
+    static constexpr bool has(int w, int m) {
+        for (int i = 0; i < NI; i++)
+            if (owner(i) == w && item_m(i) == m) return true;
+        return false;
+    }
+    static constexpr int j0(int w, int m) {  // first entry of order m
+        int o = 0;
+        for (int k = L; k > m; k--)
+            if (has(w, k)) o += ns(k);
+        return o;
+    }
+    static constexpr int NJ = [] {
+        int n = 1;
+        for (int w = 0; w < kWaves; w++) n = j0(w, 0) > n ? j0(w, 0) : n;
+        return n;
+    }();
+};
+
+// what a lane keeps for the rotations of its row's pair
+template <int L> struct RotLane {
+    float j[RotPlan<L>::NJ];        // its wave's J entries
+    float sg;                       // J_ka from J_ak: (-1)^(a - k)
+    float2 th[RotPlan<L>::RN];      // exp(-i k theta), k = 4 r + (l >> 4) - L
+    float2 ph[RotPlan<L>::RN];      // exp(+i a phi')
+    bool mq, conj_mq;               // a row of -q; q == -q on a Nyquist plane
+};
+
+template <int L, bool BACK, int M, int U, int J0>
+__device__ __forceinline__ void rot_item(Lds<float, L> &s, const RotLane<L> &c, int l) {
+    using P = Plan<L>;
+    constexpr int S0 = RotPlan<L>::s0(M), NS = RotPlan<L>::ns(M), NM = P::nmu(M), P0 = P::poff(M) + M * NM + U;
+    const int g = l >> 4, row = l & 15;
+    const float2 *src = BACK ? s.buf[row] : s.xs[row];
+    float2 x[NS];
+#pragma unroll
+    for (int q = 0; q < NS; q++) {  // positions beyond +-M read a valid entry: their J is 0
+        int a = 4 * (S0 + q) + g - L;
+        a = a < -M ? -M : (a > M ? M : a);
+        if (BACK && c.mq) a = -a;
+        x[q] = src[P0 + a * NM];
+    }
+    f4 yr = {0, 0, 0, 0}, yi = yr, zr = yr, zi = yr;
+#pragma unroll
+    for (int q = 0; q < NS; q++) {
+        const float ja = c.j[J0 + q] * c.sg;
+        yr = mfma16(ja, x[q].x, yr);
+        yi = mfma16(ja, x[q].y, yi);
+    }
+#pragma unroll
+    for (int q = 0; q < NS; q++) {
+        const float2 e = c.th[S0 + q];
+        const float ey = BACK ? -e.y : e.y, vr = yr[S0 + q], vi = yi[S0 + q];
+        zr = mfma16(c.j[J0 + q], vr * e.x - vi * ey, zr);
+        zi = mfma16(c.j[J0 + q], vr * ey + vi * e.x, zi);
+    }
+#pragma unroll
+    for (int q = 0; q < NS; q++) {
+        const int b = 4 * (S0 + q) + g - L;
+        if (b < -M || b > M) continue;
+        float2 v = make_float2(zr[S0 + q], zi[S0 + q]);
+        if ((M & 1) && c.mq) v = make_float2(-v.x, -v.y);
+        if (!BACK) {
+            s.buf[row][P0 + (c.mq ? -b : b) * NM] = v;
+        } else {
+            const float2 e = c.ph[S0 + q];
+            v = make_float2(v.x * e.x - v.y * e.y, v.x * e.y + v.y * e.x);
+            if (c.conj_mq && c.mq) v.y = -v.y;
+            s.xs[row][P0 + b * NM] = v;
+        }
+    }
+}
+
+template <int L, bool BACK, int W, int I>
+__device__ __forceinline__ void rot_items(Lds<float, L> &s, const RotLane<L> &c, int l) {
+    using R = RotPlan<L>;
+    if constexpr (I < R::NI) {
+        if constexpr (R::owner(I) == W) rot_item<L, BACK, R::item_m(I), R::item_u(I), R::j0(W, R::item_m(I))>(s, c, l);
+        rot_items<L, BACK, W, I + 1>(s, c, l);
+    }
+}
+template <int L, bool BACK, int W = 0>
+__device__ __forceinline__ void rot_wave(Lds<float, L> &s, const RotLane<L> &c, int w, int l) {
+    if constexpr (W < kWaves) {
+        if (w == W) {
+            rot_items<L, BACK, W, 0>(s, c, l);
+            if (W == kWaves - 1 && l < 16) {  // m = 0: R = 1
+                float2 v = BACK ? s.buf[l][0] : s.xs[l][0];
+                if (BACK && c.conj_mq && c.mq) v.y = -v.y;
+                (BACK ? s.xs : s.buf)[l][0] = v;
+            }
+        } else {
+            rot_wave<L, BACK, W + 1>(s, c, w, l);
+        }
+    }
 }
 
 // ---- OZ block khi on the matrix cores -------------------------------------------------
@@ -595,10 +715,9 @@ __device__ __forceinline__ void pack_out(int d, typename Ty<T>::c &oq, typename 
     }
 }
 
-// FP32: at least 7 waves per SIMD (72 registers, no spills; at the compiler's own choice of 88
-// registers, 5 waves and 2.13 against 2.01 ms at 128^3, mmax 5)
+// FP32: at least 5 waves per SIMD (96 registers; at 6 or 7 it spills: 128^3, mmax 5 1.63, 2.04 and 2.23 ms)
 template <typename T, int L, bool BF, bool PACK>
-__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 7 : 1, 8))) void ozm(typename Ty<T>::c *__restrict__ proj, OzmArgs<T> a) {
+__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 5 : 1, 8))) void ozm(typename Ty<T>::c *__restrict__ proj, OzmArgs<T> a) {
     using P = Plan<L>;
     using C = typename Ty<T>::c;
     constexpr int KP = P::kp, NP = P::np;
@@ -630,30 +749,42 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(siz
             pb[k] = reinterpret_cast<const Vec *>(proj + (size_t)tps[pr].gmq * NPK)[e];
         }
     }
-    if (tid < 8) {
-        const TilePair tp = tps[tid];
-        s.g[tid] = tp.gq;
-        s.g[8 + tid] = tp.gmq;
-        s.flag[tid] = tp.flag;
-        C abv;
-        abv.x = (T)tp.al;
-        abv.y = (T)(1.0 - tp.al);
-        s.ab[tid] = abv;
-        double ck = 1.0, sk = 0.0, cpk = 1.0, spk = 0.0;
-        for (int k = 0; k < KP; k++) {
-            s.trig[tid][0][k] = (T)ck;
-            s.trig[tid][1][k] = (T)sk;
-            C e;
-            e.x = (T)cpk;
-            e.y = (T)spk;
-            s.ph[tid][k] = e;
-            const double nc = ck * tp.ct - sk * tp.st;
-            sk = sk * tp.ct + ck * tp.st;
-            ck = nc;
-            const double nq = cpk * tp.cp - spk * tp.sp;
-            spk = spk * tp.cp + cpk * tp.sp;
-            cpk = nq;
+    if (tid < 16) {  // lanes 0-7: theta, 8-15: phi (FP32: phi - pi/2) of the pairs
+        const TilePair tp = tps[p];
+        const bool phi = tid >= 8;
+        if (!phi) {
+            s.g[p] = tp.gq;
+            s.g[8 + p] = tp.gmq;
+            s.flag[p] = tp.flag;
+            C abv;
+            abv.x = (T)tp.al;
+            abv.y = (T)(1.0 - tp.al);
+            s.ab[p] = abv;
         }
+        const double pc = sizeof(T) == 4 ? tp.sp : tp.cp, ps = sizeof(T) == 4 ? -tp.cp : tp.sp;
+        const double c1 = phi ? pc : tp.ct, s1 = phi ? ps : tp.st;
+        double ck = 1.0, sk = 0.0;
+        for (int k = 0; k < KP; k++) {
+            if (phi) {
+                C e;
+                e.x = (T)ck;
+                e.y = (T)sk;
+                s.ph[p][k] = e;
+            } else {
+                s.trig[p][0][k] = (T)ck;
+                s.trig[p][1][k] = (T)sk;
+            }
+            const double nc = ck * c1 - sk * s1;
+            sk = sk * c1 + ck * s1;
+            ck = nc;
+        }
+    }
+    [[maybe_unused]] RotLane<sizeof(T) == 4 ? L : 0> rl;
+    if constexpr (sizeof(T) == 4) {
+#pragma unroll
+        for (int q = 0; q < RotPlan<L>::NJ; q++) rl.j[q] = a.jtab[(w * RotPlan<L>::NJ + q) * 64 + l];
+        rl.sg = (((l & 15) >> 2) + (l >> 4)) & 1 ? -1.0f : 1.0f;
+        rl.mq = (l & 15) >= 8;
     }
     __syncthreads();
     if constexpr (PACK) {
@@ -705,7 +836,19 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(siz
         }
         __syncthreads();
     }
-    rot_all<T, L, P::nclass, false>(a, s, w, p, j);
+    if constexpr (sizeof(T) == 4) {
+#pragma unroll
+        for (int r = 0; r < RotPlan<L>::RN; r++) {
+            const int k = 4 * r + (l >> 4) - L, ak = k < 0 ? -k : (k > L ? L : k);
+            rl.th[r] = make_float2(s.trig[p][0][ak], k < 0 ? s.trig[p][1][ak] : -s.trig[p][1][ak]);
+            const float2 z = s.ph[p][ak];
+            rl.ph[r] = make_float2(z.x, k < 0 ? -z.y : z.y);
+        }
+        rl.conj_mq = (s.flag[p] & 3) == 3;
+        rot_wave<L, false>(s, rl, w, l);
+    } else {
+        rot_all<T, L, P::nclass, false>(a, s, w, p, j);
+    }
     __syncthreads();
     {
         const C abv = s.ab[l & 7];  // the pair of row l & 15
@@ -713,7 +856,8 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(siz
         oz_wave<T, L, BF, 0>(s, a, (size_t)(iq - 1), scr, abv.x, abv.y, w, l);
     }
     __syncthreads();
-    rot_all<T, L, P::nclass, true>(a, s, w, p, j);
+    if constexpr (sizeof(T) == 4) rot_wave<L, true>(s, rl, w, l);
+    else rot_all<T, L, P::nclass, true>(a, s, w, p, j);
     __syncthreads();
     // store rule (:648-656): both sides of real pairs; for q == -q only the -q side
     if constexpr (PACK) {
@@ -766,6 +910,8 @@ double textbook_d_h(int j, int mp, int m, double beta) {
 
 struct HostPlan {
     int L, np, kp, nclass, nfrag, nfrag32;
+    int nj = 1;
+    std::vector<int> jm, js;  // [wave][nj] order and step of each J entry of the FP32 rotations (order 0: none)
     std::vector<int> col[2 * MDFT_MAX_MMAX + 1], row[2 * MDFT_MAX_MMAX + 1];
     std::vector<int> nkb, nnb, foff, ncol, nkb32, foff32;
 };
@@ -779,6 +925,16 @@ template <int L> HostPlan host_plan() {
     h.nclass = P::nclass;
     h.nfrag = P::nfrag;
     h.nfrag32 = P::nfrag32;
+    using R = RotPlan<L>;
+    h.nj = R::NJ;
+    h.jm.assign(kWaves * R::NJ, 0);
+    h.js.assign(kWaves * R::NJ, 0);
+    for (int w = 0; w < kWaves; w++)
+        for (int m = 1; m <= L; m++)
+            for (int q = 0; R::has(w, m) && q < R::ns(m); q++) {
+                h.jm[w * R::NJ + R::j0(w, m) + q] = m;
+                h.js[w * R::NJ + R::j0(w, m) + q] = R::s0(m) + q;
+            }
     for (int khi = -L; khi <= L; khi++) {
         for (int c = 0; c < 32; c++) h.col[khi + L].push_back(P::col(khi, c));
         for (int r = 0; r < 4 * P::nnb(khi); r++) h.row[khi + L].push_back(P::row(khi, r));
@@ -817,6 +973,7 @@ template <typename T, int L, bool BF, bool PACK = false> hipError_t launch_ozm_t
     a.ftab = static_cast<const T *>(c->d_ozm_ftab);
     a.units = reinterpret_cast<const int4 *>(c->d_ozm_units);
     a.rlen = c->d_ozm_rlen;
+    a.jtab = c->d_ozm_jtab;
     for (int d = 0; d < 2; d++)
         for (int wv = 0; wv < kWaves; wv++)
             for (int k = 0; k < 4; k++) {
@@ -915,6 +1072,20 @@ int ozm_setup(mdft_ctx *c) {
                     ftab[e * kp + k] = v;
                 }
             }
+    }
+    if (c->d.precision != MDFT_PREC_FP64) {
+        // J entries of the FP32 rotations: lane l of step s holds J_kb = d^m_{k,b}(pi/2), k + L = 4 s + (l >> 4) and
+        // b + L = 4 (i & 3) + (i >> 2), i = l & 15
+        std::vector<double> jt((size_t)kWaves * h.nj * 64, 0.0);
+        for (size_t e = 0; e < h.jm.size(); e++)
+            for (int l = 0; h.jm[e] > 0 && l < 64; l++) {
+                const int m = h.jm[e], i = l & 15, k = 4 * h.js[e] + (l >> 4) - L, b = 4 * (i & 3) + (i >> 2) - L;
+                if (std::abs(k) <= m && std::abs(b) <= m) jt[e * 64 + l] = textbook_d_h(m, k, b, hp);
+            }
+        void *p = nullptr;
+        const int rc = upload_t<float>(c, &p, jt);
+        c->d_ozm_jtab = static_cast<float *>(p);
+        if (rc != MDFT_OK) return rc;
     }
     auto nmu = [](int m) { return m / 2 + 1; };
     std::vector<int> poff(L + 2, 0);

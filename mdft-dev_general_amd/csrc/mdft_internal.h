@@ -124,6 +124,7 @@ struct mdft_ctx {
     void *d_a2p_img[4] = {};      // angl2proj_t's weights: FP32, FP64, packed FP32, packed FP64
     bool packed = false;          // set during an evaluation whose projection field is packed (packed.h)
     int npk = 0;                  // packed projections per point
+    float *d_ozm_jtab = nullptr;  // FP32: d^m(pi/2) entries of the q-space kernel's rotations
     int *d_ozm_pack = nullptr;    // packed entries of the q-space kernel
     bool vext32_ok = false;       // d_vext32 holds the current vext
     size_t dpart_cap = 0;

@@ -170,20 +170,25 @@ int build_pairs(mdft_ctx *c) {
         }
     }
     const int npairs = (int)pq.size();
-    std::vector<int> order(npairs);
+    std::vector<int> order(npairs), chopped;
+    const int rc = ozm_chopped(c, pq, chopped);
+    if (rc != MDFT_OK) return fail(c, rc, "classes of the q-space pairs");
     for (int i = 0; i < npairs; i++) order[i] = i;
-    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return piq[a] < piq[b]; });
-    std::vector<int> spq(npairs), spmq(npairs), sflag(npairs), cstart, ccount, ciq;
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
+        return chopped[a] != chopped[b] ? chopped[a] < chopped[b] : piq[a] < piq[b];
+    });
+    std::vector<int> spq(npairs), spmq(npairs), sflag(npairs), cstart, ccount, ciq, cchop;
     const int CH = 256;
     for (int i = 0; i < npairs; i++) {
         const int k = order[i];
         spq[i] = pq[k];
         spmq[i] = pmq[k];
         sflag[i] = pflag[k];
-        if (cstart.empty() || ciq.back() != piq[k] || ccount.back() == CH) {
+        if (cstart.empty() || ciq.back() != piq[k] || cchop.back() != chopped[k] || ccount.back() == CH) {
             cstart.push_back(i);
             ccount.push_back(0);
             ciq.push_back(piq[k]);
+            cchop.push_back(chopped[k]);
         }
         ccount.back()++;
     }
@@ -204,6 +209,7 @@ int build_pairs(mdft_ctx *c) {
         for (int o = 0; o < ccount[k]; o += 8) {
             const int n8 = std::min(8, ccount[k] - o);
             tstart.push_back(cstart[k] + o);
+            if (!cchop[k]) p.nfold++;
             tinfo.push_back(n8 | ciq[k] << 4);
             for (int j = 0; j < 8; j++) {
                 // padding entries repeat the tile's first pair (valid memory, never stored)
@@ -526,7 +532,7 @@ void mdft_ctx_destroy(mdft_ctx *c) {
                     c->d_partials, c->d_slices, c->d_vpart, c->d_mpart, c->d_oz32_ftab, c->d_oz32_lanerow,
                     c->d_ozm_frag, c->d_ozm_frag16, c->d_ozm_col, c->d_ozm_ftab, c->d_ozm_units, c->d_ozm_rlen,
                     c->d_bf16_M, c->d_bf16_Q, c->d_chscale, c->d_adjscale, c->d_vscale, c->d_dpart, c->d_vext32,
-                    c->d_a2p_img[0], c->d_a2p_img[1], c->d_a2p_img[2], c->d_a2p_img[3], c->d_ozm_pack, c->d_ozm_jtab};
+                    c->d_a2p_img[0], c->d_a2p_img[1], c->d_a2p_img[2], c->d_a2p_img[3], c->d_ozm_pack, c->d_ozm_jfold};
     for (void *b : bufs)
         if (b) (void)dev_free(b);
     free_pairs(c->pairs);

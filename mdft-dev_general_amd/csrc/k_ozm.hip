@@ -24,15 +24,18 @@
 //  1. rotation to the q frame,
 //       A_q(m, khi, mu) = sum_mup X_q(m, mup, mu) R(mup, khi)
 //       A_-q(m, -khi, mu) = (-1)^m sum_mup X_-q(m, mup, mu) R(mup, khi),
-//     FP32: R as two products with the constant d^m(pi/2) and two phases, on the
-//     matrix cores (rot_item); FP64, whose R the reference chops entry by entry:
-//     on the vector ALUs, lanes over pairs: lane (pair p = l & 7, slot j = l >> 3)
-//     takes rotation units (m, khi) from a host-built round table (units of equal
-//     m/2 + 1 in a round, so the lanes run one instruction stream; rounds balanced
-//     over the four waves), forms R^m(mup, khi) = exp(-i mup phi_q)
-//     d^m(mup, khi)(theta_q) once per unit entry (d^m from its Fourier series in
-//     theta, coefficients host-built and read one iteration ahead) and uses it for
-//     both sides and every mu;
+//     in one of two forms:
+//     - folded (FP32; FP64 from mmax 3 on, for the pairs whose chops are those of
+//       mup = 0 only): R as a product of two constant matrices, a phase between
+//       (rot_fold), lanes over (side, pair) rows and mu;
+//     - entry by entry (rot_class; the other FP64 pairs, 5 to 9 % of them): lanes over
+//       pairs, lane (pair p = l & 7, slot j = l >> 3) takes rotation units (m, khi) from a
+//       host-built round table (units of equal m/2 + 1 in a round, so the lanes run one
+//       instruction stream; rounds balanced over the four waves), forms R^m(mup, khi) =
+//       exp(-i mup phi_q) d^m(mup, khi)(theta_q) once per unit entry (d^m from its Fourier
+//       series in theta, coefficients host-built and read one iteration ahead), chops it
+//       and uses it for both sides and every mu.
+//     The pairs are sorted by form, each form is a launch of its own;
 //  2. OZ contraction (OZ blocks khi spread over the four waves): for each khi
 //     the rows (m, mu) of both sides are
 //       gamma_s(m, khi, mu) = sum_{(n, nu)} c_{m mu; n nu}^{khi}(|q|) V_s(n, nu)
@@ -44,14 +47,13 @@
 //     order the matrix instruction reads them (ozm_frags, at c(k) upload);
 //     alpha and 1 - alpha are applied per row after the product, the result
 //     transposed through LDS to the (side, pair) rows;
-//  3. rotation back, on the same units,
+//  3. rotation back, in the same form,
 //       out_q(m, mup, mu) = sum_khi gamma_q(m, khi, mu) conj(R(mup, khi))
 //       out_-q(m, mup, mu) = (-1)^m sum_khi gamma_-q(m, khi, mu) conj(R(mup, -khi))
 //     into LDS, then copied out record by record (coalesced).
-// R is formed from the factorisation with d^m from its Fourier series (both
-// exact in FP64 to rounding), then chopped as the reference chops its
-// recursion's result; the OZ sums are summed in the matrix unit's order (a
-// rounding-level difference from the reference's order).
+// R is formed from the factorisation (exact in FP64 to rounding), then chopped as the
+// reference chops its recursion's result; the OZ sums are summed in the matrix unit's
+// order (a rounding-level difference from the reference's order).
 // BF16 contexts run the FP32 kernel with the contraction in BF16 operands and
 // FP32 accumulation (v_mfma_f32_16x16x32_bf16: 16 complex columns per
 // instruction), the c(k) fragments stored in BF16.
@@ -196,9 +198,10 @@ template <int L> struct Plan {
 };
 
 constexpr int kWaves = 4;  // waves per tile
+constexpr int kFold64 = 3;  // smallest mmax with folded rotations in FP64
 
 template <typename T> struct OzmArgs {
-    int ntiles, per;
+    int tile0, ntiles, per;     // the launch's tiles: tile0 .. tile0 + ntiles - 1
     const TilePair *tpair;      // [tile][8] the tiles' pairs
     const int *pmup;            // mup of each projection
     const int *pack;            // packed entries: projection | second << 8 | kind << 16 | (mup + 16) << 20
@@ -208,7 +211,7 @@ template <typename T> struct OzmArgs {
     const T *ftab;              // [entry][kp] Fourier coefficients of d^m(theta)
     const int4 *units;          // [round][8] rotation units
     const int *rlen;            // [round] iterations of each round
-    const float *jtab;          // FP32: [wave][RotPlan::NJ][64] entries of d^m(pi/2) in operand order
+    const T *jfold;             // [m][k][a], 0 <= k, a <= m: d^m_{k,a}(pi/2), times sqrt(2) for k > 0
     int cr0[2][kWaves][4], cnr[2][kWaves][4];  // first round and count per (direction, wave, class)
 };
 
@@ -216,10 +219,19 @@ template <typename T> struct OzmArgs {
 // padded so that a lane's four values are one aligned 16-byte-multiple read
 template <typename T> constexpr int scr_stride() { return sizeof(T) == 8 ? 18 : 20; }
 
-// LDS of one tile: X (then the rotated-back outputs; during the OZ step the transpose
-// scratch) and A (then gamma) per (side, pair) row, the pairs' angles, interpolation
-// weights and grid indices
-template <typename T, int L> struct Lds {
+// LDS of one tile, one row per (side, pair): with entry by entry rotations (FOLD false) X (then the
+// rotated-back outputs; during the OZ step the transpose scratch) and A (then gamma) apart; folded rotations
+// and the OZ step work in place, the scratch beside.  Then the pairs' angles, interpolation weights and grid
+// indices.
+template <typename T, int L, bool FOLD> struct LdsRows {
+    using C = typename Ty<T>::c;
+    C buf[16][Plan<L>::nps];
+    T scratch[kWaves * 16 * scr_stride<T>()];
+    __device__ C (*x())[Plan<L>::nps] { return buf; }
+    __device__ const C (*x() const)[Plan<L>::nps] { return buf; }
+    __device__ T *scr() { return scratch; }
+};
+template <typename T, int L> struct LdsRows<T, L, false> {
     using C = typename Ty<T>::c;
     static constexpr int kScr = kWaves * 16 * scr_stride<T>();  // scratch values (T)
     static constexpr int xrows() {
@@ -229,18 +241,27 @@ template <typename T, int L> struct Lds {
     static constexpr int kXRows = xrows();
     C xs[kXRows][Plan<L>::nps];
     C buf[16][Plan<L>::nps];
+    __device__ C (*x())[Plan<L>::nps] { return xs; }
+    __device__ const C (*x() const)[Plan<L>::nps] { return xs; }
+    __device__ T *scr() { return reinterpret_cast<T *>(&xs[0][0]); }
+};
+template <typename T, int L, bool FOLD> struct Lds : LdsRows<T, L, FOLD> {
+    using C = typename Ty<T>::c;
+    static constexpr bool kChop = sizeof(T) == 8;
     T trig[8][2][Plan<L>::kp];  // cos k theta, sin k theta of each pair
     C ph[8][Plan<L>::kp];       // exp(+i k phi) of each pair
     C ab[8];                    // (alpha, 1 - alpha) of each pair
+    static constexpr int nd = FOLD && kChop ? (L + 1) * (L + 2) / 2 : 1;
+    T d0[8][nd];                // FOLD: chopped d^m_{0,b}(theta) of each pair, (m, b >= 0) at m (m + 1) / 2 + b
     int g[16];                  // grid index of each row (q side rows 0-7, -q side rows 8-15)
     int flag[8];                // pair flags; bit 2: padding pair of a partial tile
 };
 
-// ---- FP64 rotations: one class of units (m/2 + 1 = NMU) -------------------------------
+// ---- entry by entry rotations (FP64): one class of units (m/2 + 1 = NMU) --------------
 // rotation in: X from s.xs, A to s.buf; rotation back: gamma from s.buf, the outputs
 // (sign, Nyquist conjugate applied) to s.xs
 template <typename T, int L, int NMU, bool BACK>
-__device__ __forceinline__ void rot_class(const OzmArgs<T> &a, Lds<T, L> &s, int r0, int nr, int p, int j) {
+__device__ __forceinline__ void rot_class(const OzmArgs<T> &a, Lds<T, L, false> &s, int r0, int nr, int p, int j) {
     using C = typename Ty<T>::c;
     constexpr int KP = Plan<L>::kp;
     constexpr int KC = (2 * NMU < KP) ? 2 * NMU : KP;  // coefficients that can be nonzero for m <= 2 NMU - 1
@@ -360,151 +381,164 @@ __device__ __forceinline__ void rot_class(const OzmArgs<T> &a, Lds<T, L> &s, int
 }
 
 template <typename T, int L, int NMU, bool BACK>
-__device__ __forceinline__ void rot_all(const OzmArgs<T> &a, Lds<T, L> &s, int w, int p, int j) {
+__device__ __forceinline__ void rot_all(const OzmArgs<T> &a, Lds<T, L, false> &s, int w, int p, int j) {
     rot_class<T, L, NMU, BACK>(a, s, a.cr0[BACK][w][NMU - 1], a.cnr[BACK][w][NMU - 1], p, j);
     if constexpr (NMU > 1) rot_all<T, L, NMU - 1, BACK>(a, s, w, p, j);
 }
 
-// ---- FP32 rotations on the matrix cores ------------------------------------------------
-// d^m(theta) = i^(a - b) sum_k J_ka J_kb exp(-i k theta) with the constant J = d^m(pi/2), so a rotation is
-//   A(b) i^b = sum_k J_kb exp(-i k theta) sum_a J_ka X(a) exp(-i a phi'),   phi' = phi - pi/2:
-// two products with one matrix for all pairs, X the 16 (side, pair) rows, and two phases.  (The factors
-// i^b cancel between the rotation in and the rotation back: V of an OZ block has one common factor, the
-// sums being linear in V.)  For one (m, mu2), real and imaginary parts apart, with the rows as columns of
-// the B operand: the index of the sum, position a + L = 4 step + (l >> 4), and of the result, register r of
-// lane l, position 4 r + (l >> 4), are laid out alike, so the first product's registers, times their
-// phases, are the second's B operands without leaving the lane.  (On the vector ALUs, R formed per pair
-// and entry in both directions, the kernel took 1.99 against 1.63 ms at 128^3, mmax 5, 0.67 against 0.51 at
-// 100^3, mmax 4.)
-template <int L> struct RotPlan {
-    static constexpr int s0(int m) { return (L - m) / 4; }
-    static constexpr int ns(int m) { return (L + m) / 4 - (L - m) / 4 + 1; }
-    static constexpr int RN = 2 * L / 4 + 1;  // registers with positions up to 2 L
-    // items (m, mu2), m = L .. 1, longest first onto the least loaded wave
-    static constexpr int NI = [] {
-        int n = 0;
-        for (int m = 1; m <= L; m++) n += m / 2 + 1;
-        return n;
-    }();
-    static constexpr int item_m(int i) {
-        for (int m = L; m >= 1; m--) {
-            if (i < m / 2 + 1) return m;
-            i -= m / 2 + 1;
-        }
-        return 0;
-    }
-    static constexpr int item_u(int i) {
-        for (int m = L; m >= 1; m--) {
-            if (i < m / 2 + 1) return i;
-            i -= m / 2 + 1;
-        }
-        return 0;
-    }
-    static constexpr int owner(int item) {
-        int load[kWaves] = {};
-        for (int i = 0; i < NI; i++) {
-            int best = 0;
-            for (int w = 1; w < kWaves; w++)
-                if (load[w] < load[best]) best = w;
-            load[best] += ns(item_m(i));
-            if (i == item) return best;
-        }
-        return 0;
-    }
-    // J entries of a wave: those of its orders, descending
-    static constexpr bool has(int w, int m) {
-        for (int i = 0; i < NI; i++)
-            if (owner(i) == w && item_m(i) == m) return true;
-        return false;
-    }
-    static constexpr int j0(int w, int m) {  // first entry of order m
-        int o = 0;
-        for (int k = L; k > m; k--)
-            if (has(w, k)) o += ns(k);
-        return o;
-    }
-    static constexpr int NJ = [] {
-        int n = 1;
-        for (int w = 0; w < kWaves; w++) n = j0(w, 0) > n ? j0(w, 0) : n;
-        return n;
-    }();
-};
+// ---- folded rotations ----------------------------------------------------------------
+// d^m_ab(theta) = i^(a - b) sum_k J_ka J_kb exp(-i k theta) with the constant J = d^m(pi/2), and
+// J_k,-a = (-1)^(m + k) J_ka, J_-k,a = (-1)^(m + a) J_ka.  So with x(a) = X(a) exp(-i a phi) and
+// T+-(a) = i^a (x(a) +- (-1)^a x(-a)), all sums over k, a >= 0,
+//   Ue(k) = sum_{a even} J_ka T(a), Uo(k) = sum_{a odd} J_ka T(a), T = T+ where m + k is even, T- else,
+//   Pc = cos(k theta) Ue - i sin(k theta) Uo, Ps = cos(k theta) Uo - i sin(k theta) Ue   (times 2 for k > 0),
+//   A(+-b) = (-1)^m for -b, times i^(-+b) [sum_{k even} J_kb P(k) +- sum_{k odd} J_kb P(k)],
+// P = Pc for even b, Ps for odd b, and the rotation back is the same with i -> 1 / i in front and exp(+i a phi)
+// behind.  FP64 leaves a = 0 out of the product: its entries, real and rounded to single precision by the chop,
+// come from s.d0.
+// A lane has all a and b of one row, order and mu2 in registers, reads and writes each LDS value once and
+// works in place; the J are the same for the wave.  A sixth of the multiplications of the entry by entry form,
+// whose LDS reads (every X once per khi) were its bound: 128^3, mmax 5 FP64 4.42 -> 2.64 ms, 96^3, mmax 3 644 ->
+// 379 us, with the tiles that keep that form.  In FP32, against two products with J on the matrix cores (whose
+// rate in FP32 and FP64 is the vector ALUs', here with no padding to 16 and no zeros): 128^3, mmax 5 1.61 -> 1.22
+// ms, 96^3, mmax 3 250 -> 210 us.
+template <int K, typename C> __device__ __forceinline__ C times_i(C z) {  // i^K z
+    constexpr int q = K & 3;
+    C o;
+    if constexpr (q == 0) o = z;
+    if constexpr (q == 1) o.x = -z.y, o.y = z.x;
+    if constexpr (q == 2) o.x = -z.x, o.y = -z.y;
+    if constexpr (q == 3) o.x = z.y, o.y = -z.x;
+    return o;
+}
 
-// what a lane keeps for the rotations of its row's pair
-template <int L> struct RotLane {
-    float j[RotPlan<L>::NJ];        // its wave's J entries
-    float sg;                       // J_ka from J_ak: (-1)^(a - k)
-    float2 th[RotPlan<L>::RN];      // exp(-i k theta), k = 4 r + (l >> 4) - L
-    float2 ph[RotPlan<L>::RN];      // exp(+i a phi')
-    bool mq, conj_mq;               // a row of -q; q == -q on a Nyquist plane
-};
-
-template <int L, bool BACK, int M, int U, int J0>
-__device__ __forceinline__ void rot_item(Lds<float, L> &s, const RotLane<L> &c, int l) {
-    using P = Plan<L>;
-    constexpr int S0 = RotPlan<L>::s0(M), NS = RotPlan<L>::ns(M), NM = P::nmu(M), P0 = P::poff(M) + M * NM + U;
-    const int g = l >> 4, row = l & 15;
-    const float2 *src = BACK ? s.buf[row] : s.xs[row];
-    float2 x[NS];
-#pragma unroll
-    for (int q = 0; q < NS; q++) {  // positions beyond +-M read a valid entry: their J is 0
-        int a = 4 * (S0 + q) + g - L;
-        a = a < -M ? -M : (a > M ? M : a);
-        if (BACK && c.mq) a = -a;
-        x[q] = src[P0 + a * NM];
-    }
-    f4 yr = {0, 0, 0, 0}, yi = yr, zr = yr, zi = yr;
-#pragma unroll
-    for (int q = 0; q < NS; q++) {
-        const float ja = c.j[J0 + q] * c.sg;
-        yr = mfma16(ja, x[q].x, yr);
-        yi = mfma16(ja, x[q].y, yi);
-    }
-#pragma unroll
-    for (int q = 0; q < NS; q++) {
-        const float2 e = c.th[S0 + q];
-        const float ey = BACK ? -e.y : e.y, vr = yr[S0 + q], vi = yi[S0 + q];
-        zr = mfma16(c.j[J0 + q], vr * e.x - vi * ey, zr);
-        zi = mfma16(c.j[J0 + q], vr * ey + vi * e.x, zi);
-    }
-#pragma unroll
-    for (int q = 0; q < NS; q++) {
-        const int b = 4 * (S0 + q) + g - L;
-        if (b < -M || b > M) continue;
-        float2 v = make_float2(zr[S0 + q], zi[S0 + q]);
-        if ((M & 1) && c.mq) v = make_float2(-v.x, -v.y);
-        if (!BACK) {
-            s.buf[row][P0 + (c.mq ? -b : b) * NM] = v;
-        } else {
-            const float2 e = c.ph[S0 + q];
-            v = make_float2(v.x * e.x - v.y * e.y, v.x * e.y + v.y * e.x);
-            if (c.conj_mq && c.mq) v.y = -v.y;
-            s.xs[row][P0 + b * NM] = v;
-        }
+template <int A, int B, typename F> __device__ __forceinline__ void steps(F &&f) {
+    if constexpr (A < B) {
+        f(std::integral_constant<int, A>{});
+        steps<A + 1, B>(f);
     }
 }
 
-template <int L, bool BACK, int W, int I>
-__device__ __forceinline__ void rot_items(Lds<float, L> &s, const RotLane<L> &c, int l) {
-    using R = RotPlan<L>;
-    if constexpr (I < R::NI) {
-        if constexpr (R::owner(I) == W) rot_item<L, BACK, R::item_m(I), R::item_u(I), R::j0(W, R::item_m(I))>(s, c, l);
-        rot_items<L, BACK, W, I + 1>(s, c, l);
-    }
-}
-template <int L, bool BACK, int W = 0>
-__device__ __forceinline__ void rot_wave(Lds<float, L> &s, const RotLane<L> &c, int w, int l) {
-    if constexpr (W < kWaves) {
-        if (w == W) {
-            rot_items<L, BACK, W, 0>(s, c, l);
-            if (W == kWaves - 1 && l < 16) {  // m = 0: R = 1
-                float2 v = BACK ? s.buf[l][0] : s.xs[l][0];
-                if (BACK && c.conj_mq && c.mq) v.y = -v.y;
-                (BACK ? s.xs : s.buf)[l][0] = v;
+// order M of one row and one mu2; jt: J, row k > 0 times sqrt(2)
+template <typename T, int L, int M, bool BACK>
+__device__ __forceinline__ void rot_fold(Lds<T, L, true> &s, const T *__restrict__ jt, int row, int mu) {
+    using C = typename Ty<T>::c;
+    constexpr int NM = Plan<L>::nmu(M), P0 = Plan<L>::poff(M) + M * NM, W = M + 1;
+    constexpr bool CH = Lds<T, L, true>::kChop;
+    constexpr int A0 = CH && !BACK ? 1 : 0, B0 = CH && BACK ? 1 : 0;
+    const T *J = jt + M * (M + 1) * (2 * M + 1) / 6;
+    const int p = row & 7;
+    const bool mq = row >= 8;
+    const T sg = ((M & 1) && mq) ? (T)-1 : (T)1;
+    const C *src = s.buf[row] + P0 + mu;
+    const int in = BACK && mq ? -NM : NM, out = !BACK && mq ? -NM : NM;
+    C tp[W], tm[W];
+    tp[0] = tm[0] = src[0];
+    steps<1, W>([&](auto A) {
+        constexpr int a = A.value;
+        const C x = src[a * in], y = src[-a * in];
+        C u, v;
+        u.x = x.x + y.x, u.y = x.y + y.y;
+        v.x = x.x - y.x, v.y = x.y - y.y;
+        tp[a] = times_i<BACK ? -a : a>((a & 1) ? v : u);
+        tm[a] = times_i<BACK ? -a : a>((a & 1) ? u : v);
+    });
+    C pc[W], ps[W];
+    steps<0, W>([&](auto K) {
+        constexpr int k = K.value;
+        C ue, uo;
+        ue.x = ue.y = uo.x = uo.y = (T)0;
+        steps<A0, W>([&](auto A) {
+            constexpr int a = A.value;
+            if constexpr ((k > 0 || ((M + a) & 1) == 0) && (a > 0 || ((M + k) & 1) == 0)) {
+                const C x = ((M + k) & 1) ? tm[a] : tp[a];
+                C &u = (a & 1) ? uo : ue;
+                u.x = fma(J[k * W + a], x.x, u.x);
+                u.y = fma(J[k * W + a], x.y, u.y);
             }
+        });
+        if constexpr (k == 0) {
+            pc[0].x = sg * ue.x, pc[0].y = sg * ue.y;
+            ps[0].x = sg * uo.x, ps[0].y = sg * uo.y;
         } else {
-            rot_wave<L, BACK, W + 1>(s, c, w, l);
+            const T ct = sg * s.trig[p][0][k], st = sg * s.trig[p][1][k];
+            pc[k].x = ct * ue.x + st * uo.y;
+            pc[k].y = ct * ue.y - st * uo.x;
+            ps[k].x = ct * uo.x + st * ue.y;
+            ps[k].y = ct * uo.y - st * ue.x;
         }
+    });
+    const bool cj = BACK && mq && (s.flag[p] & 3) == 3;  // q == -q on a Nyquist plane
+    C *dst = s.buf[row] + P0 + mu;
+    steps<B0, W>([&](auto B) {
+        constexpr int b = B.value;
+        C ev, od;
+        ev.x = ev.y = od.x = od.y = (T)0;
+        if constexpr (A0 == 1) {
+            const T d = sg * s.d0[p][M * (M + 1) / 2 + b];
+            const C x = times_i<b>(tp[0]);
+            C &u = (M & 1) ? od : ev;
+            u.x = d * x.x, u.y = d * x.y;
+        }
+        steps<0, W>([&](auto K) {
+            constexpr int k = K.value;
+            if constexpr ((k > 0 || ((M + b) & 1) == 0) && (b > 0 || ((M + k) & 1) == 0)) {
+                const C x = (b & 1) ? ps[k] : pc[k];
+                C &u = (k & 1) ? od : ev;
+                u.x = fma(J[k * W + b], x.x, u.x);
+                u.y = fma(J[k * W + b], x.y, u.y);
+            }
+        });
+        C f, g;
+        f.x = ev.x + od.x, f.y = ev.y + od.y;
+        g.x = ev.x - od.x, g.y = ev.y - od.y;
+        f = times_i<BACK ? b : -b>(f);
+        g = times_i<(BACK ? -b : b) + 2 * M>(g);
+        if constexpr (BACK && b > 0) {
+            const C e = s.ph[p][b];
+            const C f0 = f, g0 = g;
+            f.x = f0.x * e.x - f0.y * e.y;
+            f.y = f0.x * e.y + f0.y * e.x;
+            g.x = g0.x * e.x + g0.y * e.y;
+            g.y = g0.y * e.x - g0.x * e.y;
+        }
+        if constexpr (BACK) {
+            if (cj) f.y = -f.y, g.y = -g.y;
+        }
+        dst[b * out] = f;
+        if constexpr (b > 0) dst[-b * out] = g;
+    });
+    if constexpr (B0 == 1) {
+        C o;
+        o.x = o.y = (T)0;
+        steps<0, W>([&](auto B) {
+            constexpr int b = B.value;
+            const T d = s.d0[p][M * (M + 1) / 2 + b];
+            const C x = times_i<b>(tp[b]);
+            o.x = fma(d, x.x, o.x);
+            o.y = fma(d, x.y, o.y);
+        });
+        o.x *= sg, o.y *= cj ? -sg : sg;
+        dst[0] = o;
+    }
+}
+
+// wave R has order L - R, the last one all below too; lane: row l & 15, mu2 = l >> 4.  (Waves of different work,
+// but several tiles share a SIMD: other waves for it in every other tile made no difference.)
+template <typename T, int L, bool BACK, int R, int M>
+__device__ __forceinline__ void rot_fold_role(Lds<T, L, true> &s, const T *__restrict__ jt, int l) {
+    if constexpr (M == 0) {
+        if (BACK && l >= 8 && l < 16 && (s.flag[l & 7] & 3) == 3) s.buf[l][0].y = -s.buf[l][0].y;  // R = 1
+    } else if constexpr (M > 0) {
+        if ((l >> 4) < Plan<L>::nmu(M)) rot_fold<T, L, M, BACK>(s, jt, l & 15, l >> 4);
+    }
+    if constexpr (R == kWaves - 1 && M > 0) rot_fold_role<T, L, BACK, R, M - 1>(s, jt, l);
+}
+template <typename T, int L, bool BACK, int R = 0>
+__device__ __forceinline__ void rot_fold_all(Lds<T, L, true> &s, const T *__restrict__ jt, int w, int l) {
+    if constexpr (R < kWaves) {
+        if (w == R) rot_fold_role<T, L, BACK, R, L - R>(s, jt, l);
+        else rot_fold_all<T, L, BACK, R + 1>(s, jt, w, l);
     }
 }
 
@@ -530,8 +564,8 @@ __device__ __forceinline__ void load_x(T *x, const typename Ty<T>::c *own, const
 // 4 rr + q (OZ row 4 NB + rr; q = re lo, im lo, re hi, im hi).  Through the wave's scratch
 // lane l then takes (side, pair) row ps = l & 15 and OZ row 4 NB + (l >> 4):
 // gamma = (1 - alpha) lo + alpha hi, chopped, into the row's entry of that OZ row.
-template <typename T, int L, int KHI, int NB>
-__device__ __forceinline__ void gamma_store(typename Ty<T>::acc d, Lds<T, L> &s, T *scr, T al, T be, int l) {
+template <typename T, int L, int KHI, int NB, typename S>
+__device__ __forceinline__ void gamma_store(typename Ty<T>::acc d, S &s, T *scr, T al, T be, int l) {
     using C = typename Ty<T>::c;
     constexpr int SS = scr_stride<T>();
     constexpr int r0 = Plan<L>::row(KHI, 4 * NB), r1 = Plan<L>::row(KHI, 4 * NB + 1);
@@ -555,16 +589,16 @@ __device__ __forceinline__ void gamma_store(typename Ty<T>::acc d, Lds<T, L> &s,
     wave_sync();  // the scratch is read before the next block writes it
 }
 
-template <typename T, int L, int KHI, int... NB>
-__device__ __forceinline__ void store_all(typename Ty<T>::acc *acc, Lds<T, L> &s, T *scr, T al, T be, int l,
+template <typename T, int L, int KHI, typename S, int... NB>
+__device__ __forceinline__ void store_all(typename Ty<T>::acc *acc, S &s, T *scr, T al, T be, int l,
                                           std::integer_sequence<int, NB...>) {
     (gamma_store<T, L, KHI, NB>(acc[NB], s, scr, al, be, l), ...);
 }
 
 // blocks khi = KHI, KHI + kWaves, ... (the blocks of one wave; blocks are independent: block
 // khi reads and writes only the entries (., khi, .) of the rows)
-template <typename T, int L, int KHI>
-__device__ __forceinline__ void oz_blocks(Lds<T, L> &s, const T *__restrict__ fr, T *scr, T al, T be, int l) {
+template <typename T, int L, int KHI, typename S>
+__device__ __forceinline__ void oz_blocks(S &s, const T *__restrict__ fr, T *scr, T al, T be, int l) {
     using P = Plan<L>;
     using A = typename Ty<T>::acc;
     constexpr int NKB = P::nkb(KHI), NNB = P::nnb(KHI), F0 = P::foff(KHI);
@@ -590,8 +624,8 @@ __device__ __forceinline__ void oz_blocks(Lds<T, L> &s, const T *__restrict__ fr
 // BF16 contraction of block khi (FP32 rotations and epilogue): A (16 x 32) lane l holds row
 // l & 15, k = 8 (l >> 4) + j: column 16 kb + 4 (l >> 4) + (j >> 1), re (j even) or im; B the
 // same k, column l & 15; D as in the FP32 form.
-template <int L, int KHI>
-__device__ __forceinline__ void oz_blocks_bf(Lds<float, L> &s, const bf16x8 *__restrict__ fr,
+template <int L, int KHI, typename S>
+__device__ __forceinline__ void oz_blocks_bf(S &s, const bf16x8 *__restrict__ fr,
                                              const int *__restrict__ colent, float *scr, float al, float be, int l) {
     using P = Plan<L>;
     constexpr int NKB = P::nkb32(KHI), NNB = P::nnb(KHI), F0 = P::foff32(KHI);
@@ -620,8 +654,8 @@ __device__ __forceinline__ void oz_blocks_bf(Lds<float, L> &s, const bf16x8 *__r
     if constexpr (KHI + kWaves <= L) oz_blocks_bf<L, KHI + kWaves>(s, fr, colent, scr, al, be, l);
 }
 
-template <typename T, int L, bool BF, int W0>
-__device__ __forceinline__ void oz_wave(Lds<T, L> &s, const OzmArgs<T> &a, size_t iv, T *scr, T al, T be, int w,
+template <typename T, int L, bool BF, int W0, typename S>
+__device__ __forceinline__ void oz_wave(S &s, const OzmArgs<T> &a, size_t iv, T *scr, T al, T be, int w,
                                         int l) {
     if constexpr (W0 < kWaves && -L + W0 <= L) {
         if (w == W0) {
@@ -635,10 +669,11 @@ __device__ __forceinline__ void oz_wave(Lds<T, L> &s, const OzmArgs<T> &a, size_
 
 // ---- packed records (packed.h).  kind 0: one projection; 1: p(m, mup, 0), mup > 0, which gives
 // p(m, -mup, 0)(q) = (-1)^mup conj p(m, mup, 0)(-q) as well; 2: p(m, 0, 0) + i p(m + 1, 0, 0).
-// Into the rows of q and -q of pair pr, in FP32 times exp(-i mup phi) (see rot_class).
-template <typename T, int L>
-__device__ __forceinline__ void unpack(int d, typename Ty<T>::c xq, typename Ty<T>::c xm, Lds<T, L> &s, int pr) {
+// Into the rows of q and -q of pair pr, for folded rotations times exp(-i mup phi).
+template <typename T, int L, bool FOLD>
+__device__ __forceinline__ void unpack(int d, typename Ty<T>::c xq, typename Ty<T>::c xm, Lds<T, L, FOLD> &s, int pr) {
     using C = typename Ty<T>::c;
+    auto *xs = s.x();
     const int ip = d & 255, ip2 = (d >> 8) & 255, kind = (d >> 16) & 3, mup = (d >> 20) - 16;
     if (kind == 2) {  // mup = 0: no phase
         C e, o;
@@ -646,17 +681,17 @@ __device__ __forceinline__ void unpack(int d, typename Ty<T>::c xq, typename Ty<
         e.y = (T)0.5 * (xq.y - xm.y);
         o.x = (T)0.5 * (xq.y + xm.y);
         o.y = (T)-0.5 * (xq.x - xm.x);
-        s.xs[pr][ip] = e;
+        xs[pr][ip] = e;
         e.y = -e.y;
-        s.xs[8 + pr][ip] = e;
+        xs[8 + pr][ip] = e;
         if (ip2 != 255) {
-            s.xs[pr][ip2] = o;
+            xs[pr][ip2] = o;
             o.y = -o.y;
-            s.xs[8 + pr][ip2] = o;
+            xs[8 + pr][ip2] = o;
         }
         return;
     }
-    if constexpr (sizeof(T) == 4) {
+    if constexpr (FOLD) {
         const C z = s.ph[pr][mup < 0 ? -mup : mup];
         const T ex = z.x, ey = mup < 0 ? z.y : -z.y;
         const C u = xq, v = xm;
@@ -665,33 +700,34 @@ __device__ __forceinline__ void unpack(int d, typename Ty<T>::c xq, typename Ty<
         xm.x = v.x * ex - v.y * ey;
         xm.y = v.x * ey + v.y * ex;
     }
-    s.xs[pr][ip] = xq;
-    s.xs[8 + pr][ip] = xm;
+    xs[pr][ip] = xq;
+    xs[8 + pr][ip] = xm;
     if (kind == 1) {
         const T sg = (mup & 1) ? (T)-1 : (T)1;
         C c;
         c.x = sg * xm.x;
         c.y = -sg * xm.y;
-        s.xs[pr][ip2] = c;
+        xs[pr][ip2] = c;
         c.x = sg * xq.x;
         c.y = -sg * xq.y;
-        s.xs[8 + pr][ip2] = c;
+        xs[8 + pr][ip2] = c;
     }
 }
 
 // The part of the rotated-back outputs that the final pass reads, i.e. the projections of the real
 // part: p(m, mup, 0) <- (p(m, mup, 0)(q) + (-1)^mup conj p(m, -mup, 0)(-q)) / 2.  rq, rm: the rows
 // of q and -q, both the second's where q == -q (the store rule).
-template <typename T, int L>
-__device__ __forceinline__ void pack_out(int d, typename Ty<T>::c &oq, typename Ty<T>::c &om, const Lds<T, L> &s,
+template <typename T, int L, bool FOLD>
+__device__ __forceinline__ void pack_out(int d, typename Ty<T>::c &oq, typename Ty<T>::c &om, const Lds<T, L, FOLD> &s,
                                          int rq, int rm) {
     using C = typename Ty<T>::c;
     const int ip = d & 255, ip2 = (d >> 8) & 255, kind = (d >> 16) & 3, mup = (d >> 20) - 16;
-    oq = s.xs[rq][ip];
-    om = s.xs[rm][ip];
+    auto *xs = s.x();
+    oq = xs[rq][ip];
+    om = xs[rm][ip];
     if (kind == 1) {
         const T sg = (mup & 1) ? (T)-1 : (T)1;
-        const C u = s.xs[rm][ip2], v = s.xs[rq][ip2];
+        const C u = xs[rm][ip2], v = xs[rq][ip2];
         oq.x = (T)0.5 * (oq.x + sg * u.x);
         oq.y = (T)0.5 * (oq.y - sg * u.y);
         om.x = (T)0.5 * (om.x + sg * v.x);
@@ -700,8 +736,8 @@ __device__ __forceinline__ void pack_out(int d, typename Ty<T>::c &oq, typename 
         C o1, o2;
         o1.x = o1.y = o2.x = o2.y = (T)0;
         if (ip2 != 255) {
-            o1 = s.xs[rq][ip2];
-            o2 = s.xs[rm][ip2];
+            o1 = xs[rq][ip2];
+            o2 = xs[rm][ip2];
         }
         C e, o;  // of q; conjugated, of -q
         e.x = (T)0.5 * (oq.x + om.x);
@@ -715,21 +751,28 @@ __device__ __forceinline__ void pack_out(int d, typename Ty<T>::c &oq, typename 
     }
 }
 
-// FP32: at least 5 waves per SIMD (96 registers; at 6 or 7 it spills: 128^3, mmax 5 1.63, 2.04 and 2.23 ms)
-template <typename T, int L, bool BF, bool PACK>
-__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 5 : 1, 8))) void ozm(typename Ty<T>::c *__restrict__ proj, OzmArgs<T> a) {
+// Waves per SIMD asked for with folded rotations: FP32 5 (it gets 7 at mmax 5, 8 below; more makes no
+// difference), FP64 5 up to mmax 4, 4 at mmax 5 (without asking it gets 4 and 4: 96^3, mmax 3 453 against 379 us,
+// 128^3, mmax 5 2.67 against 2.64 ms; 5 at mmax 5 spills, 2.95 ms, and so does 4 at mmax 6).
+template <typename T, int L, bool FOLD> constexpr int ozm_waves() {
+    return !FOLD ? 1 : (sizeof(T) == 4 || L <= 4 ? 5 : (L == 5 ? 4 : 1));
+}
+template <typename T, int L, bool BF, bool PACK, bool FOLD>
+__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(ozm_waves<T, L, FOLD>(), 8)))
+void ozm(typename Ty<T>::c *__restrict__ proj, OzmArgs<T> a) {
     using P = Plan<L>;
     using C = typename Ty<T>::c;
     constexpr int KP = P::kp, NP = P::np;
     extern __shared__ __align__(16) unsigned char smem[];
-    Lds<T, L> &s = *reinterpret_cast<Lds<T, L> *>(smem);
+    Lds<T, L, FOLD> &s = *reinterpret_cast<Lds<T, L, FOLD> *>(smem);
+    auto *xs = s.x();
     const int tid = threadIdx.x, l = tid & 63, w = tid >> 6;
     const int p = l & 7, j = l >> 3;
     // XCD-aware order: consecutive workgroups go to different XCDs, so each XCD takes a
     // contiguous range of tiles (tiles of one interval share its c fragments in that L2)
     const int b = blockIdx.x;
-    const int tile = (b & 7) * a.per + (b >> 3);
-    if (tile >= a.ntiles) return;
+    const int local = (b & 7) * a.per + (b >> 3), tile = a.tile0 + local;
+    if (local >= a.ntiles) return;
     const TilePair *tps = a.tpair + (size_t)tile * 8;
     const int iq = tps[0].iq;  // the same for the tile's pairs
     // PACK: the records of q and -q, two entries (FP32, whole 16-byte words) or one per access, all
@@ -749,7 +792,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(siz
             pb[k] = reinterpret_cast<const Vec *>(proj + (size_t)tps[pr].gmq * NPK)[e];
         }
     }
-    if (tid < 16) {  // lanes 0-7: theta, 8-15: phi (FP32: phi - pi/2) of the pairs
+    if (tid < 16) {  // lanes 0-7: theta, 8-15: phi of the pairs
         const TilePair tp = tps[p];
         const bool phi = tid >= 8;
         if (!phi) {
@@ -761,8 +804,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(siz
             abv.y = (T)(1.0 - tp.al);
             s.ab[p] = abv;
         }
-        const double pc = sizeof(T) == 4 ? tp.sp : tp.cp, ps = sizeof(T) == 4 ? -tp.cp : tp.sp;
-        const double c1 = phi ? pc : tp.ct, s1 = phi ? ps : tp.st;
+        const double c1 = phi ? tp.cp : tp.ct, s1 = phi ? tp.sp : tp.st;
         double ck = 1.0, sk = 0.0;
         for (int k = 0; k < KP; k++) {
             if (phi) {
@@ -779,14 +821,24 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(siz
             ck = nc;
         }
     }
-    [[maybe_unused]] RotLane<sizeof(T) == 4 ? L : 0> rl;
-    if constexpr (sizeof(T) == 4) {
-#pragma unroll
-        for (int q = 0; q < RotPlan<L>::NJ; q++) rl.j[q] = a.jtab[(w * RotPlan<L>::NJ + q) * 64 + l];
-        rl.sg = (((l & 15) >> 2) + (l >> 4)) & 1 ? -1.0f : 1.0f;
-        rl.mq = (l & 15) >= 8;
-    }
     __syncthreads();
+    if constexpr (FOLD && sizeof(T) == 8) {
+        for (int i = tid; i < 8 * s.nd; i += 64 * kWaves) {
+            const int e = i >> 3;
+            int m = 0;
+#pragma unroll
+            for (int k = 1; k <= L; k++) m += e >= k * (k + 1) / 2 ? 1 : 0;
+            const int bb = e - m * (m + 1) / 2;
+            const T *F = a.ftab + (P::roff(m) + m * (2 * m + 1) + bb + m) * KP, *tr = s.trig[i & 7][bb & 1];
+            T v = (T)0;
+#pragma unroll
+            for (int k = 0; k < KP; k++) v = fma(F[k], tr[k], v);
+            C R;
+            R.x = v;
+            R.y = (T)0;
+            s.d0[i & 7][e] = chop_R(R).x;
+        }
+    }
     if constexpr (PACK) {
 #pragma unroll
         for (int k = 0; k < NIT; k++) {
@@ -798,8 +850,8 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(siz
         }
         __syncthreads();
     } else {
-        // X of the 16 (side, pair) rows, each row one contiguous record; in FP32 times
-        // exp(-i mup phi) for the factored rotation, two elements per 16-byte access when the
+        // X of the 16 (side, pair) rows, each row one contiguous record; for folded rotations
+        // times exp(-i mup phi), in FP32 two elements per 16-byte access when the
         // records are a whole number of 16-byte words
         if constexpr (sizeof(T) == 4 && NP % 2 == 0) {
             constexpr int NP2 = NP / 2;
@@ -816,14 +868,14 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(siz
                     out[h].x = ux * ex - uy * ey;
                     out[h].y = ux * ey + uy * ex;
                 }
-                s.xs[r][e] = out[0];
-                s.xs[r][e + 1] = out[1];
+                xs[r][e] = out[0];
+                xs[r][e + 1] = out[1];
             }
         } else {
             for (int i = tid; i < 16 * NP; i += 64 * kWaves) {
                 const int r = i / NP, e = i - r * NP;
                 C x = proj[(size_t)s.g[r] * NP + e];
-                if constexpr (sizeof(T) == 4) {
+                if constexpr (FOLD) {
                     const int mup = a.pmup[e];
                     const C z = s.ph[r & 7][mup < 0 ? -mup : mup];
                     const T ex = z.x, ey = mup < 0 ? z.y : -z.y;
@@ -831,32 +883,21 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(siz
                     x.x = u.x * ex - u.y * ey;
                     x.y = u.x * ey + u.y * ex;
                 }
-                s.xs[r][e] = x;
+                xs[r][e] = x;
             }
         }
         __syncthreads();
     }
-    if constexpr (sizeof(T) == 4) {
-#pragma unroll
-        for (int r = 0; r < RotPlan<L>::RN; r++) {
-            const int k = 4 * r + (l >> 4) - L, ak = k < 0 ? -k : (k > L ? L : k);
-            rl.th[r] = make_float2(s.trig[p][0][ak], k < 0 ? s.trig[p][1][ak] : -s.trig[p][1][ak]);
-            const float2 z = s.ph[p][ak];
-            rl.ph[r] = make_float2(z.x, k < 0 ? -z.y : z.y);
-        }
-        rl.conj_mq = (s.flag[p] & 3) == 3;
-        rot_wave<L, false>(s, rl, w, l);
-    } else {
-        rot_all<T, L, P::nclass, false>(a, s, w, p, j);
-    }
+    if constexpr (FOLD) rot_fold_all<T, L, false>(s, a.jfold, w, l);
+    else rot_all<T, L, P::nclass, false>(a, s, w, p, j);
     __syncthreads();
     {
         const C abv = s.ab[l & 7];  // the pair of row l & 15
-        T *scr = reinterpret_cast<T *>(&s.xs[0][0]) + w * 16 * scr_stride<T>();
+        T *scr = s.scr() + w * 16 * scr_stride<T>();
         oz_wave<T, L, BF, 0>(s, a, (size_t)(iq - 1), scr, abv.x, abv.y, w, l);
     }
     __syncthreads();
-    if constexpr (sizeof(T) == 4) rot_wave<L, true>(s, rl, w, l);
+    if constexpr (FOLD) rot_fold_all<T, L, true>(s, a.jfold, w, l);
     else rot_all<T, L, P::nclass, true>(a, s, w, p, j);
     __syncthreads();
     // store rule (:648-656): both sides of real pairs; for q == -q only the -q side
@@ -878,7 +919,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(siz
             const int r = i / NP2, e = 2 * (i - r * NP2);
             const int f = s.flag[r & 7];
             if ((f & 4) || (r < 8 && (f & 1))) continue;
-            const C u0 = s.xs[r][e], u1 = s.xs[r][e + 1];
+            const C u0 = xs[r][e], u1 = xs[r][e + 1];
             reinterpret_cast<float4 *>(proj + (size_t)s.g[r] * NP)[e / 2] = make_float4(u0.x, u0.y, u1.x, u1.y);
         }
     } else {
@@ -886,9 +927,52 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(siz
             const int r = i / NP, e = i - r * NP;
             const int f = s.flag[r & 7];
             if ((f & 4) || (r < 8 && (f & 1))) continue;
-            proj[(size_t)s.g[r] * NP + e] = s.xs[r][e];
+            proj[(size_t)s.g[r] * NP + e] = xs[r][e];
         }
     }
+}
+
+// Which pairs have a rotation matrix with a chopped entry R(mup, .), mup > 0, that the chop changes: a
+// component below FLT_EPSILON of an entry above 1e-13 (what it changes in a smaller one is below the rounding
+// of FP64).  A little above FLT_EPSILON, so that no rounding of d or of the phases decides.
+template <int KP>
+__global__ void chopped_pairs(const int *__restrict__ pq, int n, int nx, int ny, const double *__restrict__ kx,
+                              const double *__restrict__ ky, const double *__restrict__ kz,
+                              const double *__restrict__ ftab, int L, int *__restrict__ flag) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const int g = pq[i], ix = g % nx, iy = (g / nx) % ny, iz = g / (nx * ny);
+    const double q0 = kx[ix], q1 = ky[iy], q2 = kz[iz], rxy = sqrt(q0 * q0 + q1 * q1), qn = sqrt(rxy * rxy + q2 * q2);
+    const double ct = qn > 0.0 ? q2 / qn : 1.0, st = qn > 0.0 ? rxy / qn : 0.0;
+    const double cp = rxy > 0.0 ? q0 / rxy : 1.0, sp = rxy > 0.0 ? q1 / rxy : 0.0;
+    double tr[2][KP];
+    tr[0][0] = 1.0, tr[1][0] = 0.0;
+#pragma unroll
+    for (int k = 1; k < KP; k++) {
+        tr[0][k] = tr[0][k - 1] * ct - tr[1][k - 1] * st;
+        tr[1][k] = tr[1][k - 1] * ct + tr[0][k - 1] * st;
+    }
+    double ca = 1.0, sa = 0.0;
+    bool hit = false;
+    for (int a = 1; a <= L; a++) {
+        const double nc = ca * cp - sa * sp;
+        sa = sa * cp + ca * sp;
+        ca = nc;
+        const double low = fmin(fabs(ca), fabs(sa));
+        for (int m = a; m <= L; m++)
+            for (int b = -m; b <= m; b++) {
+                const double *F = ftab + (size_t)(m * (4 * m * m - 1) / 3 + (a + m) * (2 * m + 1) + b + m) * KP;
+                double v0 = 0.0, v1 = 0.0;
+#pragma unroll
+                for (int k = 0; k < KP; k++) {
+                    v0 += F[k] * tr[0][k];
+                    v1 += F[k] * tr[1][k];
+                }
+                const double d = fabs(((a - b) & 1) ? v1 : v0);
+                hit = hit || (d > 1e-13 && d * low < 1.0001 * (double)FLT_EPSILON);
+            }
+    }
+    flag[i] = hit ? 1 : 0;
 }
 
 // ---- host side ---------------------------------------------------------------------
@@ -910,8 +994,6 @@ double textbook_d_h(int j, int mp, int m, double beta) {
 
 struct HostPlan {
     int L, np, kp, nclass, nfrag, nfrag32;
-    int nj = 1;
-    std::vector<int> jm, js;  // [wave][nj] order and step of each J entry of the FP32 rotations (order 0: none)
     std::vector<int> col[2 * MDFT_MAX_MMAX + 1], row[2 * MDFT_MAX_MMAX + 1];
     std::vector<int> nkb, nnb, foff, ncol, nkb32, foff32;
 };
@@ -925,16 +1007,6 @@ template <int L> HostPlan host_plan() {
     h.nclass = P::nclass;
     h.nfrag = P::nfrag;
     h.nfrag32 = P::nfrag32;
-    using R = RotPlan<L>;
-    h.nj = R::NJ;
-    h.jm.assign(kWaves * R::NJ, 0);
-    h.js.assign(kWaves * R::NJ, 0);
-    for (int w = 0; w < kWaves; w++)
-        for (int m = 1; m <= L; m++)
-            for (int q = 0; R::has(w, m) && q < R::ns(m); q++) {
-                h.jm[w * R::NJ + R::j0(w, m) + q] = m;
-                h.js[w * R::NJ + R::j0(w, m) + q] = R::s0(m) + q;
-            }
     for (int khi = -L; khi <= L; khi++) {
         for (int c = 0; c < 32; c++) h.col[khi + L].push_back(P::col(khi, c));
         for (int r = 0; r < 4 * P::nnb(khi); r++) h.row[khi + L].push_back(P::row(khi, r));
@@ -960,10 +1032,20 @@ HostPlan host_plan_of(int L) {
     }
 }
 
+template <typename T, int L, bool BF, bool PACK, bool FOLD>
+hipError_t launch_tiles(mdft_ctx *c, typename Ty<T>::c *proj, OzmArgs<T> &a, int tile0, int ntiles) {
+    if (ntiles == 0) return hipSuccess;
+    a.tile0 = tile0;
+    a.ntiles = ntiles;
+    a.per = (ntiles + 7) / 8;
+    const size_t lds = sizeof(Lds<T, L, FOLD>);
+    if (lds > c->lds_limit) return hipErrorInvalidConfiguration;
+    hipLaunchKernelGGL((ozm<T, L, BF, PACK, FOLD>), dim3((unsigned)(8 * a.per)), dim3(64 * kWaves), lds, c->stream, proj, a);
+    return hipGetLastError();
+}
+
 template <typename T, int L, bool BF, bool PACK = false> hipError_t launch_ozm_t(mdft_ctx *c, typename Ty<T>::c *proj) {
     OzmArgs<T> a;
-    a.ntiles = c->pairs.ntiles;
-    a.per = (c->pairs.ntiles + 7) / 8;
     a.tpair = c->pairs.tpair;
     a.pmup = c->d_pmup;
     a.pack = c->d_ozm_pack;
@@ -973,18 +1055,19 @@ template <typename T, int L, bool BF, bool PACK = false> hipError_t launch_ozm_t
     a.ftab = static_cast<const T *>(c->d_ozm_ftab);
     a.units = reinterpret_cast<const int4 *>(c->d_ozm_units);
     a.rlen = c->d_ozm_rlen;
-    a.jtab = c->d_ozm_jtab;
+    a.jfold = static_cast<const T *>(c->d_ozm_jfold);
     for (int d = 0; d < 2; d++)
         for (int wv = 0; wv < kWaves; wv++)
             for (int k = 0; k < 4; k++) {
                 a.cr0[d][wv][k] = c->ozm_cr0[d][wv][k];
                 a.cnr[d][wv][k] = c->ozm_cnr[d][wv][k];
             }
-    if (a.ntiles == 0) return hipSuccess;
-    const size_t lds = sizeof(Lds<T, L>);
-    if (lds > c->lds_limit) return hipErrorInvalidConfiguration;
-    hipLaunchKernelGGL((ozm<T, L, BF, PACK>), dim3((unsigned)(8 * a.per)), dim3(64 * kWaves), lds, c->stream, proj, a);
-    return hipGetLastError();
+    const int nt = c->pairs.ntiles, nf = sizeof(T) == 4 ? nt : (L >= kFold64 ? c->pairs.nfold : 0);
+    hipError_t e = hipSuccess;
+    if constexpr (sizeof(T) == 4 || L >= kFold64) e = launch_tiles<T, L, BF, PACK, true>(c, proj, a, 0, nf);
+    if constexpr (sizeof(T) == 8)
+        if (e == hipSuccess) e = launch_tiles<T, L, BF, PACK, false>(c, proj, a, nf, nt - nf);
+    return e;
 }
 
 template <typename T, bool BF> hipError_t launch_ozm_any(mdft_ctx *c, typename Ty<T>::c *proj) {
@@ -1025,13 +1108,13 @@ template <typename T> int upload_t(mdft_ctx *c, void **dst, const std::vector<do
 
 static size_t ozm_lds(int L, bool fp64) {
     switch (L) {
-        case 0: return fp64 ? sizeof(Lds<double, 0>) : sizeof(Lds<float, 0>);
-        case 1: return fp64 ? sizeof(Lds<double, 1>) : sizeof(Lds<float, 1>);
-        case 2: return fp64 ? sizeof(Lds<double, 2>) : sizeof(Lds<float, 2>);
-        case 3: return fp64 ? sizeof(Lds<double, 3>) : sizeof(Lds<float, 3>);
-        case 4: return fp64 ? sizeof(Lds<double, 4>) : sizeof(Lds<float, 4>);
-        case 5: return fp64 ? sizeof(Lds<double, 5>) : sizeof(Lds<float, 5>);
-        default: return fp64 ? sizeof(Lds<double, 6>) : sizeof(Lds<float, 6>);
+        case 0: return fp64 ? sizeof(Lds<double, 0, false>) : sizeof(Lds<float, 0, true>);
+        case 1: return fp64 ? sizeof(Lds<double, 1, false>) : sizeof(Lds<float, 1, true>);
+        case 2: return fp64 ? sizeof(Lds<double, 2, false>) : sizeof(Lds<float, 2, true>);
+        case 3: return fp64 ? sizeof(Lds<double, 3, false>) : sizeof(Lds<float, 3, true>);
+        case 4: return fp64 ? sizeof(Lds<double, 4, false>) : sizeof(Lds<float, 4, true>);
+        case 5: return fp64 ? sizeof(Lds<double, 5, false>) : sizeof(Lds<float, 5, true>);
+        default: return fp64 ? sizeof(Lds<double, 6, false>) : sizeof(Lds<float, 6, true>);
     }
 }
 
@@ -1073,18 +1156,13 @@ int ozm_setup(mdft_ctx *c) {
                 }
             }
     }
-    if (c->d.precision != MDFT_PREC_FP64) {
-        // J entries of the FP32 rotations: lane l of step s holds J_kb = d^m_{k,b}(pi/2), k + L = 4 s + (l >> 4) and
-        // b + L = 4 (i & 3) + (i >> 2), i = l & 15
-        std::vector<double> jt((size_t)kWaves * h.nj * 64, 0.0);
-        for (size_t e = 0; e < h.jm.size(); e++)
-            for (int l = 0; h.jm[e] > 0 && l < 64; l++) {
-                const int m = h.jm[e], i = l & 15, k = 4 * h.js[e] + (l >> 4) - L, b = 4 * (i & 3) + (i >> 2) - L;
-                if (std::abs(k) <= m && std::abs(b) <= m) jt[e * 64 + l] = textbook_d_h(m, k, b, hp);
-            }
-        void *p = nullptr;
-        const int rc = upload_t<float>(c, &p, jt);
-        c->d_ozm_jtab = static_cast<float *>(p);
+    {
+        std::vector<double> jf;
+        for (int m = 0; m <= L; m++)
+            for (int k = 0; k <= m; k++)
+                for (int x = 0; x <= m; x++) jf.push_back(textbook_d_h(m, k, x, hp) * (k ? sqrt(2.0) : 1.0));
+        const int rc = c->d.precision == MDFT_PREC_FP64 ? upload_t<double>(c, &c->d_ozm_jfold, jf)
+                                                        : upload_t<float>(c, &c->d_ozm_jfold, jf);
         if (rc != MDFT_OK) return rc;
     }
     auto nmu = [](int m) { return m / 2 + 1; };
@@ -1191,6 +1269,29 @@ int ozm_setup(mdft_ctx *c) {
     if (hipMemcpy(c->d_ozm_col, colent.data(), sizeof(int) * colent.size(), hipMemcpyHostToDevice) != hipSuccess)
         return MDFT_EHIP;
     return MDFT_OK;
+}
+
+// 1 for the pairs (pq: grid index of q) whose tiles keep the entry by entry rotations, which is
+// for the FP64 kernel with folded rotations; 0 otherwise
+int ozm_chopped(mdft_ctx *c, const std::vector<int> &pq, std::vector<int> &flag) {
+    const int n = (int)pq.size();
+    flag.assign(n, 0);
+    if (!ozm_supported(c) || c->d.precision != MDFT_PREC_FP64 || c->L < kFold64 || n == 0) return MDFT_OK;
+    int *d = nullptr;
+    if (dev_malloc(&d, 2 * sizeof(int) * (size_t)n) != hipSuccess) return MDFT_ENOMEM;
+    const double *ft = static_cast<const double *>(c->d_ozm_ftab);
+    hipError_t e = hipMemcpy(d, pq.data(), sizeof(int) * (size_t)n, hipMemcpyHostToDevice);
+    if (e == hipSuccess) {
+        const dim3 grid((unsigned)((n + 255) / 256)), block(256);
+        auto *kernel = c->L <= 3 ? chopped_pairs<4> : (c->L <= 5 ? chopped_pairs<6> : chopped_pairs<8>);
+        hipLaunchKernelGGL(kernel, grid, block, 0, c->stream, d, n, c->d.nx, c->d.ny, c->d_kx, c->d_ky, c->d_kz, ft,
+                           c->L, d + n);
+        e = hipGetLastError();
+    }
+    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+    if (e == hipSuccess) e = hipMemcpy(flag.data(), d + n, sizeof(int) * (size_t)n, hipMemcpyDeviceToHost);
+    (void)dev_free(d);
+    return e == hipSuccess ? MDFT_OK : MDFT_EHIP;
 }
 
 // B fragments of every interpolation interval (rows iq - 1 and iq of the relayouted c(k)

@@ -66,6 +66,7 @@ struct PairSchedule {
     int ntiles = 0;           // tiles of at most 8 pairs of one chunk (the matrix-core q-space kernel)
     int *tstart = nullptr;    // first pair of each tile
     int *tinfo = nullptr;     // pair count | iq << 4 of each tile
+    int nfold = 0;            // the first tiles, whose pairs have no chopped entries beyond mup = 0
     TilePair *tpair = nullptr;  // [ntiles][8] the tiles' pairs, padded (flag bit 2 marks padding)
 };
 
@@ -124,7 +125,7 @@ struct mdft_ctx {
     void *d_a2p_img[4] = {};      // angl2proj_t's weights: FP32, FP64, packed FP32, packed FP64
     bool packed = false;          // set during an evaluation whose projection field is packed (packed.h)
     int npk = 0;                  // packed projections per point
-    float *d_ozm_jtab = nullptr;  // FP32: d^m(pi/2) entries of the q-space kernel's rotations
+    void *d_ozm_jfold = nullptr;  // d^m(pi/2) of the q-space kernel's folded rotations
     int *d_ozm_pack = nullptr;    // packed entries of the q-space kernel
     bool vext32_ok = false;       // d_vext32 holds the current vext
     size_t dpart_cap = 0;
@@ -166,6 +167,7 @@ hipError_t launch_fft3d_f32(mdft_ctx *c, float2 *proj, int sign, int batch = 0);
 hipError_t launch_oz_f64(mdft_ctx *c, double2 *proj);
 bool ozm_supported(const mdft_ctx *c);
 int ozm_setup(mdft_ctx *c);
+int ozm_chopped(mdft_ctx *c, const std::vector<int> &pq, std::vector<int> &flag);
 int ozm_frags(mdft_ctx *c, const std::vector<double2> &tab, int nq, int npc, const std::vector<int> &ia0);
 hipError_t launch_ozp_f64(mdft_ctx *c, double2 *proj);  // packed projections, mmax <= 2
 hipError_t launch_ozp_f32(mdft_ctx *c, float2 *proj);

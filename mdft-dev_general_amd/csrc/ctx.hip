@@ -492,6 +492,7 @@ int mdft_ctx_create(const mdft_desc *desc, mdft_ctx **out) {
             upload(c, &c->d_oz32_lanerow, lanerow.data(), lanerow.size()) != hipSuccess)
             return bad(MDFT_ENOMEM, "device allocation failed");
     }
+    if (log_setup(c) != MDFT_OK) return bad(MDFT_ENOMEM, "table of the logarithm");
     if (ozm_setup(c) != MDFT_OK) return bad(MDFT_ENOMEM, "matrix-core q-space tables");
     if (d.mrso == 2 && c->L <= 5 && d.precision != MDFT_PREC_BF16 && ozm_supported(c)) {
         const int npk[6] = {Packed<0>::np, Packed<1>::np, Packed<2>::np, Packed<3>::np, Packed<4>::np, Packed<5>::np};
@@ -532,7 +533,8 @@ void mdft_ctx_destroy(mdft_ctx *c) {
                     c->d_partials, c->d_slices, c->d_vpart, c->d_mpart, c->d_oz32_ftab, c->d_oz32_lanerow,
                     c->d_ozm_frag, c->d_ozm_frag16, c->d_ozm_col, c->d_ozm_ftab, c->d_ozm_units, c->d_ozm_rlen,
                     c->d_bf16_M, c->d_bf16_Q, c->d_chscale, c->d_adjscale, c->d_vscale, c->d_dpart, c->d_vext32,
-                    c->d_a2p_img[0], c->d_a2p_img[1], c->d_a2p_img[2], c->d_a2p_img[3], c->d_ozm_pack, c->d_ozm_jfold};
+                    c->d_a2p_img[0], c->d_a2p_img[1], c->d_a2p_img[2], c->d_a2p_img[3], c->d_ozm_pack, c->d_ozm_jfold,
+                    c->d_logt};
     for (void *b : bufs)
         if (b) (void)dev_free(b);
     free_pairs(c->pairs);

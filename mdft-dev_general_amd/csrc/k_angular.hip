@@ -662,21 +662,52 @@ __global__ __launch_bounds__(TH) void angl2proj_t(const double *__restrict__ xi,
     }
 }
 
+// ---- ln y, y > 0, by table (P. T. P. Tang, ACM Trans. Math. Softw. 16, 378 (1990)) ----------------
+// y = 2^k z, z in [1/2, 1); d the multiple of 1/256 next to 1 / c, c the multiple of 1/256 next to z;
+// r = z d - 1, |r| <= 0.005, all but exact in one fused operation; ln y = k ln 2 - ln d + ln(1 + r),
+// the last by its series to r^7.  k ln 2 and -ln d are split at 2^-42, so that their upper parts add
+// exactly (to 0 next to y = 1, where r is exact).  With the lower parts in the last sum: at most 0.57
+// units in the last place (60 million values against extended precision).
+constexpr int kLogC = 129;
+constexpr double kLn2Hi = 0x1.62e42fefa38p-1, kLn2Lo = 0x1.ef35793c7673p-45;
+struct LogTable {
+    double2 c[kLogC];  // d, upper part of -ln d for c = 1/2 + j / 256
+    double lo[kLogC];
+};
+__device__ __forceinline__ double log_table(double y, const LogTable &t) {
+    const double z = __builtin_amdgcn_frexp_mant(y);
+    const double k = (double)__builtin_amdgcn_frexp_exp(y);
+    // the upper word of 1/2 ends in 21 zero bits: 7 bits of the fraction, rounded (infinity: 128; NaN: limited)
+    const unsigned j0 = ((unsigned)__double2hiint(z) + 0x1000u) >> 13 & 0xffu, j = j0 < 128u ? j0 : 128u;
+    const double2 c = t.c[j];
+    const double r = fma(z, c.x, -1.0);
+    double p = fma(r, 1.0 / 7, -1.0 / 6);
+    p = fma(r, p, 1.0 / 5);
+    p = fma(r, p, -1.0 / 4);
+    p = fma(r, p, 1.0 / 3);
+    p = fma(r, p, -1.0 / 2);
+    const double h = fma(k, kLn2Hi, c.y), lo = fma(k, kLn2Lo, t.lo[j]);
+    const double s = h + r, e = (h - s) + r;
+    const double v = s + (e + fma(r * r, p, lo));
+    return y < HUGE_VAL ? v : y;
+}
+
 // Points per tile of final_t and its least waves per SIMD: elements for whole rounds of 256 threads
 // (330 x 6 = 7.7 rounds at mmax 5), as many as registers hold without spilling.  Measured, final
 // pass at 128^3, mmax 5: fast variant 4, 5, 6, 7, 8 points 3.58, 3.42, 3.38, 3.55, 4.52 ms; FP32
-// 4.54, 4.55, 3.85, 4.09, 3.97; FP64 5, 6, 7, 8 points 5.75, 5.59, 5.53, 5.81 ms (8 points at 3
-// waves); 100^3, mmax 4, FP64: 8 points at 4 waves 1.76, 9 at 3 waves 1.69 ms.
+// 4.54, 4.55, 3.85, 4.09, 3.97; FP64 6, 7, 8 points 4.32, 4.28, 4.69 ms; 100^3, mmax 4, FP64: 8, 9, 10
+// points 1.37, 1.35, 1.34 ms; 96^3, mmax 3: 15, 18, 21 points 444, 439, 436 us.  5 waves per SIMD with
+// smaller tiles: 5.97 ms, 1.84 ms, 456 us.
 template <int L, typename T> struct FinalShape {
     static constexpr int PT32 = L == 5 ? 6 : L == 4 ? 9 : L == 3 ? 24 : L == 2 ? 32 : L == 1 ? 128 : 256;
     static constexpr int PT64 = L == 5 ? 7 : L == 4 ? 9 : L == 3 ? 18 : L == 2 ? 32 : L == 1 ? 128 : 256;
     static constexpr int PT = sizeof(T) == 4 ? PT32 : PT64;
-    static constexpr int WAVES = sizeof(T) == 8 && L == 4 ? 3 : 4;
+    static constexpr int WAVES = 4;
 };
 
-// The fast variant is bound by HBM (15.3 GB at 128^3, mmax 5, in 3.38 ms: 4.5 TB/s; a plain copy
-// reaches 4.8).  FP64 (19.6 GB in 5.5 ms) is not: its logarithms and synthesis are 2.4 ms of vector
-// issue that 3 to 4 waves per SIMD do not hide wholly behind the loads.  The phi synthesis takes one
+// Bound by HBM: the fast variant moves 15.3 GB at 128^3, mmax 5, in 3.33 ms (4.6 TB/s; a plain copy
+// reaches 4.8), FP64 19.6 GB in 4.28 ms (4.6).  (FP64 with the library's logarithm, 1.4 ms of vector issue, took
+// 5.53 ms; 96^3, mmax 3 558 against 439 us, 75^3, mmax 2 152 against 115.)  The phi synthesis takes one
 // thread per (row, mu2), in place; with one thread per (row, phi, mu2), each reading 11 coefficients
 // and 11 twiddles from LDS for one output, the pass took 3.70 (fast) and 6.79 ms (FP64).
 //
@@ -692,7 +723,7 @@ template <int L, typename T> struct FinalShape {
 // memory operations issued after it, so the product operands loaded ahead stay in flight.  The
 // last tile of a grid that is not a whole number of tiles starts early, over points of the one
 // before it (whose dF is written twice, with the same values); those add nothing to the sums.
-template <int L, typename T, bool DOT32, bool PACK>
+template <int L, typename T, bool DOT32, bool PACK, bool EVAL = DOT32>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FinalShape<L, T>::WAVES, 8))) void final_t(
     const typename C2<T>::t *__restrict__ proj, const double *__restrict__ xi, const double *__restrict__ vext,
     double *__restrict__ df, double *__restrict__ partials, size_t N, AngTables t, FinalConsts k, int mode,
@@ -705,7 +736,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FinalS
     constexpr int NW = PACK ? Packed<L>::pair0 + L + 1 : NP;  // rows of the theta weights
     constexpr int ROW = R::ROW, RS = R::RS, NF = R::NF;
     constexpr int NPS = NP | 1;  // odd: the records of consecutive points in different banks
-    if constexpr (DOT32) mode = 0;
+    if constexpr (EVAL) mode = 0;
+    if constexpr (EVAL && !DOT32) {
+        xi32 = nullptr;
+        df32 = nullptr;
+    }
     __shared__ __align__(16) V Gm[PT * NPS];
     __shared__ T rows[NTH * PT * RS];  // row of (point, theta) at theta PT + point
     __shared__ V twpsi[NPSI * (H + 1)];  // (cos, sin)(2 pi mu2 ipsi / npsi) at [ipsi][mu2]
@@ -714,6 +749,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FinalS
     __shared__ T p2a[NW * NTH];
     __shared__ double wth[NTH];          // the weights depend on theta only
     __shared__ double sth[NTH];          // 1 / s of each theta
+    constexpr bool kLog = sizeof(T) == 8;
+    __shared__ std::conditional_t<kLog, LogTable, char> lt;  // FP64
     // projection index or packed entry of (m, mup, mu2), projection index of (m, -mup, 0), as bytes: the loaded index is then known to be small
     // and its products stay 24-bit multiplies (entries with m below the item's lowest m are never read)
     static_assert(R::NP <= 255, "projection indices are stored as bytes");
@@ -766,6 +803,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FinalS
         wth[i] = t.w[i * ROW];
         sth[i] = vsinv ? vsinv[i * ROW] : 1.0;
     }
+    if constexpr (kLog)
+        for (int i = tid; i < (int)(sizeof(LogTable) / sizeof(double)); i += kThreads) reinterpret_cast<double *>(&lt)[i] = t.logt[i];
     double fid = 0.0, fext = 0.0, fexc = 0.0;
     double d0 = 0.0, d1 = 0.0, d2 = 0.0;  // products of dF with the DotArgs vectors
     double dss = 0.0;                     // DOT32: the product of dF with itself
@@ -998,7 +1037,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(FinalS
                 const double ve = vr[q];
                 double gid = 0.0;
                 if (rho > DBL_EPSILON) {
-                    const double lg = log(x * x);  // ln(rho / rho0)
+                    double lg = 0.0;  // ln(rho / rho0)
+                    if constexpr (kLog) lg = log_table(x * x, lt);
                     fid += kT * dv * wio * (rho * lg - rho + rho0);
                     fext += dv * wio * rho * ve;
                     gid = wio * 2.0 * rho0 * x * (kT * lg + ve);
@@ -1114,6 +1154,23 @@ bool launch_a2p_t(mdft_ctx *c, const double *xi, typename C2<T>::t *proj, int fe
     }
 }
 
+// the table of log_table, built in extended precision
+int log_setup(mdft_ctx *c) {
+    LogTable h;
+    for (int j = 0; j < kLogC; j++) {
+        const double d = nearbyint(256.0 / (0.5 + j / 256.0)) / 256.0;
+        const long double l = -logl((long double)d);
+        const double hi = (double)(nearbyintl(l * 0x1p42L) * 0x1p-42L);
+        h.c[j] = make_double2(d, j == 0 ? -kLn2Hi : hi);
+        h.lo[j] = j == 0 ? -kLn2Lo : (double)(l - (long double)hi);
+    }
+    void *p = nullptr;
+    if (dev_malloc(&p, sizeof(h)) != hipSuccess) return MDFT_ENOMEM;
+    c->d_logt = p;
+    c->ang.logt = static_cast<const double *>(p);
+    return hipMemcpy(p, &h, sizeof(h), hipMemcpyHostToDevice) == hipSuccess ? MDFT_OK : MDFT_EHIP;
+}
+
 template <typename T, bool PACK = false>
 bool launch_final_t(mdft_ctx *c, const typename C2<T>::t *proj, const double *xi, double *df, int mode, FinalConsts k,
                     size_t npts = 0, size_t *grid_out = nullptr) {
@@ -1141,6 +1198,13 @@ bool launch_final_t(mdft_ctx *c, const typename C2<T>::t *proj, const double *xi
             } \
         } \
         const size_t nb = oversubscribed_grid(c, ntiles); \
+        if constexpr (PACK && sizeof(T) == 8) { \
+            if (mode == 0 && !c->df32 && !c->xi32) { \
+                if (grid_out) *grid_out = nb; \
+                hipLaunchKernelGGL((final_t<LL, T, false, true, true>), dim3((unsigned)nb), dim3(kThreads), 0, c->stream, proj, xi, c->d_vext, df, c->d_partials, npts, c->ang, k, 0, nullptr, c->vsinv, da, c->d_dpart, nullptr, nullptr); \
+                return true; \
+            } \
+        } \
         if (grid_out) *grid_out = nb; \
         hipLaunchKernelGGL((final_t<LL, T, false, PACK>), dim3((unsigned)nb), dim3(kThreads), 0, c->stream, proj, xi, c->d_vext, df, c->d_partials, npts, c->ang, k, mode, mode == 0 ? c->df32 : nullptr, mode == 0 ? c->vsinv : nullptr, da, c->d_dpart, mode == 0 ? c->xi32 : nullptr, nullptr); \
         return true; \

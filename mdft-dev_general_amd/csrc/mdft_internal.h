@@ -36,6 +36,7 @@ struct AngTables {
     const double *sps;   // [npsi] sin(2 pi k / npsi)
     const int *pidx;     // [(L+1)][2L+1][H+1] projection index of (m, mup, mu2)
     const int *pm, *pmup, *pmu;  // [np]
+    const double *logt;          // table of the final pass's logarithm
 };
 
 struct FftAxisPlan {
@@ -122,6 +123,7 @@ struct mdft_ctx {
     const void *dot_vec[3] = {nullptr, nullptr, nullptr};
     double *d_dpart = nullptr;    // [blocks][3] their block partials
     float *d_vext32 = nullptr;    // FP32 copy of vext read by the fast minimiser's final pass
+    void *d_logt = nullptr;       // ang.logt
     void *d_a2p_img[4] = {};      // angl2proj_t's weights: FP32, FP64, packed FP32, packed FP64
     bool packed = false;          // set during an evaluation whose projection field is packed (packed.h)
     int npk = 0;                  // packed projections per point
@@ -167,6 +169,7 @@ hipError_t launch_fft3d_f32(mdft_ctx *c, float2 *proj, int sign, int batch = 0);
 hipError_t launch_oz_f64(mdft_ctx *c, double2 *proj);
 bool ozm_supported(const mdft_ctx *c);
 int ozm_setup(mdft_ctx *c);
+int log_setup(mdft_ctx *c);
 int ozm_chopped(mdft_ctx *c, const std::vector<int> &pq, std::vector<int> &flag);
 int ozm_frags(mdft_ctx *c, const std::vector<double2> &tab, int nq, int npc, const std::vector<int> &ia0);
 hipError_t launch_ozp_f64(mdft_ctx *c, double2 *proj);  // packed projections, mmax <= 2

@@ -51,8 +51,14 @@ METRIC = "s to ΔG_solv within 0.05 kJ/mol, 128³ mmax=5: learned+mixed vs plain
 PHASES = ["angl2proj", "fft_forward", "oz", "fft_inverse", "proj2angl_ideal_grad", "reductions", "total"]
 
 
+def packed_projections(np_, mmax, precision):
+    """Projections stored per grid point in an evaluation (csrc/packed.h): the rotationally
+    independent half for mu2 = 0; BF16 contexts and mmax 6 keep all."""
+    return np_ if precision == "bf16" or mmax > 5 else (1, 2, 10, 20, 43, 70)[mmax]
+
+
 def phase_bytes(N, no, np_, b=16, fast=False):
-    """Algorithmic HBM bytes of each phase of one evaluation (complex of b bytes).
+    """Algorithmic HBM bytes of each phase of one evaluation (np_ stored projections, complex of b bytes).
     fast: the fast minimiser's evaluation -- FP32 iterate (4 B), the final pass reading the
     FP32 copy of vext (4 B) and two FP32 vectors for the gradient products (8 B) and
     writing the FP32 gradient (4 B); otherwise FP64 xi and vext read, FP64 dF written."""
@@ -70,7 +76,7 @@ def phase_bytes(N, no, np_, b=16, fast=False):
 # per-launch view of the phases: (kernel, launches per evaluation, kernel name in the traffic profile)
 KERNELS = {
     "angl2proj": ("angl2proj", 1, "angl2proj_t"),
-    "fft": ("fft_axis_r (one axis pass)", 6, "fft_axis_r"),
+    "fft": ("fft_cols (one axis pass)", 6, "fft_cols"),
     "oz": ("oz", 1, "oz"),
     "proj2angl_ideal_grad": ("final_t (proj2angl + ideal + gradient)", 1, "final_t"),
 }
@@ -293,8 +299,9 @@ def main():
         ph.append(eng.phase_times())
     ph = np.median(np.array(ph), axis=0)
     cbytes = 16 if args.precision == "fp64" else 8  # projection field: complex FP64 or FP32
-    algo = algorithmic_bytes(eng.N, eng.no, eng.np_, cbytes)
-    roof = roofline_of(ph, eng.N, eng.no, eng.np_, cbytes, traffic=args.precision == "fp32")
+    npk = packed_projections(eng.np_, w.mmax, args.precision)
+    algo = algorithmic_bytes(eng.N, eng.no, npk, cbytes)
+    roof = roofline_of(ph, eng.N, eng.no, npk, cbytes, traffic=args.precision == "fp32")
     roof.update({"whole_evaluation_algorithmic_GB": algo / 1e9, "whole_evaluation_frac": algo / dt / 1e9 / HBM_PEAK_GBS})
 
     line = {
@@ -400,7 +407,7 @@ def main():
         # the timed region
         ph32 = fast_eval_phases(e32, xi)
         line["roofline_fp64"] = line["roofline"]
-        line["roofline"] = roofline_of(ph32, e32.N, e32.no, e32.np_, 8, traffic=True, fast=True)
+        line["roofline"] = roofline_of(ph32, e32.N, e32.no, npk, 8, traffic=True, fast=True)
         line["phases_ms_fp32"] = {k: float(v) for k, v in zip(PHASES, ph32)}
         # reference-style solvation free energy of the fast path's final density
         # (src/module_pressure_correction.f90: F + PMV correction + LJ tail), outside the timed region
@@ -424,7 +431,7 @@ def main():
         dot_bytes = 2 * fast_m * vb if (vb == 4 and fast_m == 1) else (2 * fast_m + 1) * vb
         per_elem = (2 * fast_m + 1) * vb + vb + 2 * xb + dot_bytes
         # one FP32 evaluation: xi read twice (xb bytes), vext once (8), dF written (vb), projections
-        eval_bytes = eng.N * eng.no * (2 * xb + 8 + vb) + eng.N * 8 * eng.np_ * 8
+        eval_bytes = eng.N * eng.no * (2 * xb + 8 + vb) + eng.N * 8 * npk * 8
         t_roof = (res_f.evaluations * eval_bytes + res_f.iterations * per_elem * nvec) / (HBM_PEAK_GBS * 1e9)
         line["seconds_to_band_roofline"] = {"t_roofline_s": t_roof, "t_fast_s": t_fast, "frac": t_roof / t_fast,
                                             "vector_bytes_per_element_per_iteration": per_elem,

@@ -12,7 +12,7 @@
 // The chops apply to the FP64 kernel; the FP32 kernel skips them (their effect,
 // single-precision rounding of one component, is below FP32's own rounding).
 //
-// Work layout.  A workgroup of four waves takes a tile of 8 pairs that share the
+// Work layout.  A workgroup of two to four waves takes a tile of 8 pairs that share the
 // interpolation interval iq (pairs are sorted by iq on the host, one host-built
 // record per pair: grid indices of q and -q, flags, the angles of q and alpha);
 // the tile's 16 (side, pair) rows are the M dimension of the matrix products.
@@ -36,7 +36,7 @@
 //       series in theta, coefficients host-built and read one iteration ahead), chops it
 //       and uses it for both sides and every mu.
 //     The pairs are sorted by form, each form is a launch of its own;
-//  2. OZ contraction (OZ blocks khi spread over the four waves): for each khi
+//  2. OZ contraction (OZ blocks khi spread over the waves): for each khi
 //     the rows (m, mu) of both sides are
 //       gamma_s(m, khi, mu) = sum_{(n, nu)} c_{m mu; n nu}^{khi}(|q|) V_s(n, nu)
 //     with V_s(n, nu) = A_s(n, khi, |nu|) for nu < 0 and conj(A_-s(n, khi, nu))
@@ -197,7 +197,12 @@ template <int L> struct Plan {
     static constexpr int nfrag32 = foff32(L + 1);
 };
 
-constexpr int kWaves = 4;  // waves per tile
+constexpr int kWaves = 4;  // waves per tile with entry by entry rotations
+// Waves per tile with folded rotations: a tile's phases follow each other, and the fewer lanes its orders fill, the
+// more it gains from more tiles on a compute unit.  Measured with 2, 3, 4 waves: 64^3, mmax 3 FP32 57, 61, 67 us;
+// 96^3, mmax 3 FP64 340, 343, 374 us; 100^3, mmax 4 FP32 363, 364, 385, FP64 815, 760, 801 us; 128^3, mmax 5 FP32
+// 1.28, 1.20, 1.21, FP64 3.01, 2.85, 2.55 ms.
+template <int L, bool FOLD> constexpr int tile_waves() { return !FOLD ? kWaves : (L <= 3 ? 2 : L == 4 ? 3 : 4); }
 constexpr int kFold64 = 3;  // smallest mmax with folded rotations in FP64
 
 template <typename T> struct OzmArgs {
@@ -226,7 +231,7 @@ template <typename T> constexpr int scr_stride() { return sizeof(T) == 8 ? 18 : 
 template <typename T, int L, bool FOLD> struct LdsRows {
     using C = typename Ty<T>::c;
     C buf[16][Plan<L>::nps];
-    T scratch[kWaves * 16 * scr_stride<T>()];
+    T scratch[tile_waves<L, true>() * 16 * scr_stride<T>()];
     __device__ C (*x())[Plan<L>::nps] { return buf; }
     __device__ const C (*x() const)[Plan<L>::nps] { return buf; }
     __device__ T *scr() { return scratch; }
@@ -398,10 +403,10 @@ __device__ __forceinline__ void rot_all(const OzmArgs<T> &a, Lds<T, L, false> &s
 // come from s.d0.
 // A lane has all a and b of one row, order and mu2 in registers, reads and writes each LDS value once and
 // works in place; the J are the same for the wave.  A sixth of the multiplications of the entry by entry form,
-// whose LDS reads (every X once per khi) were its bound: 128^3, mmax 5 FP64 4.42 -> 2.64 ms, 96^3, mmax 3 644 ->
-// 379 us, with the tiles that keep that form.  In FP32, against two products with J on the matrix cores (whose
-// rate in FP32 and FP64 is the vector ALUs', here with no padding to 16 and no zeros): 128^3, mmax 5 1.61 -> 1.22
-// ms, 96^3, mmax 3 250 -> 210 us.
+// whose LDS reads (every X once per khi) were its bound: 128^3, mmax 5 FP64 4.42 -> 2.64 ms, 96^3, mmax 3 644
+// -> 379 us (4 waves per tile), with the tiles that keep that form.  In FP32, against two products with J on the
+// matrix cores (whose rate in FP32 and FP64 is the vector ALUs', here with no padding to 16 and no zeros): 128^3,
+// mmax 5 1.61 -> 1.22 ms, 96^3, mmax 3 250 -> 208 us.
 template <int K, typename C> __device__ __forceinline__ C times_i(C z) {  // i^K z
     constexpr int q = K & 3;
     C o;
@@ -532,11 +537,11 @@ __device__ __forceinline__ void rot_fold_role(Lds<T, L, true> &s, const T *__res
     } else if constexpr (M > 0) {
         if ((l >> 4) < Plan<L>::nmu(M)) rot_fold<T, L, M, BACK>(s, jt, l & 15, l >> 4);
     }
-    if constexpr (R == kWaves - 1 && M > 0) rot_fold_role<T, L, BACK, R, M - 1>(s, jt, l);
+    if constexpr (R == tile_waves<L, true>() - 1 && M > 0) rot_fold_role<T, L, BACK, R, M - 1>(s, jt, l);
 }
 template <typename T, int L, bool BACK, int R = 0>
 __device__ __forceinline__ void rot_fold_all(Lds<T, L, true> &s, const T *__restrict__ jt, int w, int l) {
-    if constexpr (R < kWaves) {
+    if constexpr (R < tile_waves<L, true>()) {
         if (w == R) rot_fold_role<T, L, BACK, R, L - R>(s, jt, l);
         else rot_fold_all<T, L, BACK, R + 1>(s, jt, w, l);
     }
@@ -595,9 +600,9 @@ __device__ __forceinline__ void store_all(typename Ty<T>::acc *acc, S &s, T *scr
     (gamma_store<T, L, KHI, NB>(acc[NB], s, scr, al, be, l), ...);
 }
 
-// blocks khi = KHI, KHI + kWaves, ... (the blocks of one wave; blocks are independent: block
+// blocks khi = KHI, KHI + NW, ... (the blocks of one wave; blocks are independent: block
 // khi reads and writes only the entries (., khi, .) of the rows)
-template <typename T, int L, int KHI, typename S>
+template <typename T, int L, int NW, int KHI, typename S>
 __device__ __forceinline__ void oz_blocks(S &s, const T *__restrict__ fr, T *scr, T al, T be, int l) {
     using P = Plan<L>;
     using A = typename Ty<T>::acc;
@@ -618,13 +623,13 @@ __device__ __forceinline__ void oz_blocks(S &s, const T *__restrict__ fr, T *scr
         for (int nb = 0; nb < NNB; nb++) acc[nb] = mfma16(x[kb], b[kb * NNB + nb], acc[nb]);
     // every read of block khi precedes its writes in the wave's LDS order
     store_all<T, L, KHI>(acc, s, scr, al, be, l, std::make_integer_sequence<int, NNB>{});
-    if constexpr (KHI + kWaves <= L) oz_blocks<T, L, KHI + kWaves>(s, fr, scr, al, be, l);
+    if constexpr (KHI + NW <= L) oz_blocks<T, L, NW, KHI + NW>(s, fr, scr, al, be, l);
 }
 
 // BF16 contraction of block khi (FP32 rotations and epilogue): A (16 x 32) lane l holds row
 // l & 15, k = 8 (l >> 4) + j: column 16 kb + 4 (l >> 4) + (j >> 1), re (j even) or im; B the
 // same k, column l & 15; D as in the FP32 form.
-template <int L, int KHI, typename S>
+template <int L, int NW, int KHI, typename S>
 __device__ __forceinline__ void oz_blocks_bf(S &s, const bf16x8 *__restrict__ fr,
                                              const int *__restrict__ colent, float *scr, float al, float be, int l) {
     using P = Plan<L>;
@@ -651,18 +656,18 @@ __device__ __forceinline__ void oz_blocks_bf(S &s, const bf16x8 *__restrict__ fr
             acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, fr[(F0 + kb * NNB + nb) * 64 + l], acc[nb], 0, 0, 0);
     }
     store_all<float, L, KHI>(acc, s, scr, al, be, l, std::make_integer_sequence<int, NNB>{});
-    if constexpr (KHI + kWaves <= L) oz_blocks_bf<L, KHI + kWaves>(s, fr, colent, scr, al, be, l);
+    if constexpr (KHI + NW <= L) oz_blocks_bf<L, NW, KHI + NW>(s, fr, colent, scr, al, be, l);
 }
 
-template <typename T, int L, bool BF, int W0, typename S>
+template <typename T, int L, bool BF, int NW, int W0, typename S>
 __device__ __forceinline__ void oz_wave(S &s, const OzmArgs<T> &a, size_t iv, T *scr, T al, T be, int w,
                                         int l) {
-    if constexpr (W0 < kWaves && -L + W0 <= L) {
+    if constexpr (W0 < NW && -L + W0 <= L) {
         if (w == W0) {
-            if constexpr (BF) oz_blocks_bf<L, -L + W0>(s, a.frag16 + iv * Plan<L>::nfrag32 * 64, a.colent, scr, al, be, l);
-            else oz_blocks<T, L, -L + W0>(s, a.frag + iv * Plan<L>::nfrag * 64, scr, al, be, l);
+            if constexpr (BF) oz_blocks_bf<L, NW, -L + W0>(s, a.frag16 + iv * Plan<L>::nfrag32 * 64, a.colent, scr, al, be, l);
+            else oz_blocks<T, L, NW, -L + W0>(s, a.frag + iv * Plan<L>::nfrag * 64, scr, al, be, l);
         } else {
-            oz_wave<T, L, BF, W0 + 1>(s, a, iv, scr, al, be, w, l);
+            oz_wave<T, L, BF, NW, W0 + 1>(s, a, iv, scr, al, be, w, l);
         }
     }
 }
@@ -751,16 +756,17 @@ __device__ __forceinline__ void pack_out(int d, typename Ty<T>::c &oq, typename 
     }
 }
 
-// Waves per SIMD asked for with folded rotations: FP32 5 (it gets 7 at mmax 5, 8 below; more makes no
-// difference), FP64 5 up to mmax 4, 4 at mmax 5 (without asking it gets 4 and 4: 96^3, mmax 3 453 against 379 us,
+// Waves per SIMD asked for with folded rotations: FP32 5 (it gets 7 at mmax 5, 8 below; more makes
+// no difference), FP64 5 up to mmax 4, 4 at mmax 5 (without asking it gets 4 and 4: 96^3, mmax 3 453 against 379 us,
 // 128^3, mmax 5 2.67 against 2.64 ms; 5 at mmax 5 spills, 2.95 ms, and so does 4 at mmax 6).
 template <typename T, int L, bool FOLD> constexpr int ozm_waves() {
     return !FOLD ? 1 : (sizeof(T) == 4 || L <= 4 ? 5 : (L == 5 ? 4 : 1));
 }
 template <typename T, int L, bool BF, bool PACK, bool FOLD>
-__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(ozm_waves<T, L, FOLD>(), 8)))
+__global__ __launch_bounds__((64 * tile_waves<L, FOLD>())) __attribute__((amdgpu_waves_per_eu(ozm_waves<T, L, FOLD>(), 8)))
 void ozm(typename Ty<T>::c *__restrict__ proj, OzmArgs<T> a) {
     using P = Plan<L>;
+    constexpr int NW = tile_waves<L, FOLD>(), TH = 64 * NW;
     using C = typename Ty<T>::c;
     constexpr int KP = P::kp, NP = P::np;
     extern __shared__ __align__(16) unsigned char smem[];
@@ -778,7 +784,7 @@ void ozm(typename Ty<T>::c *__restrict__ proj, OzmArgs<T> a) {
     // PACK: the records of q and -q, two entries (FP32, whole 16-byte words) or one per access, all
     // of a thread's loads issued before the angles are formed
     constexpr int NPK = PACK ? Packed<L>::np : 1, VE = (sizeof(T) == 4 && NPK % 2 == 0) ? 2 : 1;
-    constexpr int NPV = NPK / VE, NIT = (8 * NPV + 64 * kWaves - 1) / (64 * kWaves);
+    constexpr int NPV = NPK / VE, NIT = (8 * NPV + TH - 1) / (TH);
     struct alignas(VE * sizeof(C)) Vec {
         C v[VE];
     };
@@ -786,7 +792,7 @@ void ozm(typename Ty<T>::c *__restrict__ proj, OzmArgs<T> a) {
     if constexpr (PACK) {
 #pragma unroll
         for (int k = 0; k < NIT; k++) {
-            const int i = tid + k * 64 * kWaves, ii = i < 8 * NPV ? i : 8 * NPV - 1;
+            const int i = tid + k * TH, ii = i < 8 * NPV ? i : 8 * NPV - 1;
             const int pr = ii / NPV, e = ii - pr * NPV;
             pa[k] = reinterpret_cast<const Vec *>(proj + (size_t)tps[pr].gq * NPK)[e];
             pb[k] = reinterpret_cast<const Vec *>(proj + (size_t)tps[pr].gmq * NPK)[e];
@@ -823,7 +829,7 @@ void ozm(typename Ty<T>::c *__restrict__ proj, OzmArgs<T> a) {
     }
     __syncthreads();
     if constexpr (FOLD && sizeof(T) == 8) {
-        for (int i = tid; i < 8 * s.nd; i += 64 * kWaves) {
+        for (int i = tid; i < 8 * s.nd; i += TH) {
             const int e = i >> 3;
             int m = 0;
 #pragma unroll
@@ -842,7 +848,7 @@ void ozm(typename Ty<T>::c *__restrict__ proj, OzmArgs<T> a) {
     if constexpr (PACK) {
 #pragma unroll
         for (int k = 0; k < NIT; k++) {
-            const int i = tid + k * 64 * kWaves;
+            const int i = tid + k * TH;
             if (i >= 8 * NPV) break;
             const int pr = i / NPV, e = (i - pr * NPV) * VE;
 #pragma unroll
@@ -855,7 +861,7 @@ void ozm(typename Ty<T>::c *__restrict__ proj, OzmArgs<T> a) {
         // records are a whole number of 16-byte words
         if constexpr (sizeof(T) == 4 && NP % 2 == 0) {
             constexpr int NP2 = NP / 2;
-            for (int i = tid; i < 16 * NP2; i += 64 * kWaves) {
+            for (int i = tid; i < 16 * NP2; i += TH) {
                 const int r = i / NP2, e = 2 * (i - r * NP2);
                 const float4 x2 = reinterpret_cast<const float4 *>(proj + (size_t)s.g[r] * NP)[e / 2];
                 C out[2];
@@ -872,7 +878,7 @@ void ozm(typename Ty<T>::c *__restrict__ proj, OzmArgs<T> a) {
                 xs[r][e + 1] = out[1];
             }
         } else {
-            for (int i = tid; i < 16 * NP; i += 64 * kWaves) {
+            for (int i = tid; i < 16 * NP; i += TH) {
                 const int r = i / NP, e = i - r * NP;
                 C x = proj[(size_t)s.g[r] * NP + e];
                 if constexpr (FOLD) {
@@ -894,7 +900,7 @@ void ozm(typename Ty<T>::c *__restrict__ proj, OzmArgs<T> a) {
     {
         const C abv = s.ab[l & 7];  // the pair of row l & 15
         T *scr = s.scr() + w * 16 * scr_stride<T>();
-        oz_wave<T, L, BF, 0>(s, a, (size_t)(iq - 1), scr, abv.x, abv.y, w, l);
+        oz_wave<T, L, BF, NW, 0>(s, a, (size_t)(iq - 1), scr, abv.x, abv.y, w, l);
     }
     __syncthreads();
     if constexpr (FOLD) rot_fold_all<T, L, true>(s, a.jfold, w, l);
@@ -902,7 +908,7 @@ void ozm(typename Ty<T>::c *__restrict__ proj, OzmArgs<T> a) {
     __syncthreads();
     // store rule (:648-656): both sides of real pairs; for q == -q only the -q side
     if constexpr (PACK) {
-        for (int i = tid; i < 8 * NPV; i += 64 * kWaves) {
+        for (int i = tid; i < 8 * NPV; i += TH) {
             const int pr = i / NPV, e = (i - pr * NPV) * VE, f = s.flag[pr];
             if (f & 4) continue;
             Vec oq, om;
@@ -915,7 +921,7 @@ void ozm(typename Ty<T>::c *__restrict__ proj, OzmArgs<T> a) {
     }
     if constexpr (sizeof(T) == 4 && NP % 2 == 0) {
         constexpr int NP2 = NP / 2;
-        for (int i = tid; i < 16 * NP2; i += 64 * kWaves) {
+        for (int i = tid; i < 16 * NP2; i += TH) {
             const int r = i / NP2, e = 2 * (i - r * NP2);
             const int f = s.flag[r & 7];
             if ((f & 4) || (r < 8 && (f & 1))) continue;
@@ -923,7 +929,7 @@ void ozm(typename Ty<T>::c *__restrict__ proj, OzmArgs<T> a) {
             reinterpret_cast<float4 *>(proj + (size_t)s.g[r] * NP)[e / 2] = make_float4(u0.x, u0.y, u1.x, u1.y);
         }
     } else {
-        for (int i = tid; i < 16 * NP; i += 64 * kWaves) {
+        for (int i = tid; i < 16 * NP; i += TH) {
             const int r = i / NP, e = i - r * NP;
             const int f = s.flag[r & 7];
             if ((f & 4) || (r < 8 && (f & 1))) continue;
@@ -1040,7 +1046,7 @@ hipError_t launch_tiles(mdft_ctx *c, typename Ty<T>::c *proj, OzmArgs<T> &a, int
     a.per = (ntiles + 7) / 8;
     const size_t lds = sizeof(Lds<T, L, FOLD>);
     if (lds > c->lds_limit) return hipErrorInvalidConfiguration;
-    hipLaunchKernelGGL((ozm<T, L, BF, PACK, FOLD>), dim3((unsigned)(8 * a.per)), dim3(64 * kWaves), lds, c->stream, proj, a);
+    hipLaunchKernelGGL((ozm<T, L, BF, PACK, FOLD>), dim3((unsigned)(8 * a.per)), dim3(64 * tile_waves<L, FOLD>()), lds, c->stream, proj, a);
     return hipGetLastError();
 }
 

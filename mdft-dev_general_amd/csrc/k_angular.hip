@@ -705,8 +705,8 @@ template <int L, typename T> struct FinalShape {
     static constexpr int WAVES = 4;
 };
 
-// Bound by HBM: the fast variant moves 15.3 GB at 128^3, mmax 5, in 3.33 ms (4.6 TB/s; a plain copy
-// reaches 4.8), FP64 19.6 GB in 4.28 ms (4.6).  (FP64 with the library's logarithm, 1.4 ms of vector issue, took
+// Bound by HBM: the fast variant moves 15.0 GB at 128^3, mmax 5, in 3.33 ms (4.5 TB/s; a plain copy
+// reaches 4.8), FP64 19.0 GB in 4.28 ms (4.4).  (FP64 with the library's logarithm, 1.4 ms of vector issue, took
 // 5.53 ms; 96^3, mmax 3 558 against 439 us, 75^3, mmax 2 152 against 115.)  The phi synthesis takes one
 // thread per (row, mu2), in place; with one thread per (row, phi, mu2), each reading 11 coefficients
 // and 11 twiddles from LDS for one output, the pass took 3.70 (fast) and 6.79 ms (FP64).

@@ -7,8 +7,8 @@
 // all indices being compile-time constants, where the tiles of k_ozm.hip (8 pairs per workgroup of 256
 // threads) leave most threads idle between barriers.  Pairs are sorted by interpolation interval, so
 // that a wave's threads read the same two rows of c.  Bound by the gather of the pairs' records, at
-// mmax 2 by the two to eight waves per compute unit that the registers allow.  k_ozm.hip -> here, FP32 /
-// FP64: 96^3, mmax 1 115 -> 24 / 162 -> 28 us; 75^3, mmax 2 117 -> 46 / 217 -> 88; 64^3, mmax 0 30 -> 9 / 40 -> 10.
+// mmax 2 by the one (FP64) or two (FP32) waves per SIMD that the registers allow.  k_ozm.hip -> here, FP32 /
+// FP64: 96^3, mmax 1 115 -> 24 / 162 -> 26 us; 75^3, mmax 2 117 -> 44 / 217 -> 81; 64^3, mmax 0 30 -> 9 / 40 -> 10.
 #include <cfloat>
 #include <type_traits>
 
@@ -16,7 +16,9 @@
 
 namespace {
 
-constexpr int kThreads = 256;
+// Threads of a workgroup.  FP64 at mmax 2 holds one wave per SIMD, which single waves fill as they end (64, 128, 256
+// threads: 64^3 54, 60, 59 us, 128^3 330, 350, 353); FP32, 186, 179, 169 us at 128^3, shares the lines of c.
+template <typename T> constexpr int threads() { return sizeof(T) == 8 ? 64 : 256; }
 
 template <typename T> struct C2;
 template <> struct C2<double> { using t = double2; };
@@ -105,8 +107,16 @@ __device__ __forceinline__ typename C2<T>::t entry_r(const T *__restrict__ ftab,
     return r;
 }
 
+// o += a b in four multiply-adds (as a sum of two products, one of each three becomes an addition)
+template <typename T> __device__ __forceinline__ void mac(T &ox, T &oy, T ax, T ay, T bx, T by) {
+    ox = fma(ax, bx, ox);
+    oy = fma(ax, by, oy);
+    ox = fma(-ay, by, ox);
+    oy = fma(ay, bx, oy);
+}
+
 template <int L, typename T>
-__global__ __launch_bounds__(kThreads) void ozp(typename C2<T>::t *__restrict__ proj, const TilePair *__restrict__ pairs,
+__global__ __launch_bounds__(threads<T>()) void ozp(typename C2<T>::t *__restrict__ proj, const TilePair *__restrict__ pairs,
                                                unsigned n, unsigned per, const double2 *__restrict__ ck, int npc,
                                                const T *__restrict__ ftab) {
     using C = typename C2<T>::t;
@@ -114,7 +124,7 @@ __global__ __launch_bounds__(kThreads) void ozp(typename C2<T>::t *__restrict__ 
     using P = Packed<L>;
     constexpr int NP = I::np, NPK = P::np;
     // workgroups go to the 8 XCDs round robin: each takes a contiguous range of |q|
-    const unsigned i = ((blockIdx.x & 7) * per + (blockIdx.x >> 3)) * kThreads + threadIdx.x;
+    const unsigned i = ((blockIdx.x & 7) * per + (blockIdx.x >> 3)) * threads<T>() + threadIdx.x;
     if (i >= n) return;
     const TilePair tp = pairs[i];
     if (tp.flag & 4) return;  // padding
@@ -180,10 +190,8 @@ __global__ __launch_bounds__(kThreads) void ozp(typename C2<T>::t *__restrict__ 
                 each<0, NU>([&](auto u) {
                     const C v = x[I::p(m, mup, u)], w = y[I::p(m, mup, u)];
                     C &oa = a[(khi + m) * NU + u], &ob = b[(m - khi) * NU + u];
-                    oa.x += v.x * r.x - v.y * r.y;
-                    oa.y += v.x * r.y + v.y * r.x;
-                    ob.x += w.x * r.x - w.y * r.y;
-                    ob.y += w.x * r.y + w.y * r.x;
+                    mac(oa.x, oa.y, v.x, v.y, r.x, r.y);
+                    mac(ob.x, ob.y, w.x, w.y, r.x, r.y);
                 });
             });
         });
@@ -213,10 +221,8 @@ __global__ __launch_bounds__(kThreads) void ozp(typename C2<T>::t *__restrict__ 
                             p.y = -p.y;
                             q.y = -q.y;
                         }
-                        gx += cx * p.x - cy * p.y;
-                        gy += cx * p.y + cy * p.x;
-                        hx += cx * q.x - cy * q.y;
-                        hy += cx * q.y + cy * q.x;
+                        mac(gx, gy, p.x, p.y, cx, cy);
+                        mac(hx, hy, q.x, q.y, cx, cy);
                     });
                 });
                 chop_g(gx, gy);
@@ -251,10 +257,8 @@ __global__ __launch_bounds__(kThreads) void ozp(typename C2<T>::t *__restrict__ 
                 each<0, NU>([&](auto u) {
                     const C v = x[I::p(m, khi, u)], w = y[I::p(m, -khi, u)];
                     C &oa = a[(mup + m) * NU + u], &ob = b[(mup + m) * NU + u];
-                    oa.x += v.x * r.x + v.y * r.y;
-                    oa.y += v.y * r.x - v.x * r.y;
-                    ob.x += w.x * r.x + w.y * r.y;
-                    ob.y += w.y * r.x - w.x * r.y;
+                    mac(oa.x, oa.y, v.x, v.y, r.x, -r.y);
+                    mac(ob.x, ob.y, w.x, w.y, r.x, -r.y);
                 });
             });
         });
@@ -315,8 +319,9 @@ __global__ __launch_bounds__(kThreads) void ozp(typename C2<T>::t *__restrict__ 
 template <int L, typename T> hipError_t launch_ozp_t(mdft_ctx *c, typename C2<T>::t *proj) {
     const unsigned n = 8u * (unsigned)c->pairs.ntiles;
     if (n == 0) return hipSuccess;
-    const unsigned nb = (n + kThreads - 1) / kThreads, per = (nb + 7) / 8;
-    hipLaunchKernelGGL((ozp<L, T>), dim3(8 * per), dim3(kThreads), 0, c->stream, proj, c->pairs.tpair, n, per, c->d_ck,
+    constexpr unsigned TH = threads<T>();
+    const unsigned nb = (n + TH - 1) / TH, per = (nb + 7) / 8;
+    hipLaunchKernelGGL((ozp<L, T>), dim3(8 * per), dim3(TH), 0, c->stream, proj, c->pairs.tpair, n, per, c->d_ck,
                        c->npc, static_cast<const T *>(c->d_ozm_ftab));
     return hipGetLastError();
 }

@@ -5,6 +5,7 @@ import threading
 
 import numpy as np
 import pytest
+import torch  # before the library: it brings the HIP runtime that both use
 
 pytestmark = pytest.mark.gpu
 
@@ -57,7 +58,6 @@ def test_contexts_in_two_threads_share_the_kept_blocks():
 
 
 def test_the_last_context_gives_the_memory_back():
-    import torch
     from mdft.gpu import DeviceBuffer
     one = _engine()
     free0 = torch.cuda.mem_get_info()[0]

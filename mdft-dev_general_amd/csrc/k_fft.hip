@@ -414,9 +414,9 @@ bool launch_cols(int n, const Cols &g, hipStream_t st, V *proj, const double2 *t
     }
 }
 
-// one axis of `outer` blocks [n][C] from `data` on
+// one axis of `outer` blocks [n][C] from `data` on, of a field of np numbers per grid point
 template <typename V>
-hipError_t launch_axis(mdft_ctx *c, V *data, int ax, size_t C, size_t outer, double sign, double scale) {
+hipError_t launch_axis(mdft_ctx *c, V *data, int ax, size_t C, size_t outer, size_t np, double sign, double scale) {
     const int n = c->fft[ax].n;
     const unsigned PB = columns<V>();
     Cols g;
@@ -438,9 +438,19 @@ hipError_t launch_axis(mdft_ctx *c, V *data, int ax, size_t C, size_t outer, dou
             g.lines = 1;
             g.pb = (unsigned)g.C;
             g.nwg = g.nouter;
-            g.run = g.nwg < 8 * kRun ? (g.nwg + 7) / 8 : kRun;
         }
-        const size_t lds = sizeof(V) * 2 * (size_t)g.pb * (n + 1);
+        // LDS holds the lines of the columns twice.  From 640 points on that is more than there is for PB of
+        // them (160 KB); 4 are taken then where a point has fewer than PB numbers (mmax <= 1, in FP32 2), up to
+        // 1279 points, in FP32 2559.
+        const size_t line = sizeof(V) * 2 * (size_t)(n + 1);
+        if (g.pb * line > c->lds_limit && g.pb > 4 && np < PB) {
+            g.pb = 4;
+            g.nbatch = (unsigned)((C + 3) / 4);
+            g.nwg = g.nouter * g.nbatch;
+        }
+        const size_t lds = g.pb * line;
+        if (lds > c->lds_limit) return hipErrorInvalidConfiguration;
+        g.run = g.nwg < 8 * kRun ? (g.nwg + 7) / 8 : kRun;
         hipLaunchKernelGGL((fft_axis<V>), dim3((g.nwg + 8 * g.run - 1) / (8 * g.run) * 8 * g.run), dim3(kThreads), lds,
                            c->stream, data, g, c->fft[ax], sign, scale);
     }
@@ -463,17 +473,18 @@ hipError_t launch_fft3d(mdft_ctx *c, V *proj, int sign, int batch) {
     if (nslab > nz) nslab = nz;
     const size_t planes = (nz + nslab - 1) / nslab;  // per slab
     hipError_t e = hipSuccess;
-    if (sign < 0) e = launch_axis(c, proj, 2, plane, 1, sign, scale);
+    if (sign < 0) e = launch_axis(c, proj, 2, plane, 1, np, sign, scale);
     for (size_t z = 0; e == hipSuccess && z < nz; z += planes) {
         const size_t m = nz - z < planes ? nz - z : planes;
         V *p = proj + z * plane;
         const int first = sign < 0 ? 1 : 0;
         for (int k = 0; e == hipSuccess && k < 2; k++) {
             const int ax = k == 0 ? first : 1 - first;
-            e = ax == 0 ? launch_axis(c, p, 0, np, ny * m, sign, 1.0) : launch_axis(c, p, 1, nx * np, m, sign, 1.0);
+            e = ax == 0 ? launch_axis(c, p, 0, np, ny * m, np, sign, 1.0)
+                        : launch_axis(c, p, 1, nx * np, m, np, sign, 1.0);
         }
     }
-    if (e == hipSuccess && sign > 0) e = launch_axis(c, proj, 2, plane, 1, sign, scale);
+    if (e == hipSuccess && sign > 0) e = launch_axis(c, proj, 2, plane, 1, np, sign, scale);
     return e;
 }
 

@@ -6,7 +6,8 @@
 // most kKeep bytes per device, the oldest given back first; all are given back when the last
 // context of the device is destroyed, and when any allocation here fails.  A block is kept only
 // after the device has finished all work (as hipFree does; or its caller has waited for all that
-// used it), so its next owner may use it on any stream; the list is locked, so contexts in several threads share it.
+// used it), so its next owner may use it on any stream.  Contexts in several threads share the list under a
+// lock, which no one holds while it waits for the device (hipFree waits too).
 #include <list>
 #include <mutex>
 #include <unordered_map>
@@ -28,20 +29,22 @@ std::unordered_map<void *, Block> &live = *new std::unordered_map<void *, Block>
 std::list<Block> &idle = *new std::list<Block>;                                    // oldest first
 std::unordered_map<int, int> &users = *new std::unordered_map<int, int>;           // contexts per device
 
-// gives back idle blocks of a device, oldest first, until at most `keep` bytes of it are idle
-void trim(int device, size_t keep) {
+// takes idle blocks of a device off the list, oldest first, until at most `keep` bytes of it are idle (lock held)
+std::list<Block> taken(int device, size_t keep) {
     size_t n = 0;
     for (const Block &b : idle)
         if (b.device == device) n += b.bytes;
+    std::list<Block> out;
     for (auto it = idle.begin(); it != idle.end() && n > keep;) {
-        if (it->device != device) {
-            ++it;
-            continue;
-        }
-        n -= it->bytes;
-        (void)hipFree(it->p);
-        it = idle.erase(it);
+        const auto at = it++;
+        if (at->device != device) continue;
+        n -= at->bytes;
+        out.splice(out.end(), idle, at);
     }
+    return out;
+}
+void give_back(const std::list<Block> &blocks) {
+    for (const Block &b : blocks) (void)hipFree(b.p);
 }
 
 }  // namespace
@@ -52,42 +55,72 @@ hipError_t dev_malloc_bytes(void **p, size_t bytes) {
     int device = 0;
     hipError_t e = hipGetDevice(&device);
     if (e != hipSuccess) return e;
-    const std::lock_guard<std::mutex> hold(lock);
-    for (auto it = idle.begin(); it != idle.end(); ++it)
-        if (it->device == device && it->bytes == bytes) {
-            *p = it->p;
-            live[it->p] = *it;
-            idle.erase(it);
-            return hipSuccess;
-        }
+    {
+        const std::lock_guard<std::mutex> hold(lock);
+        for (auto it = idle.begin(); it != idle.end(); ++it)
+            if (it->device == device && it->bytes == bytes) {
+                *p = it->p;
+                live[it->p] = *it;
+                idle.erase(it);
+                return hipSuccess;
+            }
+    }
     e = hipMalloc(p, bytes);
     if (e == hipErrorOutOfMemory) {
         (void)hipGetLastError();
-        trim(device, 0);
+        std::list<Block> blocks;
+        {
+            const std::lock_guard<std::mutex> hold(lock);
+            blocks = taken(device, 0);
+        }
+        give_back(blocks);
         e = hipMalloc(p, bytes);
     }
-    if (e == hipSuccess) live[*p] = Block{*p, bytes, device};
-    else *p = nullptr;
-    return e;
+    if (e != hipSuccess) {
+        *p = nullptr;
+        return e;
+    }
+    const std::lock_guard<std::mutex> hold(lock);
+    live[*p] = Block{*p, bytes, device};
+    return hipSuccess;
 }
 
 hipError_t dev_free(void *p, bool synced) {
     if (!p) return hipSuccess;
-    const std::lock_guard<std::mutex> hold(lock);
-    const auto it = live.find(p);
-    if (it == live.end()) return hipFree(p);  // not from dev_malloc
-    const Block b = it->second;
-    live.erase(it);
+    Block b{};
+    bool keep = false;
+    {
+        const std::lock_guard<std::mutex> hold(lock);
+        const auto it = live.find(p);
+        if (it != live.end()) {  // else not from dev_malloc
+            b = it->second;
+            live.erase(it);
+            keep = b.bytes <= kKeep && users[b.device] > 0;
+        }
+    }
     int device = 0;
-    if (b.bytes > kKeep || hipGetDevice(&device) != hipSuccess || device != b.device || !users[b.device] ||
-        (!synced && hipDeviceSynchronize() != hipSuccess))
-        return hipFree(p);
-    trim(device, kKeep - b.bytes);
-    idle.push_back(b);
+    keep = keep && hipGetDevice(&device) == hipSuccess && device == b.device &&
+           (synced || hipDeviceSynchronize() == hipSuccess);
+    if (!keep) return hipFree(p);
+    std::list<Block> blocks;
+    {
+        const std::lock_guard<std::mutex> hold(lock);
+        if (users[device] > 0) {
+            blocks = taken(device, kKeep - b.bytes);
+            idle.push_back(b);
+        } else {  // the last context has gone meanwhile
+            blocks.push_back(b);
+        }
+    }
+    give_back(blocks);
     return hipSuccess;
 }
 
 void dev_context(int device, int change) {
-    const std::lock_guard<std::mutex> hold(lock);
-    if ((users[device] += change) <= 0) trim(device, 0);
+    std::list<Block> blocks;
+    {
+        const std::lock_guard<std::mutex> hold(lock);
+        if ((users[device] += change) <= 0) blocks = taken(device, 0);
+    }
+    give_back(blocks);
 }

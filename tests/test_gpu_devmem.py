@@ -70,3 +70,21 @@ def test_the_last_context_gives_the_memory_back():
     two.close()
     one.close()
     assert torch.cuda.mem_get_info()[0] >= free0 - (64 << 20)
+
+
+def test_a_freed_block_is_the_next_of_its_size():
+    from mdft.gpu import DeviceBuffer
+    eng = _engine()
+    a = DeviceBuffer(eng, 123456)
+    at = a.ptr.value
+    a.free()
+    b, c = DeviceBuffer(eng, 123464), DeviceBuffer(eng, 123456)
+    assert b.ptr.value != at and c.ptr.value == at
+    for v in (b, c):
+        v.free()
+    free0 = torch.cuda.mem_get_info()[0]
+    v = [DeviceBuffer(eng, 1 << 29) for _ in range(6)]
+    for x in v:
+        x.free()
+    assert torch.cuda.mem_get_info()[0] <= free0 - (1 << 30)   # some of them are still held
+    eng.close()

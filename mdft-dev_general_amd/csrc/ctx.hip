@@ -950,47 +950,52 @@ int mdft_compute_vext_ex(mdft_ctx *c, int natom, const double *atoms, int nsite,
     for (int io = 0; io < c->no; io++)
         for (int s : placed) pcol.push_back(col[(size_t)io * nsite + s]);
     VextPlaces pl{(int)col_site.size(), (int)placed.size(), nullptr, nullptr};
-    double *d_off = nullptr, *d_sp = nullptr, *d_at = nullptr, *d_S = nullptr, *d_cpos = nullptr;
-    int *d_col = nullptr, *d_csite = nullptr, *d_live = nullptr;
-    if (pl.ncols > 0 && dev_malloc(&d_S, sizeof(double) * c->N * pl.ncols) != hipSuccess) {
-        // no room for the places: their sites are summed per orientation
-        (void)hipGetLastError();
-        d_S = nullptr;
-        live.insert(live.end(), placed.begin(), placed.end());
-        pl.ncols = pl.nsite = 0;
-    }
-    hipError_t e = upload(c, &d_off, off.data(), off.size());
-    if (e == hipSuccess) e = upload(c, &d_sp, sp.data(), sp.size());
-    if (e == hipSuccess) e = upload(c, &d_at, at.data(), at.size());
-    if (e == hipSuccess && !live.empty()) e = upload(c, &d_live, live.data(), live.size());
-    if (e == hipSuccess && pl.ncols > 0) {
-        e = upload(c, &d_col, pcol.data(), pcol.size());
-        if (e == hipSuccess) e = upload(c, &d_cpos, col_pos.data(), col_pos.size());
-        if (e == hipSuccess) e = upload(c, &d_csite, col_site.data(), col_site.size());
-        if (e == hipSuccess)
-            e = launch_site_potential(c, natom, d_at, nsite, d_sp, rcut, qfact, direct, pl.ncols, d_cpos, d_csite, d_S);
-        pl.S = d_S;
-        pl.col = d_col;
-    }
     // the clip at qfact/2 (src/module_vext.f90:638-640) follows the sum of all terms.  Where every site
     // stands at few places, the Poisson path adds them as it writes vext
     const double clip = qfact / 2.0;
-    if (e == hipSuccess && !live.empty())
-        e = launch_vext(c, natom, d_at, nsite, d_sp, d_off, rcut, qfact, poisson ? HUGE_VAL : clip, direct, pl,
-                        (int)live.size(), d_live);
-    bool done = false;
-    if (e == hipSuccess && poisson) {
-        std::vector<double> sq(nsite);
-        for (int s = 0; s < nsite; s++) sq[s] = sites[6 * s + 3];
-        VextPlaces base = pl;
-        if (!live.empty()) base.ncols = -1;
-        e = launch_poisson_vext(c, natom, at.data(), nsite, sq.data(), off.data(), d_off, qfact, base, clip, &done);
-        if (e == hipSuccess && !done && !live.empty()) e = launch_vext_clip(c, clip);
+    auto compute = [&]() -> hipError_t {
+        double *d_off = nullptr, *d_sp = nullptr, *d_at = nullptr, *d_S = nullptr, *d_cpos = nullptr;
+        int *d_col = nullptr, *d_csite = nullptr, *d_live = nullptr;
+        hipError_t e = pl.ncols > 0 ? dev_malloc(&d_S, sizeof(double) * c->N * pl.ncols) : hipSuccess;
+        if (e == hipSuccess) e = upload(c, &d_off, off.data(), off.size());
+        if (e == hipSuccess) e = upload(c, &d_sp, sp.data(), sp.size());
+        if (e == hipSuccess) e = upload(c, &d_at, at.data(), at.size());
+        if (e == hipSuccess && !live.empty()) e = upload(c, &d_live, live.data(), live.size());
+        if (e == hipSuccess && pl.ncols > 0) {
+            e = upload(c, &d_col, pcol.data(), pcol.size());
+            if (e == hipSuccess) e = upload(c, &d_cpos, col_pos.data(), col_pos.size());
+            if (e == hipSuccess) e = upload(c, &d_csite, col_site.data(), col_site.size());
+            if (e == hipSuccess)
+                e = launch_site_potential(c, natom, d_at, nsite, d_sp, rcut, qfact, direct, pl.ncols, d_cpos, d_csite, d_S);
+        }
+        pl.S = d_S;
+        pl.col = d_col;
+        if (e == hipSuccess && !live.empty())
+            e = launch_vext(c, natom, d_at, nsite, d_sp, d_off, rcut, qfact, poisson ? HUGE_VAL : clip, direct, pl,
+                            (int)live.size(), d_live);
+        bool done = false;
+        if (e == hipSuccess && poisson) {
+            std::vector<double> sq(nsite);
+            for (int s = 0; s < nsite; s++) sq[s] = sites[6 * s + 3];
+            VextPlaces base = pl;
+            if (!live.empty()) base.ncols = -1;
+            e = launch_poisson_vext(c, natom, at.data(), nsite, sq.data(), off.data(), d_off, qfact, base, clip, &done);
+            if (e == hipSuccess && !done && !live.empty()) e = launch_vext_clip(c, clip);
+        }
+        if (e == hipSuccess && live.empty() && !done) e = launch_vext_from_places(c, pl, clip);
+        if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+        void *tmp[] = {d_off, d_sp, d_at, d_S, d_cpos, d_col, d_csite, d_live};
+        for (void *p : tmp) (void)dev_free(p, e == hipSuccess);
+        return e;
+    };
+    hipError_t e = compute();
+    if (e == hipErrorOutOfMemory && pl.ncols > 0) {
+        // no room for the places, or beside them for the Poisson fields: their sites are summed per orientation
+        (void)hipGetLastError();
+        live.insert(live.end(), placed.begin(), placed.end());
+        pl.ncols = pl.nsite = 0;
+        e = compute();
     }
-    if (e == hipSuccess && live.empty() && !done) e = launch_vext_from_places(c, pl, clip);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    void *tmp[] = {d_off, d_sp, d_at, d_S, d_cpos, d_col, d_csite, d_live};
-    for (void *p : tmp) (void)dev_free(p, e == hipSuccess);
     HIPCHK(c, e);
     c->have_vext = true;
     c->vext32_ok = false;

@@ -939,8 +939,11 @@ void ozm(typename Ty<T>::c *__restrict__ proj, OzmArgs<T> a) {
 }
 
 // Which pairs have a rotation matrix with a chopped entry R(mup, .), mup > 0, that the chop changes: a
-// component below FLT_EPSILON of an entry above 1e-13 (what it changes in a smaller one is below the rounding
-// of FP64).  A little above FLT_EPSILON, so that no rounding of d or of the phases decides.
+// component below FLT_EPSILON of an entry above kNoise.  Entries that vanish come out of the Fourier series as
+// at most 5e-16, which to keep or to drop is the rounding of the sums over them; those above kNoise are values.
+// (In boxes as they are used the classes are the same from 5e-16 to 1e-13: no entry lies between.)  A little
+// above FLT_EPSILON, so that no rounding of d or of the phases decides.
+constexpr double kNoise = 2e-15;
 template <int KP>
 __global__ void chopped_pairs(const int *__restrict__ pq, int n, int nx, int ny, const double *__restrict__ kx,
                               const double *__restrict__ ky, const double *__restrict__ kz,
@@ -975,7 +978,7 @@ __global__ void chopped_pairs(const int *__restrict__ pq, int n, int nx, int ny,
                     v1 += F[k] * tr[1][k];
                 }
                 const double d = fabs(((a - b) & 1) ? v1 : v0);
-                hit = hit || (d > 1e-13 && d * low < 1.0001 * (double)FLT_EPSILON);
+                hit = hit || (d > kNoise && d * low < 1.0001 * (double)FLT_EPSILON);
             }
     }
     flag[i] = hit ? 1 : 0;

@@ -42,3 +42,29 @@ def test_rotation_forms(precision, mmax):
         assert np.abs(parts - pref).max() <= bar * np.abs(pref).max(), (n, parts, pref)
         assert np.abs(df - dref).max() <= bar * np.abs(dref).max(), n
         eng.close()
+
+
+@pytest.mark.parametrize("mmax", [3, 4, 5, 6])
+def test_small_entries_are_chopped(mmax):
+    """Directions 1e-14 off the plane theta = pi/2: entries of the rotation that vanish there are up to 5e-14, which the
+    chop sets to 0.  Kept, they change the field by some 1e-14 of it.  Rounding: the square root of the at most
+    4 (mmax + 1)^2 products per sum, eps each, once for the rotations and once for the contraction; of the largest
+    modulus among the directions off the special planes."""
+    from mdft import ck
+    from mdft.gpu import Engine
+    from oracle import oracle as O
+    n, length = (5, 6, 3), (3.0, 4.1, 3.0e14)
+    table = ck.synthetic_ck(mmax, 1024, 0.05, seed=5 + mmax, n0=0.0333)
+    eng = Engine(n, length, mmax, 2, 2.4777, 0.0333, "fp64")
+    ora = O.Oracle(n, length, mmax, 2, 2.4777, 0.0333)
+    for e in (eng, ora):
+        e.set_ck(table)
+    xi = 1.0 + 0.3 * np.random.default_rng(mmax).uniform(-1, 1, eng.N * eng.no)
+    eng.set_vext(np.zeros(xi.size))
+    ref = ora.excess_stage(xi, 3)
+    got = eng.excess_stage(xi, 3)
+    eng.close()
+    ref, got = (v.reshape(3, 6, 5, -1)[1:, [1, 2, 4, 5], 1:] for v in (ref, got))
+    err = np.abs(got - ref).max() / np.abs(ref).max()
+    print(f"[qspace] mmax={mmax} {err:.2e}", flush=True)
+    assert err <= 4.0 * (mmax + 1) * np.finfo(np.float64).eps

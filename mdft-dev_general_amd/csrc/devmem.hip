@@ -77,6 +77,7 @@ hipError_t dev_malloc_bytes(void **p, size_t bytes) {
         e = hipMalloc(p, bytes);
     }
     if (e != hipSuccess) {
+        (void)hipGetLastError();  // told by the return value; the next launch's check is not to find it
         *p = nullptr;
         return e;
     }

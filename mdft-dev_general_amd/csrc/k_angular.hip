@@ -1114,6 +1114,7 @@ hipError_t ensure_partials(mdft_ctx *c, size_t nblocks) {
     if (c->partials_cap >= nblocks * 3) return hipSuccess;
     if (c->d_partials) (void)dev_free(c->d_partials);
     c->d_partials = nullptr;
+    c->partials_cap = 0;
     hipError_t e = dev_malloc(&c->d_partials, sizeof(double) * nblocks * 3);
     if (e == hipSuccess) c->partials_cap = nblocks * 3;
     return e;

@@ -471,6 +471,7 @@ int backward(mdft_wsnet *n, const float *d_in, float *d_gin) {
     if (need > n->part_cap) {
         (void)dev_free(n->part);
         n->part = nullptr;
+        n->part_cap = 0;
         WSCHK(n, dev_malloc(&n->part, sizeof(float) * need));
         n->part_cap = need;
     }

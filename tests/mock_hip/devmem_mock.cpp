@@ -16,6 +16,7 @@ size_t used = 0, room = 0;
 uintptr_t next_at = 4096;
 int device = 0, waiting = 0;
 bool gate = true;
+hipError_t last = hipSuccess;
 
 void wait_device() {
     std::unique_lock<std::mutex> l(mu);
@@ -28,11 +29,15 @@ void wait_device() {
 
 extern "C" {
 hipError_t hipGetDevice(int *d) { return *d = device, hipSuccess; }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() {
+    const hipError_t e = last;
+    last = hipSuccess;
+    return e;
+}
 hipError_t hipDeviceSynchronize() { return wait_device(), hipSuccess; }
 hipError_t hipMalloc(void **p, size_t n) {
     const std::lock_guard<std::mutex> l(mu);
-    if (used + n > room) return hipErrorOutOfMemory;
+    if (used + n > room) return last = hipErrorOutOfMemory;
     *p = reinterpret_cast<void *>(next_at);
     next_at += (n + 4095) / 4096 * 4096;  // no address is given twice
     held[*p] = n;

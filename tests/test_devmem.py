@@ -85,6 +85,7 @@ def test_an_allocation_that_fails_gets_the_kept_memory(mem):
     b = mem.alloc(GIB)
     assert b > 4095 and not mem.lib.mock_holds(a)
     assert mem.alloc(8) == -OUT_OF_MEMORY
+    assert mem.lib.hipGetLastError() == 0  # not left for the next launch's check
     mem.free(b)
     c = mem.alloc(8)
     mem.free(c)

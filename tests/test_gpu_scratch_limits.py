@@ -87,3 +87,56 @@ def test_vext_without_room_for_the_places(off_axis):
     eng.close()
     print("held")
     """, off_axis)
+
+
+def test_calls_after_a_refused_scratch_allocation():
+    """A larger call whose scratch memory is refused, then the smaller one that ran before: the same results."""
+    run("""
+    n, mmax, N = (6, 5, 4), 2, 120
+    eng = Engine(n, [0.5 * v for v in n], mmax, 2, 2.4777, 0.0333, "fp64")
+    eng.set_ck(ck.synthetic_ck(mmax, 512, 0.05, seed=1, n0=0.0333))
+    rng = np.random.default_rng(0)
+    eng.set_vext(rng.uniform(-2.0, 5.0, N * eng.no))
+    xi = 1.0 + 0.2 * rng.uniform(-1, 1, N * eng.no)
+    parts, df = eng.energy_and_gradient(xi)
+    npts = 5000
+    p, f = DeviceBuffer(eng, 16 * npts * eng.np_), DeviceBuffer(eng, 8 * npts * eng.no)
+    p.upload(rng.standard_normal(2 * npts * eng.np_))
+    print("projections to angles", flush=True)
+    before = limit.limit_failures()
+    limit.limit_size(24 * ((npts + 3) // 4))
+    try:
+        eng._check(eng.lib.mdft_proj2angl(eng._h, p.ptr, npts, f.ptr))
+        raise SystemExit("a transform without its scratch memory")
+    except MdftError as e:
+        assert e.code == ENOMEM and limit.limit_failures() > before, e
+    limit.limit_size(0)
+    again = eng.energy_and_gradient(xi)
+    assert np.array_equal(again[0], parts) and np.array_equal(again[1], df)
+
+    from mdft.warmstart import WarmStartNet
+    net = WarmStartNet((5, 8, 2), (1, 3), (1, 1), seed=5)
+    def buffers(n):
+        N = n[0] * n[1] * n[2]
+        b = DeviceBuffer(eng, 20 * N), DeviceBuffer(eng, 8 * N)
+        for v in b:
+            v.upload(rng.standard_normal(v.nbytes // 4).astype(np.float32))
+        return b
+    small, big = (4, 4, 4), (16, 16, 16)   # weight gradients in 1 and 4 slices of 2 8 27 + 2 sums
+    sx, st = buffers(small)
+    bx, bt = buffers(big)
+    loss, grads = net.loss_grad(small, sx, st), net.get_grads()
+    print("training step", flush=True)
+    before = limit.limit_failures()
+    limit.limit_size(4 * 4 * 434)
+    try:
+        net.loss_grad(big, bx, bt)
+        raise SystemExit("a gradient without its scratch memory")
+    except RuntimeError:
+        assert limit.limit_failures() > before
+    limit.limit_size(0)
+    assert net.loss_grad(small, sx, st) == loss and np.array_equal(net.get_grads(), grads)
+    net.close()
+    eng.close()
+    print("held")
+    """)

@@ -628,6 +628,7 @@ int mdft_set_ck(mdft_ctx *c, int np_file, const int *m, const int *n, const int 
             // conj (cproj_mrso.f90:415) then the sign folding (:420-429)
             tab[(size_t)iq * npc + ia] = make_double2(sgn[ia] * v[0], sgn[ia] * -v[1]);
         }
+    c->have_ck = false;  // until all that is made from the table is there
     if (c->d_ck) (void)dev_free(c->d_ck);
     c->d_ck = nullptr;
     HIPCHK(c, upload(c, &c->d_ck, tab.data(), tab.size()));

@@ -140,3 +140,48 @@ def test_calls_after_a_refused_scratch_allocation():
     eng.close()
     print("held")
     """)
+
+
+@pytest.mark.parametrize("precision,mmax", [("fp64", 1), ("fp64", 3), ("fp32", 4)])
+def test_no_evaluation_after_a_table_that_did_not_fit(precision, mmax):
+    """set_ck that fails half way leaves no table: an evaluation then says so instead of using what is left of two."""
+    run("""
+    precision, mmax = sys.argv[1], int(sys.argv[2])
+    n, N = (6, 5, 4), 120
+    eng = Engine(n, [0.5 * v for v in n], mmax, 2, 2.4777, 0.0333, precision)
+    one, two = (ck.synthetic_ck(mmax, 1024, dq, seed=1, n0=0.0333) for dq in (0.05, 0.04))
+    eng.set_ck(one)
+    rng = np.random.default_rng(0)
+    eng.set_vext(rng.uniform(-2.0, 5.0, N * eng.no))
+    xi = 1.0 + 0.2 * rng.uniform(-1, 1, N * eng.no)
+    parts, df = eng.energy_and_gradient(xi)
+    eng.set_ck(two)
+    # of the second table, and of its fragments for the matrix cores (per block khi 2 columns by 4 rows)
+    frags = sum((sum(2 * (m // 2) + 1 for m in range(abs(k), mmax + 1)) + 1) // 2 *
+                ((sum(m // 2 + 1 for m in range(abs(k), mmax + 1)) + 3) // 4) for k in range(-mmax, mmax + 1))
+    sizes = 16 * eng.npc * eng.nq, (8 if precision == "fp64" else 4) * 64 * frags * (eng.nq - 1)
+    for size in sizes:
+        eng.close()
+        eng = Engine(n, [0.5 * v for v in n], mmax, 2, 2.4777, 0.0333, precision)
+        eng.set_vext(np.zeros(N * eng.no))
+        eng.set_ck(one)
+        print("refusing", size, flush=True)
+        before = limit.limit_failures()
+        limit.limit_size(size)
+        try:
+            eng.set_ck(two)
+            raise SystemExit("a table without room")
+        except MdftError as e:
+            assert e.code == ENOMEM and limit.limit_failures() > before, e
+        limit.limit_size(0)
+        try:
+            eng.energy_and_gradient(xi)
+            raise SystemExit("an evaluation without a table")
+        except MdftError as e:
+            print(e, flush=True)
+            assert "c(k)" in str(e)
+    eng.set_ck(one)
+    eng.energy_and_gradient(xi)
+    eng.close()
+    print("held")
+    """, precision, mmax)

@@ -185,3 +185,40 @@ def test_no_evaluation_after_a_table_that_did_not_fit(precision, mmax):
     eng.close()
     print("held")
     """, precision, mmax)
+
+
+@pytest.mark.parametrize("mmax", [3, 4, 5, 6])
+def test_classes_of_pairs_without_memory(mmax):
+    """Without memory for the classes of the q-space pairs all of them keep the entry by entry rotations, which are
+    right for any: field, energies and gradient against the oracle at the bars of the two forms (1e-10)."""
+    run("""
+    mmax = int(sys.argv[1])
+    n, length = (9, 10, 8), (4.1, 5.3, 3.7)
+    table = ck.synthetic_ck(mmax, 1024, 0.05, seed=5 + mmax, n0=0.0333)
+    eng = Engine(n, length, mmax, 2, 2.4777, 0.0333, "fp64")
+    ora = O.Oracle(n, length, mmax, 2, 2.4777, 0.0333)
+    rng = np.random.default_rng(3)
+    xi = 1.0 + 0.3 * rng.uniform(-1, 1, eng.N * eng.no)
+    vext = rng.uniform(-2.0, 5.0, eng.N * eng.no)
+    eng.set_vext(vext)
+    # pairs: the half space of q, and of each plane that is its own image the half plane
+    pairs = sum(1 for z in range(n[2] // 2 + 1) for y in range(n[1]) for x in range(n[0])
+                if (n[2] - z) % n[2] != z or ((n[1] - y) % n[1], (n[0] - x) % n[0]) >= (y, x))
+    limit.limit_size(8 * pairs)
+    for e in (eng, ora):
+        e.set_ck(table)
+    assert limit.limit_failures() > 0
+    limit.limit_size(0)
+    ref = ora.excess_stage(xi, 3)
+    assert np.abs(eng.excess_stage(xi, 3) - ref).max() <= 1e-10 * np.abs(ref).max()
+    parts, df = eng.energy_and_gradient(xi)
+    pref, dref = ora.energy_and_gradient(xi, vext)
+    assert np.abs(parts - pref).max() <= 1e-10 * np.abs(pref).max()
+    assert np.abs(df - dref).max() <= 1e-10 * np.abs(dref).max()
+    eng.set_ck(table)   # and with memory again
+    again, da = eng.energy_and_gradient(xi)
+    assert np.abs(again - pref).max() <= 1e-10 * np.abs(pref).max()
+    assert np.abs(da - dref).max() <= 1e-10 * np.abs(dref).max()
+    eng.close()
+    print("held")
+    """, mmax)

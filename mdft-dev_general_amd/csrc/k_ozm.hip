@@ -113,7 +113,6 @@ __device__ inline double2 chop_R(double2 z) {
     }
     return make_double2(re, im);
 }
-__device__ inline float2 chop_R(float2 z) { return z; }
 
 // DBL_EPSILON chop of gamma (:618-623)
 __device__ inline void chop_gamma(double &re, double &im) {
@@ -1081,10 +1080,7 @@ template <typename T, int L, bool BF, bool PACK = false> hipError_t launch_ozm_t
 
 template <typename T, bool BF> hipError_t launch_ozm_any(mdft_ctx *c, typename Ty<T>::c *proj) {
     if constexpr (!BF) {
-        if (c->packed) switch (c->L) {
-                case 0: return launch_ozm_t<T, 0, false, true>(c, proj);
-                case 1: return launch_ozm_t<T, 1, false, true>(c, proj);
-                case 2: return launch_ozm_t<T, 2, false, true>(c, proj);
+        if (c->packed) switch (c->L) {  // (up to mmax 2: k_ozp.hip)
                 case 3: return launch_ozm_t<T, 3, false, true>(c, proj);
                 case 4: return launch_ozm_t<T, 4, false, true>(c, proj);
                 case 5: return launch_ozm_t<T, 5, false, true>(c, proj);
@@ -1255,7 +1251,7 @@ int ozm_setup(mdft_ctx *c) {
     if (hipMemcpy(c->d_ozm_units, units.data(), sizeof(int) * units.size(), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(c->d_ozm_rlen, rlen.data(), sizeof(int) * rlen.size(), hipMemcpyHostToDevice) != hipSuccess)
         return MDFT_EHIP;
-    if (L <= 5) {  // packed entries
+    if (L >= 3 && L <= 5) {  // packed entries
         std::vector<int> pk;
         auto item = [&](int mup, int mu2) {
             for (int m = std::max(std::abs(mup), 2 * mu2); m <= L; m++)

@@ -1277,11 +1277,18 @@ int ozm_setup(mdft_ctx *c) {
 }
 
 // 1 for the pairs (pq: grid index of q) whose tiles keep the entry by entry rotations, which is
-// for the FP64 kernel with folded rotations; 0 otherwise
+// for the FP64 kernel with folded rotations; 0 otherwise.  All pairs of a small box keep them: up to two tiles
+// per compute unit the chip is not full, and a second launch costs more than the folded form saves.  Evaluation
+// in one launch / in two: 8^3, mmax 4 73 / 83 us, 5 80 / 94; 16^3, mmax 3 65 / 73, 5 100 / 112; 20^3 (4004
+// pairs), mmax 3 70 / 78, 5 129 / 142, 6 414 / 408; 24^3 (6916), mmax 3 81 / 88, 5 180 / 176, 6 649 / 647.
 int ozm_chopped(mdft_ctx *c, const std::vector<int> &pq, std::vector<int> &flag) {
     const int n = (int)pq.size();
     flag.assign(n, 0);
     if (!ozm_supported(c) || c->d.precision != MDFT_PREC_FP64 || c->L < kFold64 || n == 0) return MDFT_OK;
+    if (n <= 16 * c->num_cus) {
+        flag.assign(n, 1);
+        return MDFT_OK;
+    }
     int *d = nullptr;
     if (dev_malloc(&d, 2 * sizeof(int) * (size_t)n) != hipSuccess) {  // the entry by entry form is right for all
         (void)hipGetLastError();

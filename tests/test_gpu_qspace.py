@@ -53,7 +53,7 @@ def test_small_entries_are_chopped(mmax):
     from mdft import ck
     from mdft.gpu import Engine
     from oracle import oracle as O
-    n, length = (5, 6, 3), (3.0, 4.1, 3.0e14)
+    n, length = (25, 30, 12), (3.0, 4.1, 3.0e14)
     table = ck.synthetic_ck(mmax, 1024, 0.05, seed=5 + mmax, n0=0.0333)
     eng = Engine(n, length, mmax, 2, 2.4777, 0.0333, "fp64")
     ora = O.Oracle(n, length, mmax, 2, 2.4777, 0.0333)
@@ -64,7 +64,39 @@ def test_small_entries_are_chopped(mmax):
     ref = ora.excess_stage(xi, 3)
     got = eng.excess_stage(xi, 3)
     eng.close()
-    ref, got = (v.reshape(3, 6, 5, -1)[1:, [1, 2, 4, 5], 1:] for v in (ref, got))
+    ref, got = (v.reshape(12, 30, 25, -1)[1:, [y for y in range(30) if y % 15], 1:] for v in (ref, got))
     err = np.abs(got - ref).max() / np.abs(ref).max()
     print(f"[qspace] mmax={mmax} {err:.2e}", flush=True)
     assert err <= 4.0 * (mmax + 1) * np.finfo(np.float64).eps
+
+
+# more than 4096 pairs, below which FP64 keeps one form for all: a plane along z and one across (all directions
+# special; of theta = pi/2 only), a long polar axis, unequal lengths, an even box
+LARGE_GRIDS = (((1, 90, 96), (3.0, 31.0, 35.0)), ((96, 90, 1), (35.0, 31.0, 3.0)), ((6, 5, 300), (24.0, 20.0, 24.0)),
+               ((18, 20, 25), (4.1, 5.3, 3.7)), ((24, 20, 18), (12.0, 10.0, 9.0)))
+
+
+@pytest.mark.parametrize("mmax", range(3, 7))
+def test_rotation_forms_of_large_grids(mmax):
+    from mdft import ck
+    from mdft.gpu import Engine
+    from oracle import oracle as O
+    table = ck.synthetic_ck(mmax, 1024, 0.05, seed=5 + mmax, n0=0.0333)
+    for n, length in LARGE_GRIDS:
+        print(f"[qspace] mmax={mmax} {n}", flush=True)
+        eng = Engine(n, length, mmax, 2, 2.4777, 0.0333, "fp64")
+        ora = O.Oracle(n, length, mmax, 2, 2.4777, 0.0333)
+        for e in (eng, ora):
+            e.set_ck(table)
+        rng = np.random.default_rng(sum(n))
+        xi = 1.0 + 0.3 * rng.uniform(-1, 1, eng.N * eng.no)
+        vext = rng.uniform(-2.0, 5.0, eng.N * eng.no)
+        eng.set_vext(vext)
+        ref = ora.excess_stage(xi, 3)
+        got = eng.excess_stage(xi, 3)
+        assert np.abs(got - ref).max() <= 1e-10 * np.abs(ref).max(), n
+        parts, df = eng.energy_and_gradient(xi)
+        pref, dref = ora.energy_and_gradient(xi, vext)
+        assert np.abs(parts - pref).max() <= 1e-10 * np.abs(pref).max(), (n, parts, pref)
+        assert np.abs(df - dref).max() <= 1e-10 * np.abs(dref).max(), n
+        eng.close()

@@ -193,7 +193,7 @@ def test_classes_of_pairs_without_memory(mmax):
     right for any: field, energies and gradient against the oracle at the bars of the two forms (1e-10)."""
     run("""
     mmax = int(sys.argv[1])
-    n, length = (9, 10, 8), (4.1, 5.3, 3.7)
+    n, length = (18, 20, 25), (4.1, 5.3, 3.7)   # (in a smaller box all pairs keep that form anyway)
     table = ck.synthetic_ck(mmax, 1024, 0.05, seed=5 + mmax, n0=0.0333)
     eng = Engine(n, length, mmax, 2, 2.4777, 0.0333, "fp64")
     ora = O.Oracle(n, length, mmax, 2, 2.4777, 0.0333)

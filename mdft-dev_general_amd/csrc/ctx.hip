@@ -928,9 +928,13 @@ int mdft_compute_vext_ex(mdft_ctx *c, int natom, const double *atoms, int nsite,
             const double *o = &off[((size_t)io * nsite + s) * 3];
             at_place[io] = place.emplace(std::make_tuple(o[0] + 0.0, o[1] + 0.0, o[2] + 0.0), (int)place.size()).first->second;
         }
-        // a place costs a column of N values and its sum over the atoms; from four orientations per
-        // place on that is less than the sum for each orientation
-        if (place.size() > 1 && 4 * place.size() > (size_t)c->no) {
+        // A place costs a column of N values, written once and read for each of its orientations, where a sum per
+        // orientation costs its atoms.  64^3, three sites on the axis, Lennard-Jones, places against
+        // orientations: five orientations per place (mmax 5) 1 atom 1.44 / 0.68 ms, 4 1.44 / 1.24, 6 1.44 / 1.63,
+        // 20 1.50 / 4.38, 300 4.6 / 59; with the Coulomb term 2 atoms 1.48 / 1.33, 4 1.50 / 2.21.  At three per place
+        // (mmax 2, 3) a site's columns are a third of vext's memory; they are not taken there, though from a few
+        // atoms on they would be faster as well (96^3, mmax 3, 20 atoms 1.65 / 3.34 ms; 64^3, 2 atoms 0.50 / 0.28).
+        if (place.size() > 1 && (natom < 4 || 4 * place.size() > (size_t)c->no)) {
             live.push_back(s);
             continue;
         }

@@ -78,3 +78,27 @@ def test_c2r_by_weighted_complex_inverse(shape):
     Z = np.zeros((nz, ny, nx), dtype=complex)
     Z[:, :, : nx // 2 + 1] = H * w
     assert np.abs(np.fft.ifftn(Z).real - ref).max() < 1e-13
+
+
+@pytest.mark.parametrize("shape", [(6, 5, 8), (7, 4, 9), (4, 6, 5), (1, 2, 1), (2, 1, 2), (3, 3, 1)])
+def test_two_c2r_by_one_complex_inverse(shape):
+    """Two half spectra (arbitrary, not Hermitian) by one complex inverse, as the device's Poisson solver takes two
+    orientations: each is completed to the Hermitian spectrum with that half on 0 < kx < nx/2, its conjugate at the
+    opposite wave vectors, and the Hermitian part of the planes kx = 0 and (even nx) nx/2; one is the real and the
+    other the imaginary part."""
+    nz, ny, nx = shape
+    rng = np.random.default_rng(sum(shape))
+    H = rng.normal(size=(2, nz, ny, nx // 2 + 1)) + 1j * rng.normal(size=(2, nz, ny, nx // 2 + 1))
+    S = np.zeros((2, nz, ny, nx), dtype=complex)
+    for z in range(nz):
+        for y in range(ny):
+            for x in range(nx // 2 + 1):
+                opposite = -z % nz, -y % ny, -x % nx
+                if x == opposite[2]:
+                    S[:, z, y, x] = (H[:, z, y, x] + H[:, opposite[0], opposite[1], x].conj()) / 2
+                else:
+                    S[:, z, y, x] = H[:, z, y, x]
+                    S[(slice(None),) + opposite] = H[:, z, y, x].conj()
+    both = np.fft.ifftn(S[0] + 1j * S[1])
+    for got, h in zip((both.real, both.imag), H):
+        assert np.abs(got - np.fft.irfftn(h, s=shape, axes=(0, 1, 2))).max() < 1e-13

@@ -593,9 +593,11 @@ __global__ void out_lanes_build(OutLane<L, T> *__restrict__ out, AngTables t) {
 // density guess xi and k0 = dv / 2: dF/dr / w for r = rho/rho0, whose angl2proj is the
 // adjoint of proj2angl up to a per-projection factor (the warm start's training gradient);
 // feat = 4: o = xi (the plain transform). k0 is rho0 for feat 0.
-// Bound by HBM: at 128^3, mmax 5 it reads 5.5 GB of FP64 xi and writes 1.5 (FP32) or 3.0 GB (FP64
-// projections) in 1.22 and 1.79 ms, 5.7 and 4.8 TB/s.  (One thread per psi sum, per phi sum and per
-// projection, tables in LDS: 2.22 and 3.72 ms, the time of its reads of values and twiddles from LDS.)
+// At 128^3, mmax 5, the stored 70 of 88 projections: FP64 reads 5.5 GB of xi and writes 2.35 GB in 1.61 ms, 4.9
+// TB/s, HBM; FP32 with FP64 xi reads as much and writes 1.17 GB in 1.21 ms, 5.5 TB/s, HBM; with the FP32
+// iterate of the fast minimiser it moves 3.9 GB in 1.16 ms, 3.4 TB/s, bound by vector issue (0.83 ms).  (One
+// thread per psi sum, per phi sum and per projection, tables in LDS, all 88 projections: 2.22 ms FP32 and 3.72 ms
+// FP64, the time of its reads of values and twiddles from LDS; by rows 1.22 and 1.79.)
 // The theta contraction gives a thread one projection, its weights in registers, and a group of
 // threads consecutive projections of a point, so the stores are whole records.
 template <int L, int PT, int TH, typename T, bool PACK>

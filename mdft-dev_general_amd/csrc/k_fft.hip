@@ -200,9 +200,9 @@ struct Cols {
 // Workgroups go to the 8 XCDs round robin in dispatch order.  `run` consecutive ones are given to
 // one XCD (one L2), so that the 128-byte lines that two workgroups share are read from HBM once,
 // while all XCDs stay within 8 run workgroups of each other: ranges an eighth of the field apart
-// meet in the same memory channels.  Measured per evaluation (128^3, mmax 5, FP64; 6 passes): one
-// range per XCD 7.00 ms, runs of 96 6.95, 24 6.55-7.0, 8 7.02, round robin 7.69 ms; FP32 (shared
-// lines along x) 3.52, 3.45, 3.47, 3.52, 4.40 ms.
+// meet in the same memory channels.  Measured per evaluation (128^3, mmax 5, FP64; 6 passes over all 88
+// projections, each over the whole field): one range per XCD 7.00 ms, runs of 96 6.95, 24 6.55-7.0, 8 7.02, round
+// robin 7.69 ms; FP32 (shared lines along x) 3.52, 3.45, 3.47, 3.52, 4.40 ms.
 constexpr unsigned kRun = 24;
 __device__ inline unsigned xcd_order(unsigned run) {
     const unsigned g = blockIdx.x / (8 * run), w = blockIdx.x - g * 8 * run;
@@ -258,9 +258,12 @@ __global__ __launch_bounds__(kThreads) void fft_axis(V *__restrict__ data, Cols 
 
 // ---- line lengths known at compile time: constant trip counts and twiddle indices, one LDS
 // buffer, the stages staged through registers.  A pass is bound by HBM: 4.8-5.3 TB/s of its one
-// read and one write at 96-180 points, where a plain copy reaches 4.8.  The lengths are those of
-// everyday boxes; the kernel above, with runtime radices, takes three to four times as long (six
-// FP32 passes at 100^3, mmax 4: 3.16 against 1.01 ms; at 180^3, mmax 5: 39.4 against 10.3 ms).
+// read and one write at 96-180 points, where a plain copy reaches 4.8.  The kernel above, with runtime
+// radices, takes about twice as long, 3.6 times at most (six passes in an evaluation, FP32: 100^3, mmax 4 1.71
+// against 0.73 ms, 180^3, mmax 5 24.7 against 6.9; FP64: 128^3, mmax 5 10.2 against 5.1, 48^3, mmax 1 56 against
+// 30 us).  The lengths are all products of 2, 3 and 5 from 16 to 128, where boxes mostly are, and eight of the
+// fourteen from there to 256.  135, 162, 216, 225, 243, 250 and all beyond 256 take the kernel above as the sizes
+// below 16 do: no workload has them (216^3, mmax 3, FP32: 14.1 of an evaluation's 21.9 ms).
 constexpr bool is_radix(int r) {
     return r == 2 || r == 3 || r == 4 || r == 5 || r == 6 || r == 8 || r == 9 || r == 10 || r == 12 || r == 15 || r == 16;
 }
@@ -277,7 +280,7 @@ constexpr int pick_radix(int rem, int rmax) {
     return 0;
 }
 // The largest radix: registers against passes over LDS.  FP64: a butterfly of 16 holds 64
-// registers (128^3: 16 and 8 took 7.85 ms where 8, 4 and 4 took 7.69).
+// registers (128^3, all 88 projections: 16 and 8 took 7.85 ms where 8, 4 and 4 took 7.69).
 template <typename V> constexpr int rmax() { return sizeof(V) == 16 ? 10 : 16; }
 
 template <typename V> constexpr int columns() { return 128 / (int)sizeof(V); }
@@ -353,7 +356,7 @@ __device__ inline void run_stages(V *A, const V *twl, decltype(V::x) s, V *__res
 
 // threads of a workgroup: the butterflies of its largest stage, at most 256 (one butterfly of the
 // first stage each, which at 128 points of FP64 leaves half of them without a load: 128 threads
-// took 7.14 against 7.00 ms per evaluation)
+// took 7.14 against 7.00 ms per evaluation, over all 88 projections)
 template <int N, int REM, typename V> constexpr int stage_tasks() {
     constexpr int R = REM <= rmax<V>() && is_radix(REM) && REM != N ? REM : pick_radix(REM, rmax<V>());
     constexpr int t = columns<V>() * (N / R);

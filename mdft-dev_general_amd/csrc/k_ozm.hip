@@ -940,7 +940,7 @@ void ozm(typename Ty<T>::c *__restrict__ proj, OzmArgs<T> a) {
 // Which pairs have a rotation matrix with a chopped entry R(mup, .), mup > 0, that the chop changes: a
 // component below FLT_EPSILON of an entry above kNoise.  Entries that vanish come out of the Fourier series as
 // at most 5e-16, which to keep or to drop is the rounding of the sums over them; those above kNoise are values.
-// (In boxes as they are used the classes are the same from 5e-16 to 1e-13: no entry lies between.)  A little
+// (In boxes as they are used the share of such pairs is the same for any bound from 5e-16 to 1e-13.)  A little
 // above FLT_EPSILON, so that no rounding of d or of the phases decides.
 constexpr double kNoise = 2e-15;
 template <int KP>

@@ -25,10 +25,10 @@
 //       A_q(m, khi, mu) = sum_mup X_q(m, mup, mu) R(mup, khi)
 //       A_-q(m, -khi, mu) = (-1)^m sum_mup X_-q(m, mup, mu) R(mup, khi),
 //     in one of two forms:
-//     - folded (FP32; FP64 from mmax 3 on, for the pairs whose chops are those of
-//       mup = 0 only): R as a product of two constant matrices, a phase between
+//     - folded (FP32; FP64 from mmax 3 and 16 pairs per compute unit on, for the
+//       pairs whose chops are those of mup = 0 only): R as a product of two constant matrices, a phase between
 //       (rot_fold), lanes over (side, pair) rows and mu;
-//     - entry by entry (rot_class; the other FP64 pairs, 5 to 9 % of them): lanes over
+//     - entry by entry (rot_class; the other FP64 pairs, 5 to 9 % of a large box): lanes over
 //       pairs, lane (pair p = l & 7, slot j = l >> 3) takes rotation units (m, khi) from a
 //       host-built round table (units of equal m/2 + 1 in a round, so the lanes run one
 //       instruction stream; rounds balanced over the four waves), forms R^m(mup, khi) =
